@@ -1,18 +1,19 @@
 // MXFP4 -> dense dequant and checkpoint -> row-tile repack (gfx950).
 //
-// Dequant is HBM bound (1 byte of codes + 1/32 byte of scale in, 2 bytes out
-// per value for bfloat16), so the kernel is built around coalesced traffic:
-// a workgroup owns a strip of 64 output columns (64 checkpoint rows, i.e. a
-// contiguous 64 x groups x 16-byte region) and walks the input dimension in
-// chunks of 16 groups.  Packed bytes are staged in LDS, then every thread
-// decodes a 4 (input rows) x 8 (output columns) block and writes four 16-byte
-// rows, so each wave-wide store covers full 128-byte lines of the transposed
-// [in, out] output.  The stores carry the non-temporal hint (the output is
-// written once and not read back by this kernel): 555 -> 536-548 us for 128
-// 2880 x 2880 matrices to bfloat16.  Values come from gfx950's scaled E2M1 conversions
-// (v_cvt_scalef32_pk_{bf16,f16,f32}_fp4), exact for every scale byte below
-// 255; the MX NaN scale 255 takes an integer path (mxfp4_f32_bits) that
-// reproduces the reference's +-inf / NaN.
+// Dequant is HBM bound (1 byte of codes + 1/32 byte of scale in, 2 or 4 bytes
+// out per value), and the transposed [in, out] output sets its pace: each
+// output row is one input column of the checkpoint, so what counts is that a
+// workgroup writes long runs of every output row it touches and that there
+// are enough workgroups for the chip however few matrices a call has.
+// Measured against workgroups that own 64 output columns for all groups:
+// 1 x 5760 x 90 groups to float16 25.0 -> 10.4 us, 16 x 2880 x 90 75 -> 73,
+// 100 x 2880 x 90 to float32 1,386 -> 749 (5.0 TB/s, a copy's rate), 32 x 2881
+// x 90 to bfloat16 468 -> 171 (odd rows: one unaligned 16-byte store instead
+// of eight 2-byte ones), one packed 5760 x 90 to bfloat16 24.7 -> 8.9; 128 x
+// 2880 x 90 to bfloat16 stays at 502 us (5.35 TB/s).  Values come from
+// gfx950's scaled E2M1 conversions (v_cvt_scalef32_pk_{bf16,f16,f32}_fp4),
+// exact for every scale byte below 255; the MX NaN scale 255 takes an integer
+// path (mxfp4_f32_bits) that reproduces the reference's +-inf / NaN.
 #include <algorithm>
 #include <type_traits>
 
@@ -20,12 +21,6 @@
 
 namespace klc {
 namespace {
-
-constexpr int kDqThreads = 256;
-constexpr int kDqCols = 64;      // output columns (= checkpoint rows) per workgroup
-constexpr int kDqGroups = 16;    // MX groups (32 inputs each) per iteration
-constexpr int kLdsStride = kDqGroups * 4 + 1;  // dwords per staged row: data + 1 pad (bank spread)
-constexpr int kSclStride = kDqGroups + 1;      // dwords per staged scale row
 
 // Converts one exact float32 bit pattern to the output dtype's bits.
 template <int kDtype>
@@ -39,263 +34,81 @@ __device__ __forceinline__ uint32_t to_out_bits(uint32_t f32bits) {
   }
 }
 
-// Workgroup barrier that orders LDS accesses only: __syncthreads' release
-// fence would also wait for every outstanding global store.
-__device__ __forceinline__ void lds_barrier() {
-  __builtin_amdgcn_fence(__ATOMIC_RELEASE, "workgroup", "local");
-  __builtin_amdgcn_s_barrier();
-  __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "workgroup", "local");
-}
-
 typedef __bf16 bf16x2_t __attribute__((ext_vector_type(2)));
 typedef _Float16 f16x2_t __attribute__((ext_vector_type(2)));
 typedef float f32x2_t __attribute__((ext_vector_type(2)));
 
-// Byte `h` of `v16` (two E2M1 codes, low nibble first) times `scale`, as two
-// 16-bit values packed low-first (bfloat16 or float16 per kDtype).
+// Elements 2q, 2q + 1 of the 8 codes in `word` times `scale`, as two 16-bit
+// values packed low-first (bfloat16 or float16 per kDtype).
 template <int kDtype>
-__device__ __forceinline__ uint32_t cvt_pair(uint32_t v16, float scale, int h) {
+__device__ __forceinline__ void cvt_word(uint32_t word, float scale, uint32_t (&pr)[4]) {
   if constexpr (kDtype == KLC_DTYPE_F16) {
-    const f16x2_t v = h ? __builtin_amdgcn_cvt_scalef32_pk_f16_fp4(v16, scale, 1)
-                        : __builtin_amdgcn_cvt_scalef32_pk_f16_fp4(v16, scale, 0);
-    return __builtin_bit_cast(uint32_t, v);
+    pr[0] = __builtin_bit_cast(uint32_t, __builtin_amdgcn_cvt_scalef32_pk_f16_fp4(word, scale, 0));
+    pr[1] = __builtin_bit_cast(uint32_t, __builtin_amdgcn_cvt_scalef32_pk_f16_fp4(word, scale, 1));
+    pr[2] = __builtin_bit_cast(uint32_t, __builtin_amdgcn_cvt_scalef32_pk_f16_fp4(word, scale, 2));
+    pr[3] = __builtin_bit_cast(uint32_t, __builtin_amdgcn_cvt_scalef32_pk_f16_fp4(word, scale, 3));
   } else {
-    const bf16x2_t v = h ? __builtin_amdgcn_cvt_scalef32_pk_bf16_fp4(v16, scale, 1)
-                         : __builtin_amdgcn_cvt_scalef32_pk_bf16_fp4(v16, scale, 0);
-    return __builtin_bit_cast(uint32_t, v);
+    pr[0] = __builtin_bit_cast(uint32_t, __builtin_amdgcn_cvt_scalef32_pk_bf16_fp4(word, scale, 0));
+    pr[1] = __builtin_bit_cast(uint32_t, __builtin_amdgcn_cvt_scalef32_pk_bf16_fp4(word, scale, 1));
+    pr[2] = __builtin_bit_cast(uint32_t, __builtin_amdgcn_cvt_scalef32_pk_bf16_fp4(word, scale, 2));
+    pr[3] = __builtin_bit_cast(uint32_t, __builtin_amdgcn_cvt_scalef32_pk_bf16_fp4(word, scale, 3));
   }
 }
 
-__device__ __forceinline__ f32x2_t cvt_pair_f32(uint32_t v16, float scale, int h) {
-  return h ? __builtin_amdgcn_cvt_scalef32_pk_f32_fp4(v16, scale, 1)
-           : __builtin_amdgcn_cvt_scalef32_pk_f32_fp4(v16, scale, 0);
-}
+// 2^(e - 127) of a scale byte below 255, exact (e = 0: the float32 subnormal)
+__device__ __forceinline__ float scale_f32(uint32_t e) { return __uint_as_float(e == 0u ? 0x00400000u : (e << 23)); }
 
-template <int kDtype, bool kPacked>
-__global__ __launch_bounds__(kDqThreads) void dequant_kernel(const uint8_t* __restrict__ blocks,
-                                                             const uint8_t* __restrict__ scales,
-                                                             void* __restrict__ out, int rows, int groups,
-                                                             int64_t packed_stride) {
-  __shared__ uint32_t s_blk[kDqCols * kLdsStride];
-  __shared__ uint32_t s_scl[kDqCols * kSclStride];
-
-  const int strips = (rows + kDqCols - 1) / kDqCols;
-  const int m = blockIdx.x / strips;
-  const int col0 = (blockIdx.x - m * strips) * kDqCols;
-  const int tid = threadIdx.x;
-  const int in_dim = groups * 32;
-
-  // load mapping: 16-byte chunks (row, 4 * i + gi), i = 0..3, per thread
-  const int l_row = tid >> 2;
-  const int l_gi = tid & 3;
-  // compute mapping: 4 input rows x 8 output columns per thread and sub-chunk
-  const int c_oc = tid & 7;
-  const int c_iq = tid >> 3;          // 0..31 quads of input rows in a 4-group sub-chunk
-  const int c_gi = c_iq >> 3;         // group within the sub-chunk
-  const int c_q4 = c_iq & 7;          // quad within the group
-  const int col = col0 + c_oc * 8;
-
-  const uint8_t* mat = blocks;
-  if constexpr (kPacked) mat = blocks + (int64_t)m * packed_stride;
-
-  // ---- one iteration = 16 groups: loads into registers, staged in LDS,
-  // decoded 4 groups at a time and stored as 16-byte rows of [in, out] ----
-  const int r_ld = col0 + l_row;
-  uint4 v[4];
-  uint32_t e[4];
-  // kClamp: every load reads a valid chunk (groups past the end re-read the
-  // last one; their values are never stored), so no branch guards a load
-  auto load_chunks = [&](int g0, auto clamp) {
-    constexpr bool kClamp = decltype(clamp)::value;
-#pragma unroll
-    for (int i = 0; i < 4; ++i) {
-      int g = g0 + 4 * i + l_gi;
-      if constexpr (kClamp) g = min(g, groups - 1);
-      v[i] = make_uint4(0u, 0u, 0u, 0u);
-      e[i] = 127u;
-      if (kClamp || (r_ld < rows && g < groups)) {
-        if constexpr (kPacked) {
-          const uint8_t* src = mat + ((int64_t)(r_ld / kTileRows) * groups + g) * 1024 + (r_ld % kTileRows) * 16;
-          v[i] = *reinterpret_cast<const uint4*>(src);
-          e[i] = mat[packed_scale_offset(rows, groups, r_ld, g)];
-        } else {
-          const int64_t chunk = ((int64_t)m * rows + r_ld) * groups + g;
-          v[i] = *reinterpret_cast<const uint4*>(blocks + chunk * 16);
-          e[i] = scales[chunk];
-        }
-      }
-    }
-  };
-  auto stage = [&]() {
-#pragma unroll
-    for (int i = 0; i < 4; ++i) {
-      uint32_t* dst = s_blk + l_row * kLdsStride + (4 * i + l_gi) * 4;
-      dst[0] = v[i].x;
-      dst[1] = v[i].y;
-      dst[2] = v[i].z;
-      dst[3] = v[i].w;
-      s_scl[l_row * kSclStride + 4 * i + l_gi] = e[i];
-    }
-  };
-  // 4 groups (sub-chunk sc) of the staged iteration: 4 input rows x 8 output
-  // columns per thread.  kFull: the strip's 64 columns and the 4 groups all
-  // exist and rows % 8 == 0, so every store is one unconditional 16-byte row.
-  auto compute = [&](int g0, int sc, auto full) {
-    constexpr bool kFull = decltype(full)::value;
-    const int gl = 4 * sc + c_gi;  // group within the iteration
-    uint32_t bits[4][8];
-#pragma unroll
-    for (int j = 0; j < 8; ++j) {
-      const int lr = c_oc * 8 + j;
-      const uint32_t word = s_blk[lr * kLdsStride + gl * 4 + (c_q4 >> 1)];
-      const uint32_t v16 = (word >> ((c_q4 & 1) * 16)) & 0xffffu;
-      const uint32_t ee = s_scl[lr * kSclStride + gl];
-      // hardware E2M1 x 2^(e-127) conversion, exact for e < 255 (e = 0: the
-      // float32 subnormal 2^-127 as scale).  E8M0 255 (the MX NaN scale):
-      // the reference's fp32 ldexp gives +-inf, and NaN for the zero codes;
-      // that value is selected, not branched to, so the loop body has no
-      // branch (a branch made the compiler wait for every store at the
-      // next iteration's loads).
-      const bool nan_scale = ee == 255u;
-      const float scale = __uint_as_float(ee == 0u ? 0x00400000u : (ee << 23));
-#pragma unroll
-      for (int h = 0; h < 2; ++h) {  // rows 2h and 2h + 1
-        if constexpr (kDtype == KLC_DTYPE_F32) {
-          const f32x2_t cv = cvt_pair_f32(v16, scale, h);
-          bits[2 * h][j] = __float_as_uint(cv.x);
-          bits[2 * h + 1][j] = __float_as_uint(cv.y);
-        } else {
-          const uint32_t pair = cvt_pair<kDtype>(v16, scale, h);
-          bits[2 * h][j] = pair & 0xffffu;
-          bits[2 * h + 1][j] = pair >> 16;
-        }
-      }
-#pragma unroll
-      for (int r = 0; r < 4; ++r) {
-        const uint32_t nan_bits = to_out_bits<kDtype>(mxfp4_f32_bits((v16 >> (4 * r)) & 0xfu, 255u));
-        bits[r][j] = nan_scale ? nan_bits : bits[r][j];
-      }
-    }
-    const int i0 = (g0 + gl) * 32 + c_q4 * 4;
-#pragma unroll
-    for (int r = 0; r < 4; ++r) {
-      const int64_t row_off = ((int64_t)m * in_dim + i0 + r) * rows;
-      if constexpr (kDtype == KLC_DTYPE_F32) {
-        float* o = static_cast<float*>(out) + row_off + col;
-        if (kFull || (col + 8 <= rows && (rows & 3) == 0)) {
-          __builtin_nontemporal_store(u32x4_t{bits[r][0], bits[r][1], bits[r][2], bits[r][3]},
-                                      reinterpret_cast<u32x4_t*>(o));
-          __builtin_nontemporal_store(u32x4_t{bits[r][4], bits[r][5], bits[r][6], bits[r][7]},
-                                      reinterpret_cast<u32x4_t*>(o) + 1);
-        } else {
-          for (int j = 0; j < 8; ++j)
-            if (col + j < rows) o[j] = __uint_as_float(bits[r][j]);
-        }
-      } else {
-        uint16_t* o = static_cast<uint16_t*>(out) + row_off + col;
-        if (kFull || (col + 8 <= rows && (rows & 7) == 0)) {
-          __builtin_nontemporal_store(u32x4_t{bits[r][0] | (bits[r][1] << 16), bits[r][2] | (bits[r][3] << 16),
-                                              bits[r][4] | (bits[r][5] << 16), bits[r][6] | (bits[r][7] << 16)},
-                                      reinterpret_cast<u32x4_t*>(o));
-        } else {
-          for (int j = 0; j < 8; ++j)
-            if (col + j < rows) o[j] = (uint16_t)bits[r][j];
-        }
-      }
-    }
-  };
-
-  int g0 = 0;
-  if (col0 + kDqCols <= rows && (rows & 7) == 0 && groups >= kDqGroups) {
-    // Full iterations of a full strip, in straight-line code: the next
-    // iteration's loads are issued before this iteration's stores.  Loads and
-    // stores share one completion counter and retire in order, so waiting
-    // for those loads leaves the stores in flight; the LDS-only barriers do
-    // not wait for them either.
-    // The first iteration is peeled, so the loop is entered, like its back
-    // edge, with one iteration's loads and then its stores outstanding (a
-    // loop entered with only loads outstanding gets one wait for all).
-    const int full = groups / kDqGroups * kDqGroups;
-    auto iteration = [&](int g) {
-      stage();
-      lds_barrier();
-      load_chunks(g + kDqGroups < groups ? g + kDqGroups : g, std::true_type{});
-#pragma unroll
-      for (int sc = 0; sc < kDqGroups / 4; ++sc) compute(g, sc, std::true_type{});
-    };
-    load_chunks(0, std::true_type{});
-    iteration(0);
-    for (g0 = kDqGroups; g0 < full; g0 += kDqGroups) {
-      lds_barrier();  // every thread is done reading the staged chunks
-      iteration(g0);
-    }
-    if (g0 < groups) {  // the tail iteration's chunks are already loaded
-      lds_barrier();
-      stage();
-      lds_barrier();
-#pragma unroll 1
-      for (int sc = 0; sc < kDqGroups / 4; ++sc) {
-        if (g0 + 4 * sc + c_gi >= groups) break;  // uniform per 8-lane group; no barrier inside
-        compute(g0, sc, std::false_type{});
-      }
-    }
-    return;
-  }
-  // Partial strips: one iteration at a time.
-  for (; g0 < groups; g0 += kDqGroups) {
-    load_chunks(g0, std::false_type{});
-    stage();
-    __syncthreads();
-#pragma unroll 1
-    for (int sc = 0; sc < kDqGroups / 4; ++sc) {
-      if (g0 + 4 * sc + c_gi >= groups) break;  // uniform per 8-lane group; no barrier inside
-      compute(g0, sc, std::false_type{});
-    }
-    __syncthreads();
+// One 16-byte piece of an output row: whole lines are streamed past the L2;
+// at an odd row length the piece has element alignment only (one unaligned
+// store) and shares its lines with its neighbours, so those stay in the L2.
+template <bool kAligned>
+__device__ __forceinline__ void store_piece(void* dst, u32x4_t v) {
+  if constexpr (kAligned) {
+    __builtin_nontemporal_store(v, static_cast<u32x4_t*>(dst));
+  } else {
+    typedef u32x4_t loose_t __attribute__((aligned(2)));
+    *static_cast<loose_t*>(dst) = v;
   }
 }
 
-// Checkpoint layout -> bfloat16 [in, out] in long output runs: workgroup
-// (matrix, column block, group quad) stages 4 groups' code chunks (a 64-byte
-// run of each checkpoint row) and scale bytes of up to kDqrCols checkpoint
-// rows (= output columns) in LDS, word-major (word w of row r at
-// sw[w * kDqrCols + r]), and writes output rows 128 q .. 128 q + 127 at its
-// columns: runs of 2 * ncols bytes.  The two quads that share a 128-byte
-// line of each row run side by side on one XCD (workgroups go to the XCDs
-// round-robin), so that line is fetched once.  A task is 8 output rows (a
-// band: one word of one group's chunks) x 8 output columns; the threads take
-// consecutive tasks, so a task's 8 16-byte stores are, across the workgroup,
-// runs of consecutive 16-byte pieces of output rows.  The scaled conversion
-// (exact for every scale byte below 255) gives pairs of input elements of one
-// row; v_perm_b32 pairs them up as pairs of columns.  Scale byte 255 (the MX
-// NaN scale) is rare: those tasks are written again with the exact integer
-// path (mxfp4_f32_bits) after the main loop, by the thread that wrote them
-// (program order), so the main loop has no branch for it.
-//
-// Measured (128 x 2880 x 2880 to bfloat16): 768 columns and 512 threads
-// (52 KB of LDS, 3 workgroups per CU) 511-518 us against 535-551 us for the
-// 64-column strips above; 1536 columns (one workgroup per CU) 551-558 us; one
-// group per workgroup (16-byte reads at the row stride) 1,010 us; several
-// items per workgroup with the next one's loads in flight, or buffer stores,
-// were slower.
-constexpr int kDqrThreads = 512;
-constexpr int kDqrGroups = 4;                                    // groups per workgroup
-constexpr int kDqrCols = 768;                                    // checkpoint rows per column block
-constexpr int kDqrRounds = kDqrCols * kDqrGroups / kDqrThreads;  // 16-byte loads per thread
-static_assert(kDqrCols * kDqrGroups % kDqrThreads == 0, "whole load rounds");
+// MXFP4 -> dense [in, out] in long output runs: workgroup (matrix, column
+// block, group quad) stages 4 groups' code chunks and scale bytes of up to
+// kCols checkpoint rows (= output columns) in LDS, word-major (word w of row
+// r at sw[w * kCols + r]), and writes output rows 128 q .. 128 q + 127 at its
+// columns.  In the checkpoint layout the 4 groups are a 64-byte run of each
+// row, and the two quads that share a 128-byte line of each row run side by
+// side on one XCD (workgroups go to the XCDs round-robin), so that line is
+// fetched once; in the packed layout a group's chunks of 64 rows are
+// contiguous.  A task is 8 output rows (a band: one word of one group's
+// chunks) x 16 bytes of output columns; the threads take consecutive tasks,
+// so a task's 8 stores are, across the workgroup, runs of consecutive 16-byte
+// pieces of output rows.  The scaled conversion (exact for every scale byte
+// below 255) gives pairs of input elements of one row; v_perm_b32 pairs them
+// up as pairs of columns.  Scale byte 255 (the MX NaN scale) is rare: those
+// tasks are written again with the exact integer path (mxfp4_f32_bits) after
+// the main loop, by the thread that wrote them (program order), so the main
+// loop has no branch for it.
+constexpr int kDqGroups = 4;  // groups per workgroup
 
-__host__ __device__ constexpr int dqr_col_blocks(int rows) { return (rows + kDqrCols - 1) / kDqrCols; }
-// Column block cb of nb over rows (a multiple of 64): nearly equal widths, multiples of 64 columns
-__host__ __device__ inline int dqr_col0(int rows, int nb, int cb) { return (int)((int64_t)rows / 64 * cb / nb) * 64; }
+// Column block cb of nb over rows: nearly equal widths, multiples of 64 columns but for the last
+__host__ __device__ inline int dq_col0(int rows, int nb, int cb) {
+  const int col = (int)((int64_t)((rows + 63) / 64) * cb / nb) * 64;
+  return col < rows ? col : rows;
+}
 
-__global__ __launch_bounds__(kDqrThreads) void dequant_rows_bf16_kernel(const uint8_t* __restrict__ blocks,
-                                                                        const uint8_t* __restrict__ scales,
-                                                                        uint16_t* __restrict__ out, int n_mat,
-                                                                        int rows, int groups) {
-  extern __shared__ __align__(16) uint32_t lds_words[];  // [16][kDqrCols] code words, then scale bytes
+template <int kDtype, bool kPacked, bool kAligned, int kThreads, int kCols>
+__global__ __launch_bounds__(kThreads) void dequant_kernel(const uint8_t* __restrict__ blocks,
+                                                           const uint8_t* __restrict__ scales, uint8_t* __restrict__ out,
+                                                           int n_mat, int rows, int groups, int nb,
+                                                           int64_t packed_stride) {
+  constexpr int kElem = kDtype == KLC_DTYPE_F32 ? 4 : 2;
+  constexpr int kPiece = 16 / kElem;                     // output columns of a 16-byte piece
+  constexpr int kRounds = kCols * kDqGroups / kThreads;  // 16-byte loads per thread
+  static_assert(kCols * kDqGroups % kThreads == 0, "whole load rounds");
+  __shared__ __align__(16) uint32_t sw[4 * kDqGroups * kCols];
+  __shared__ __align__(16) uint8_t ss[kDqGroups * kCols];
   // workgroup -> (pair of quads P, half h): P's two workgroups are 8 apart in a window of 16
-  const int nb = dqr_col_blocks(rows);
-  const int quads = (groups + kDqrGroups - 1) / kDqrGroups;
+  const int quads = (groups + kDqGroups - 1) / kDqGroups;
   const int pairs = (quads + 1) / 2;
   const int b = blockIdx.x;
   const int pair = (b >> 4) * 8 + (b & 7);
@@ -304,95 +117,137 @@ __global__ __launch_bounds__(kDqrThreads) void dequant_rows_bf16_kernel(const ui
   if (quad >= quads || mcb >= n_mat * nb) return;
   const int m = mcb / nb;
   const int cb = mcb - m * nb;
-  const int col0 = dqr_col0(rows, nb, cb);
-  const int ncols = dqr_col0(rows, nb, cb + 1) - col0;
-  const int g0 = quad * kDqrGroups;
-  const int ng = min(kDqrGroups, groups - g0);
-  uint32_t* sw = lds_words;
-  uint8_t* ss = reinterpret_cast<uint8_t*>(lds_words + 4 * kDqrGroups * kDqrCols);
+  const int col0 = dq_col0(rows, nb, cb);
+  const int ncols = dq_col0(rows, nb, cb + 1) - col0;
+  const int g0 = quad * kDqGroups;
+  const int ng = min(kDqGroups, groups - g0);
   const int tid = threadIdx.x;
-  const int64_t first = (int64_t)m * rows * groups + (int64_t)col0 * groups + g0;  // chunk (col0, g0)
-  const int span = (ncols - 1) * groups + ng;                                     // chunks to the last one
-  const __amdgpu_buffer_rsrc_t cbuf =
-      __builtin_amdgcn_make_buffer_rsrc((void*)(blocks + first * 16), (short)0, span * 16, kBufferWord3);
-  const __amdgpu_buffer_rsrc_t sbuf =
-      __builtin_amdgcn_make_buffer_rsrc((void*)(scales + first), (short)0, span, kBufferWord3);
-  // load i: row r = (tid + i * threads) / 4, chunk c = tid % 4; rows and groups past the end read out of
-  // range (zeros, no traffic).  Every load first, then the LDS writes.
-  const int c = tid & 3;
-  u32x4_t v[kDqrRounds];
-  uint32_t e[kDqrRounds];
+  // Load i of this thread is chunk c of row r; rows and groups past the end
+  // read the last one again (the line is there already), so no load is
+  // guarded.  Every load first, then the LDS writes.
+  auto where = [&](int i, int& r, int& c) {
+    const int idx = tid + i * kThreads;
+    if constexpr (kPacked) {  // a wave reads one group's 64-row tile
+      r = (idx & 63) + (idx >> 8) * 64;
+      c = (idx >> 6) & 3;
+    } else {
+      r = idx >> 2;
+      c = idx & 3;
+    }
+  };
+  u32x4_t v[kRounds];
+  uint32_t e[kRounds];
 #pragma unroll
-  for (int i = 0; i < kDqrRounds; ++i) {
-    const int r = (tid >> 2) + i * (kDqrThreads / 4);
-    const bool live = r < ncols && c < ng;
-    const uint32_t chunk = (uint32_t)r * (uint32_t)groups + (uint32_t)c;
-    v[i] = __builtin_amdgcn_raw_buffer_load_b128(cbuf, live ? chunk * 16u : kOutOfRange, 0, 0);
-    e[i] = __builtin_amdgcn_raw_buffer_load_b8(sbuf, live ? chunk : kOutOfRange, 0, 0);
+  for (int i = 0; i < kRounds; ++i) {
+    int r, c;
+    where(i, r, c);
+    r = col0 + min(r, ncols - 1);
+    c = g0 + min(c, ng - 1);
+    if constexpr (kPacked) {
+      const uint8_t* mat = blocks + (int64_t)m * packed_stride;
+      v[i] = *reinterpret_cast<const u32x4_t*>(mat + ((int64_t)(r / kTileRows) * groups + c) * 1024 + (r % kTileRows) * 16);
+      e[i] = mat[packed_scale_offset(rows, groups, r, c)];
+    } else {
+      const int64_t chunk = ((int64_t)m * rows + r) * groups + c;
+      v[i] = *reinterpret_cast<const u32x4_t*>(blocks + chunk * 16);
+      e[i] = scales[chunk];
+    }
   }
 #pragma unroll
-  for (int i = 0; i < kDqrRounds; ++i) {
-    const int r = (tid >> 2) + i * (kDqrThreads / 4);
+  for (int i = 0; i < kRounds; ++i) {
+    int r, c;
+    where(i, r, c);
     if (r < ncols) {
 #pragma unroll
-      for (int w = 0; w < 4; ++w) sw[(4 * c + w) * kDqrCols + r] = v[i][w];
-      ss[c * kDqrCols + r] = (uint8_t)e[i];
+      for (int w = 0; w < 4; ++w) sw[(4 * c + w) * kCols + r] = v[i][w];
+      ss[c * kCols + r] = (uint8_t)e[i];
     }
   }
   __syncthreads();
 
-  const int cpr = ncols >> 3;  // 16-byte pieces (8 columns) per output run
-  const int ntask = 4 * ng * cpr;
-  uint16_t* obase = out + ((int64_t)m * groups + g0) * 32 * rows + col0;
+  const int ppr = (ncols + kPiece - 1) / kPiece;  // pieces per output run
+  const int ntask = 4 * ng * ppr;
+  const int64_t row_bytes = (int64_t)rows * kElem;
+  uint8_t* obase = out + ((int64_t)m * groups + g0) * 32 * row_bytes + (int64_t)col0 * kElem;
   bool nan_scale = false;
-  for (int t = tid; t < ntask; t += kDqrThreads) {
-    const int band = t / cpr;  // group band / 4, word band % 4
-    const int oc = t - band * cpr;
-    const uint32_t* wrow = sw + band * kDqrCols + oc * 8;
-    const u32x4_t wa = *reinterpret_cast<const u32x4_t*>(wrow);
-    const u32x4_t wb = *reinterpret_cast<const u32x4_t*>(wrow + 4);
-    const uint2 sc8 = *reinterpret_cast<const uint2*>(ss + (band >> 2) * kDqrCols + oc * 8);
-    const uint32_t word[8] = {wa[0], wa[1], wa[2], wa[3], wb[0], wb[1], wb[2], wb[3]};
-    // pr[j][q]: elements 2q, 2q + 1 of the band for column j (checkpoint row col0 + 8 oc + j)
-    uint32_t pr[8][4];
+  for (int t = tid; t < ntask; t += kThreads) {
+    const int band = t / ppr;  // group band / 4, word band % 4
+    const int pc = t - band * ppr;
+    const uint32_t* wrow = sw + band * kCols + pc * kPiece;
+    const uint8_t* srow = ss + (band >> 2) * kCols + pc * kPiece;
+    uint8_t* o = obase + (int64_t)(8 * band) * row_bytes + pc * 16;
+    u32x4_t row[8];
+    if constexpr (kElem == 4) {
+      const u32x4_t wa = *reinterpret_cast<const u32x4_t*>(wrow);
+      const uint32_t sc4 = *reinterpret_cast<const uint32_t*>(srow);
 #pragma unroll
-    for (int j = 0; j < 8; ++j) {
-      const uint32_t eb = ((j < 4 ? sc8.x : sc8.y) >> (8 * (j & 3))) & 0xffu;
-      nan_scale |= eb == 255u;
-      const float scale = __uint_as_float(eb == 0u ? 0x00400000u : (eb << 23));
-      pr[j][0] = __builtin_bit_cast(uint32_t, __builtin_amdgcn_cvt_scalef32_pk_bf16_fp4(word[j], scale, 0));
-      pr[j][1] = __builtin_bit_cast(uint32_t, __builtin_amdgcn_cvt_scalef32_pk_bf16_fp4(word[j], scale, 1));
-      pr[j][2] = __builtin_bit_cast(uint32_t, __builtin_amdgcn_cvt_scalef32_pk_bf16_fp4(word[j], scale, 2));
-      pr[j][3] = __builtin_bit_cast(uint32_t, __builtin_amdgcn_cvt_scalef32_pk_bf16_fp4(word[j], scale, 3));
+      for (int j = 0; j < 4; ++j) {
+        const uint32_t eb = (sc4 >> (8 * j)) & 0xffu;
+        nan_scale |= eb == 255u;
+        const float scale = scale_f32(eb);
+        const f32x2_t p0 = __builtin_amdgcn_cvt_scalef32_pk_f32_fp4(wa[j], scale, 0);
+        const f32x2_t p1 = __builtin_amdgcn_cvt_scalef32_pk_f32_fp4(wa[j], scale, 1);
+        const f32x2_t p2 = __builtin_amdgcn_cvt_scalef32_pk_f32_fp4(wa[j], scale, 2);
+        const f32x2_t p3 = __builtin_amdgcn_cvt_scalef32_pk_f32_fp4(wa[j], scale, 3);
+        row[0][j] = __float_as_uint(p0.x), row[1][j] = __float_as_uint(p0.y);
+        row[2][j] = __float_as_uint(p1.x), row[3][j] = __float_as_uint(p1.y);
+        row[4][j] = __float_as_uint(p2.x), row[5][j] = __float_as_uint(p2.y);
+        row[6][j] = __float_as_uint(p3.x), row[7][j] = __float_as_uint(p3.y);
+      }
+    } else {
+      const u32x4_t wa = *reinterpret_cast<const u32x4_t*>(wrow);
+      const u32x4_t wb = *reinterpret_cast<const u32x4_t*>(wrow + 4);
+      const uint2 sc8 = *reinterpret_cast<const uint2*>(srow);
+      const uint32_t word[8] = {wa[0], wa[1], wa[2], wa[3], wb[0], wb[1], wb[2], wb[3]};
+      uint32_t pr[8][4];  // pr[j][q]: elements 2q, 2q + 1 of the band for column j
+#pragma unroll
+      for (int j = 0; j < 8; ++j) {
+        const uint32_t eb = ((j < 4 ? sc8.x : sc8.y) >> (8 * (j & 3))) & 0xffu;
+        nan_scale |= eb == 255u;
+        cvt_word<kDtype>(word[j], scale_f32(eb), pr[j]);
+      }
+#pragma unroll
+      for (int i = 0; i < 8; ++i) {  // output row i: half i % 2 of every column's pair i / 2, columns paired low-first
+        const int q = i >> 1;
+        const uint32_t sel = (i & 1) ? 0x07060302u : 0x05040100u;
+        row[i] = u32x4_t{__builtin_amdgcn_perm(pr[1][q], pr[0][q], sel), __builtin_amdgcn_perm(pr[3][q], pr[2][q], sel),
+                         __builtin_amdgcn_perm(pr[5][q], pr[4][q], sel), __builtin_amdgcn_perm(pr[7][q], pr[6][q], sel)};
+      }
     }
-    uint16_t* o = obase + (int64_t)(8 * band) * rows + oc * 8;
+    if (kAligned || (pc + 1) * kPiece <= ncols) {
 #pragma unroll
-    for (int q = 0; q < 4; ++q) {
+      for (int i = 0; i < 8; ++i) store_piece<kAligned>(o + i * row_bytes, row[i]);
+    } else {  // the last columns of an odd row length
 #pragma unroll
-      for (int h = 0; h < 2; ++h) {
-        // output row 8 band + 2 q + h: half h of every column's pair q, columns paired low-first
-        const uint32_t sel = h ? 0x07060302u : 0x05040100u;
-        const u32x4_t row = {__builtin_amdgcn_perm(pr[1][q], pr[0][q], sel), __builtin_amdgcn_perm(pr[3][q], pr[2][q], sel),
-                             __builtin_amdgcn_perm(pr[5][q], pr[4][q], sel), __builtin_amdgcn_perm(pr[7][q], pr[6][q], sel)};
-        __builtin_nontemporal_store(row, reinterpret_cast<u32x4_t*>(o + (int64_t)(2 * q + h) * rows));
+      for (int j = 0; j < kPiece - 1; ++j) {
+        if (pc * kPiece + j >= ncols) break;
+#pragma unroll
+        for (int i = 0; i < 8; ++i) {
+          if constexpr (kElem == 4)
+            reinterpret_cast<uint32_t*>(o + i * row_bytes)[j] = row[i][j];
+          else
+            reinterpret_cast<uint16_t*>(o + i * row_bytes)[j] = (uint16_t)(row[i][j >> 1] >> (16 * (j & 1)));
+        }
       }
     }
   }
   if (!__syncthreads_or(nan_scale)) return;
   // tasks with a scale byte 255, again with the integer path, by the same threads (same addresses,
   // program order: these stores land after the first ones)
-  for (int t = tid; t < ntask; t += kDqrThreads) {
-    const int band = t / cpr;
-    const int oc = t - band * cpr;
-    const uint8_t* sc = ss + (band >> 2) * kDqrCols + oc * 8;
-    bool any = false;
-    for (int j = 0; j < 8; ++j) any |= sc[j] == 255u;
-    if (!any) continue;
-    uint16_t* o = obase + (int64_t)(8 * band) * rows + oc * 8;
-    for (int i = 0; i < 8; ++i) {
-      for (int j = 0; j < 8; ++j) {
-        const uint32_t code = (sw[band * kDqrCols + oc * 8 + j] >> (4 * i)) & 0xfu;
-        o[(int64_t)i * rows + j] = (uint16_t)(mxfp4_f32_bits(code, sc[j]) >> 16);
+  for (int t = tid; t < ntask; t += kThreads) {
+    const int band = t / ppr;
+    const int pc = t - band * ppr;
+    uint8_t* o = obase + (int64_t)(8 * band) * row_bytes + pc * 16;
+    for (int j = 0; j < min(kPiece, ncols - pc * kPiece); ++j) {
+      const uint32_t eb = ss[(band >> 2) * kCols + pc * kPiece + j];
+      if (eb != 255u) continue;
+      const uint32_t word = sw[band * kCols + pc * kPiece + j];
+      for (int i = 0; i < 8; ++i) {
+        const uint32_t bits = to_out_bits<kDtype>(mxfp4_f32_bits((word >> (4 * i)) & 0xfu, eb));
+        if constexpr (kElem == 4)
+          reinterpret_cast<uint32_t*>(o + i * row_bytes)[j] = bits;
+        else
+          reinterpret_cast<uint16_t*>(o + i * row_bytes)[j] = (uint16_t)bits;
       }
     }
   }
@@ -536,43 +391,60 @@ int launch_pack(const uint8_t* blocks, const uint8_t* scales, uint8_t* out_block
 
 namespace {
 
+// One launch with workgroups of kThreads over column blocks of at most kCols.
+template <int kDtype, bool kPacked, int kThreads, int kCols>
+int launch_dequant_shape(const uint8_t* blocks, const uint8_t* scales, uint8_t* out, int64_t n_mat, int64_t rows,
+                         int64_t groups, int64_t nb, int64_t packed_stride, hipStream_t stream) {
+  const int64_t pairs = ((groups + kDqGroups - 1) / kDqGroups + 1) / 2;
+  const int64_t grid = (n_mat * nb * pairs + 7) / 8 * 16;
+  KLC_REQUIRE(grid <= 0x7fffffff, KLC_ERR_UNSUPPORTED, "dequant: too many matrices (%lld)", (long long)n_mat);
+  if (rows % (kDtype == KLC_DTYPE_F32 ? 4 : 8) == 0) {
+    dequant_kernel<kDtype, kPacked, true, kThreads, kCols><<<(unsigned)grid, kThreads, 0, stream>>>(
+        blocks, scales, out, (int)n_mat, (int)rows, (int)groups, (int)nb, packed_stride);
+  } else if constexpr (!kPacked) {  // packed matrices have whole 64-row tiles
+    dequant_kernel<kDtype, kPacked, false, kThreads, kCols><<<(unsigned)grid, kThreads, 0, stream>>>(
+        blocks, scales, out, (int)n_mat, (int)rows, (int)groups, (int)nb, packed_stride);
+  }
+  return check_launch("dequant_kernel");
+}
+
+// The workgroup shape: long runs (1024 columns, two workgroups per CU) once
+// they give 2048 workgroups, else 384 columns, and fewer (down to 128) until
+// there are 768 workgroups.  Measured, wide against 384 columns: 128 x 2880 x
+// 90 groups to bfloat16 502 against 509 us, 32 x 2881 x 90 (2,304 wide
+// workgroups) 171 against 193; 16 x 2880 x 90 (1,152) packed 66 against 62, 4
+// x 2880 x 90 21.8 against 17.4, 1 x 2880 x 90 8.2 against 6.0 (6.6 without
+// the narrower blocks).
+template <int kDtype, bool kPacked>
+int launch_dequant_as(const uint8_t* blocks, const uint8_t* scales, uint8_t* out, int64_t n_mat, int64_t rows,
+                      int64_t groups, int64_t packed_stride, hipStream_t stream) {
+  const int64_t per_block = n_mat * ((groups + 2 * kDqGroups - 1) / (2 * kDqGroups)) * 2;  // workgroups
+  const int64_t wide = (rows + 1023) / 1024;
+  if (per_block * wide >= 2048)
+    return launch_dequant_shape<kDtype, kPacked, 512, 1024>(blocks, scales, out, n_mat, rows, groups, wide,
+                                                            packed_stride, stream);
+  const int64_t most = std::max((rows + 383) / 384, rows / 128);
+  const int64_t nb = std::clamp((768 + per_block - 1) / per_block, (rows + 383) / 384, most);
+  return launch_dequant_shape<kDtype, kPacked, 256, 384>(blocks, scales, out, n_mat, rows, groups, nb, packed_stride,
+                                                         stream);
+}
+
 template <bool kPacked>
 int launch_dequant(const void* blocks, const void* scales, void* out, int64_t n_mat, int64_t rows, int64_t groups,
                    int dtype, int64_t packed_stride, hipStream_t stream) {
-  if constexpr (!kPacked) {
-    // checkpoint layout to bfloat16, rows a multiple of 64: long output runs per workgroup (a
-    // matrix's codes below kOutOfRange bytes, so the out-of-range loads stay out of range)
-    if (dtype == KLC_DTYPE_BF16 && rows % 64 == 0 && rows * groups * 16 < (int64_t)kOutOfRange) {
-      const int64_t pairs = n_mat * dqr_col_blocks((int)rows) * (((groups + kDqrGroups - 1) / kDqrGroups + 1) / 2);
-      const int64_t grid = (pairs + 7) / 8 * 16;
-      if (grid <= 0x7fffffff) {
-        const size_t lds = (size_t)kDqrCols * kDqrGroups * 17;
-        dequant_rows_bf16_kernel<<<(unsigned)grid, kDqrThreads, lds, stream>>>(
-            static_cast<const uint8_t*>(blocks), static_cast<const uint8_t*>(scales), static_cast<uint16_t*>(out),
-            (int)n_mat, (int)rows, (int)groups);
-        return check_launch("dequant_rows_bf16_kernel");
-      }
-    }
-  }
-  const int64_t strips = (rows + kDqCols - 1) / kDqCols;
-  const int64_t grid = n_mat * strips;
-  KLC_REQUIRE(grid <= 0x7fffffff, KLC_ERR_UNSUPPORTED, "dequant: too many matrices (%lld)", (long long)n_mat);
   const auto* b = static_cast<const uint8_t*>(blocks);
   const auto* s = static_cast<const uint8_t*>(scales);
+  auto* o = static_cast<uint8_t*>(out);
   switch (dtype) {
     case KLC_DTYPE_BF16:
-      dequant_kernel<KLC_DTYPE_BF16, kPacked><<<(unsigned)grid, kDqThreads, 0, stream>>>(b, s, out, (int)rows, (int)groups, packed_stride);
-      break;
+      return launch_dequant_as<KLC_DTYPE_BF16, kPacked>(b, s, o, n_mat, rows, groups, packed_stride, stream);
     case KLC_DTYPE_F16:
-      dequant_kernel<KLC_DTYPE_F16, kPacked><<<(unsigned)grid, kDqThreads, 0, stream>>>(b, s, out, (int)rows, (int)groups, packed_stride);
-      break;
+      return launch_dequant_as<KLC_DTYPE_F16, kPacked>(b, s, o, n_mat, rows, groups, packed_stride, stream);
     case KLC_DTYPE_F32:
-      dequant_kernel<KLC_DTYPE_F32, kPacked><<<(unsigned)grid, kDqThreads, 0, stream>>>(b, s, out, (int)rows, (int)groups, packed_stride);
-      break;
+      return launch_dequant_as<KLC_DTYPE_F32, kPacked>(b, s, o, n_mat, rows, groups, packed_stride, stream);
     default:
       return set_error(KLC_ERR_ARGUMENT, "dequant: unknown dtype %d", dtype);
   }
-  return check_launch("dequant_kernel");
 }
 
 }  // namespace

@@ -67,6 +67,23 @@ def test_dequant_seeded_matches_oracle(gpu, n_mat, out_dim, groups):
     same_bits_nan_aware(bf16_bits(got), want, "bf16")
 
 
+@pytest.mark.parametrize("dtype,kind", [(torch.bfloat16, "bf16"), (torch.float16, "f16"), (torch.float32, "f32")])
+@pytest.mark.parametrize("n_mat,out_dim,groups", [(1, 1, 1), (2, 7, 5), (1, 63, 9), (3, 65, 4), (1, 385, 8), (1, 770, 3),
+                                                   (2, 1028, 1), (5, 129, 11), (1, 5760, 3), (64, 33, 128),
+                                                   (64, 36, 125), (256, 64, 31), (1, 1029, 4093)])
+def test_dequant_shapes_match_oracle(gpu, n_mat, out_dim, groups, dtype, kind):
+    """Both workgroup shapes (the last four calls take the wide one) over odd and aligned row
+    lengths, partial group quads and column blocks, every scale byte: bit-exact."""
+    blocks, scales = synth.mxfp4_expert_tensors(out_dim, groups, n_mat, out_dim, groups * 32, 0, 255)
+    got = ops.mxfp4_dequant(torch.from_numpy(blocks).to(gpu), torch.from_numpy(scales).to(gpu), dtype)
+    g = bf16_bits(got) if kind == "bf16" else got.cpu().numpy()
+    same_bits_nan_aware(g, omx.dequantize_batch(blocks, scales, kind), kind)
+    if out_dim % 64 == 0:
+        packed = ops.mxfp4_pack(torch.from_numpy(blocks).to(gpu), torch.from_numpy(scales).to(gpu))
+        again = ops.mxfp4_dequant_packed(packed, out_dim, groups, dtype)
+        assert torch.equal(again.view(torch.uint8), got.view(torch.uint8))
+
+
 def test_dequant_single_matrix_shape_and_errors(gpu):
     blocks, scales = synth.mxfp4_expert_tensors(1, 2, 1, 64, 64)
     b = torch.from_numpy(blocks[0]).to(gpu)
