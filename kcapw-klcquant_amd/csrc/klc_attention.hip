@@ -16,11 +16,16 @@
 // sum, which accumulates in float32 per split and float64 across splits, is
 // rounded to the cache's type and then to bfloat16 (o_proj's input type).
 //
-// Kernels per step: scores (workgroup = one KV head x 64 keys, its whole
-// query group), probabilities x values (workgroup = one query head x 256
-// keys, each taking its head's max and sum over all the scores first), and
-// the sum of the splits; a window of at most 256 keys (one split) runs as
-// one launch, scores to context, one workgroup per query head.
+// Kernels per step: scores with per-block maxima and sums (workgroup = one KV
+// head x 64 or 256 keys, its whole query group), probabilities x values
+// (workgroup = one KV head x 128 or 256 keys), and the sum of the splits; a
+// window of at most 256 keys runs as one launch, scores to context, one
+// workgroup per query head.  Measured for 64 / 8 heads x 64, float16 (cold
+// rings): 4,096 keys 23.7 -> 17.6 us, 8,192 40.2 -> 21.2, 16,384 81.6 ->
+// 29.8, 32,768 200 -> 43.2 against value workgroups per query head that each
+// took their head's statistics over all its scores (quadratic in the
+// context: 186 of the 200 us) and vector float64 dot products per query head
+// (38 us -> 20).
 #include <math.h>
 
 #include "klc_common.h"
@@ -29,10 +34,10 @@ namespace klc {
 namespace {
 
 constexpr int kAttnThreads = 256;
-constexpr int kScoreKeys = 64;   // keys per scores workgroup
-constexpr int kPvKeys = 256;     // keys per value-sum workgroup
+constexpr int kPvKeys = 256;     // most keys of a value workgroup, and of a one-launch window
 constexpr int kMaxHeadDim = 128;
 constexpr int kMaxGroup = 16;    // query heads per KV head
+typedef double f64x4_t __attribute__((ext_vector_type(4)));
 
 __device__ __forceinline__ float bf(uint16_t b) { return __uint_as_float((uint32_t)b << 16); }
 __device__ __forceinline__ uint16_t to_bf(float f) { return (uint16_t)f32_to_bf16_rne(f); }
@@ -69,44 +74,6 @@ __global__ __launch_bounds__(kAttnThreads) void rope_append_kernel(
       const int e = i - pairs;
       v_cache[slot * nkv * d + e] = f16 ? to_kv(bf(v[e]), true) : v[e];
     }
-  }
-}
-
-// scores[h][i] for the keys i in [64 * blockIdx.y, +64) of KV head blockIdx.x
-__global__ __launch_bounds__(kAttnThreads) void attn_scores_kernel(
-    const uint16_t* __restrict__ q, const uint16_t* __restrict__ k_cache, float* __restrict__ scores, int64_t cap,
-    int64_t first, int count, int nh, int nkv, int d, float sqrt_d, bool f16) {
-  __shared__ float qs[kMaxGroup][kMaxHeadDim];
-  const int g = nh / nkv, kvh = blockIdx.x;
-  const int key = blockIdx.y * kScoreKeys + (threadIdx.x % kScoreKeys);
-  const int part = threadIdx.x / kScoreKeys;  // 4 parts share the group's heads
-  const bool live = key < count;
-  // the key row goes into registers before the query staging, so its loads
-  // overlap the staging and its barrier
-  uint4 kr[kMaxHeadDim / 8] = {};
-  const uint16_t* krow = k_cache + (((first + (live ? key : 0)) % cap) * nkv + kvh) * d;
-#pragma unroll
-  for (int c = 0; c < kMaxHeadDim / 8; ++c)
-    if (live && c * 8 < d) kr[c] = *reinterpret_cast<const uint4*>(krow + c * 8);
-  for (int i = threadIdx.x; i < g * d; i += blockDim.x) qs[i / d][i % d] = bf(q[(int64_t)(kvh * g + i / d) * d + i % d]);
-  __syncthreads();
-  if (!live) return;
-  for (int hh = part; hh < g; hh += kAttnThreads / kScoreKeys) {
-    double acc = 0.0;
-#pragma unroll
-    for (int c = 0; c < kMaxHeadDim / 8; ++c) {
-      if (c * 8 >= d) break;
-      // opaque per head: the conversions stay in the loop instead of being
-      // hoisted as 128 float64 values
-      uint32_t wd[4] = {kr[c].x, kr[c].y, kr[c].z, kr[c].w};
-      asm volatile("" : "+v"(wd[0]), "+v"(wd[1]), "+v"(wd[2]), "+v"(wd[3]));
-#pragma unroll
-      for (int t = 0; t < 4; ++t) {
-        acc = fma((double)kv_f((uint16_t)(wd[t] & 0xffffu), f16), (double)qs[hh][8 * c + 2 * t], acc);
-        acc = fma((double)kv_f((uint16_t)(wd[t] >> 16), f16), (double)qs[hh][8 * c + 2 * t + 1], acc);
-      }
-    }
-    scores[(int64_t)(kvh * g + hh) * count + key] = (float)acc / sqrt_d;
   }
 }
 
@@ -158,25 +125,20 @@ __device__ __forceinline__ void head_stats(const float* __restrict__ s, int coun
   l_out = (float)t;
 }
 
-// The body of a value workgroup: partial[h][split][d] = sum over the
-// split's keys of p * v, p rounded to the cache type, for query head
-// h = blockIdx.x whose `count` scores s_head holds (global memory or LDS).
-// The workgroup first takes its head's max and sum over all the scores
-// (16 KB of L2 reads at 4,096 keys: cheaper than a launch of its own).
-// kWhole (count <= 256, one split): it also writes the context, so the step
-// needs no combine launch.
-template <bool kWhole>
+// The value half of a window workgroup: the context of query head
+// h = blockIdx.x whose `count` <= 256 scores s_head (LDS) holds; p rounded to
+// the cache type, the slices' float32 sums in `partial` [h][d].
 __device__ __forceinline__ void pv_body(const float* __restrict__ s_head, const uint16_t* __restrict__ sinks,
                                         const uint16_t* __restrict__ v_cache, float* __restrict__ partial,
                                         uint16_t* __restrict__ context, int64_t cap, int64_t first, int count, int nh,
                                         int nkv, int d, bool f16) {
   __shared__ float p[kPvKeys];
   __shared__ float acc_s[kAttnThreads / 32][kMaxHeadDim];
-  const int h = blockIdx.x, split = blockIdx.y, g = nh / nkv, kvh = h / g;
-  const int k0 = split * kPvKeys, nk = min(kPvKeys, count - k0);
+  const int h = blockIdx.x, g = nh / nkv, kvh = h / g;
+  const int nk = count;
   float m, l;
   head_stats(s_head, count, sinks, h, m, l);
-  for (int i = threadIdx.x; i < nk; i += kAttnThreads) p[i] = rkv(expf(s_head[k0 + i] - m) / l, f16);
+  for (int i = threadIdx.x; i < nk; i += kAttnThreads) p[i] = rkv(expf(s_head[i] - m) / l, f16);
   __syncthreads();
   // thread (slice, four dims): slices of keys; each thread issues the 8-byte
   // loads of four keys before their multiply-adds, so L2 round trips overlap
@@ -184,7 +146,7 @@ __device__ __forceinline__ void pv_body(const float* __restrict__ s_head, const 
   const int dq = threadIdx.x % quads, sl = threadIdx.x / quads;
   float a[4] = {0.f, 0.f, 0.f, 0.f};
   auto vrow = [&](int i) {
-    return *reinterpret_cast<const uint2*>(v_cache + (((first + k0 + i) % cap) * nkv + kvh) * d + 4 * dq);
+    return *reinterpret_cast<const uint2*>(v_cache + (((first + i) % cap) * nkv + kvh) * d + 4 * dq);
   };
   auto add = [&](float pi, uint2 w) {
     a[0] = fmaf(pi, kv_f((uint16_t)(w.x & 0xffffu), f16), a[0]);
@@ -213,28 +175,13 @@ __device__ __forceinline__ void pv_body(const float* __restrict__ s_head, const 
     if ((int)threadIdx.x < d) {
       float t = 0.f;
       for (int s2 = 0; s2 < min(kAttnThreads / 32, slices - base); ++s2) t += acc_s[s2][threadIdx.x];
-      float* out = partial + ((int64_t)h * gridDim.y + split) * d + threadIdx.x;
+      float* out = partial + (int64_t)h * d + threadIdx.x;
       *out = base == 0 ? t : *out + t;
     }
     __syncthreads();
   }
-  if constexpr (kWhole) {
-    if ((int)threadIdx.x < d) {
-      const float t = partial[((int64_t)h * gridDim.y + split) * d + threadIdx.x];
-      context[(int64_t)h * d + threadIdx.x] = to_bf(rkv(t, f16));
-    }
-  }
-}
-
-__global__ __launch_bounds__(kAttnThreads) void attn_pv_kernel(const float* __restrict__ scores,
-                                                               const uint16_t* __restrict__ sinks,
-                                                               const uint16_t* __restrict__ v_cache,
-                                                               float* __restrict__ partial,
-                                                               uint16_t* __restrict__ context, int64_t cap,
-                                                               int64_t first, int count, int nh, int nkv, int d,
-                                                               bool f16) {
-  pv_body<false>(scores + (int64_t)blockIdx.x * count, sinks, v_cache, partial, context, cap, first, count, nh, nkv,
-                 d, f16);
+  if ((int)threadIdx.x < d)
+    context[(int64_t)h * d + threadIdx.x] = to_bf(rkv(partial[(int64_t)h * d + threadIdx.x], f16));
 }
 
 // A window of at most 256 keys in one launch: workgroup = query head
@@ -272,32 +219,280 @@ __global__ __launch_bounds__(kAttnThreads) void attn_window_kernel(
     sc[key] = (float)acc / sqrt_d;
   }
   __syncthreads();
-  pv_body<true>(sc, sinks, v_cache, partial, context, cap, first, count, nh, nkv, d, f16);
+  pv_body(sc, sinks, v_cache, partial, context, cap, first, count, nh, nkv, d, f16);
 }
 
-// context[h][d] = bf16(sum over splits of partial[h][split][d])
-__global__ __launch_bounds__(kAttnThreads) void attn_combine_kernel(const float* __restrict__ partial, int splits,
-                                                                    int nh, int d, uint16_t* __restrict__ context,
-                                                                    bool f16) {
-  const int i = blockIdx.x * blockDim.x + threadIdx.x;
-  if (i >= nh * d) return;
-  const int h = i / d, e = i - h * d;
-  const float* src = partial + (int64_t)h * splits * d + e;
-  // 8 loads in flight, summed in split order
-  double t = 0.0;
-  int s = 0;
-  for (; s + 7 < splits; s += 8) {
-    float x[8];
+// ring slot of key i of a span starting at slot `first`
+__device__ __forceinline__ int64_t ring_slot(int64_t first, int64_t i, int64_t cap) {
+  const int64_t s = first + i;
+  return s >= cap ? s - cap : s;
+}
+
+// 8 elements of the cache type as float64 operands
+template <bool kF16>
+__device__ __forceinline__ double kv_d(const uint4& v, int i) {
+  const uint32_t w = i < 2 ? v.x : i < 4 ? v.y : i < 6 ? v.z : v.w;
+  return (double)kv_f((uint16_t)((i & 1) ? w >> 16 : w & 0xffffu), kF16);
+}
+
+// Scores of one KV head's query group against 64 * T keys (blockIdx.y), and
+// per head the block's maximum and sum of exp(score - maximum).
+//
+// A wave multiplies 16-key tiles with v_mfma_f64_16x16x4_f64: A = keys (lane
+// l holds key row l % 16, dims 32 c + 8 (l / 16) + i), B = the group's
+// queries (column l % 16, same dims), so every key element is converted to
+// float64 once for all heads (a vector dot product per head converted it g
+// times), and 16 lanes' loads cover 64 contiguous bytes of each key.  D lane l register i is
+// row l / 16 + 4 i; tile row m holds key 4 (m % 4) + m / 4, so a lane ends up
+// with 4 consecutive keys of head l % 16 and stores them as one float4.
+// Groups of fewer than 16 heads leave MFMA columns idle.
+template <int T, bool kF16>
+__global__ __launch_bounds__(kAttnThreads) void attn_scores_kernel(
+    const uint16_t* __restrict__ q, const uint16_t* __restrict__ k_cache, float* __restrict__ scores,
+    float* __restrict__ stat_m, double* __restrict__ stat_l, int64_t cap, int64_t first, int count, int cs, int nh,
+    int nkv, int d, float sqrt_d) {
+  __shared__ __align__(16) uint16_t qs[kMaxGroup][kMaxHeadDim + 8];
+  __shared__ float wm[kAttnThreads / kWave][kMaxGroup];
+  __shared__ double wl[kAttnThreads / kWave][kMaxGroup];
+  const int g = nh / nkv, kvh = blockIdx.x, blk = blockIdx.y;
+  const int lane = threadIdx.x % kWave, wave = threadIdx.x / kWave;
+  const int r = lane & 15, kq = lane >> 4;  // MFMA row / column, dim quarter
+  const int key0 = (blk * (kAttnThreads / kWave) + wave) * 16 * T;
+  constexpr int kC = kMaxHeadDim / 32;
+  // dims 32 c + 8 kq of the head exist: d is a multiple of 8
+  uint4 kr[T][kC];
 #pragma unroll
-    for (int j = 0; j < 8; ++j) x[j] = src[(int64_t)(s + j) * d];
+  for (int t = 0; t < T; ++t) {
+    const int key = min(key0 + 16 * t + 4 * (r & 3) + (r >> 2), count - 1);
+    const uint16_t* row = k_cache + (ring_slot(first, key, cap) * nkv + kvh) * d + 8 * kq;
 #pragma unroll
-    for (int j = 0; j < 8; ++j) t += x[j];
+    for (int c = 0; c < kC; ++c)
+      kr[t][c] = 32 * c + 8 * kq < d ? *reinterpret_cast<const uint4*>(row + 32 * c) : make_uint4(0, 0, 0, 0);
   }
-  for (; s < splits; ++s) t += src[(int64_t)s * d];
-  context[i] = to_bf(rkv((float)t, f16));  // the cache type's einsum result, then bfloat16
+  for (int i = threadIdx.x; i < g * d; i += kAttnThreads) qs[i / d][i % d] = q[(int64_t)kvh * g * d + i];
+  __syncthreads();
+  uint4 qr[kC];
+#pragma unroll
+  for (int c = 0; c < kC; ++c) {
+    qr[c] = make_uint4(0, 0, 0, 0);
+    if (32 * c + 8 * kq < d && r < g) qr[c] = *reinterpret_cast<const uint4*>(&qs[r][32 * c + 8 * kq]);
+  }
+  f64x4_t acc[T] = {};
+#pragma unroll
+  for (int c = 0; c < kC; ++c) {
+    if (32 * c >= d) break;
+#pragma unroll
+    for (int i = 0; i < 8; ++i) {
+      const double qd = kv_d<false>(qr[c], i);
+#pragma unroll
+      for (int t = 0; t < T; ++t)
+        acc[t] = __builtin_amdgcn_mfma_f64_16x16x4f64(kv_d<kF16>(kr[t][c], i), qd, acc[t], 0, 0, 0);
+    }
+  }
+  const int h = kvh * g + r;
+  float s[T][4];
+  float m = -INFINITY;
+#pragma unroll
+  for (int t = 0; t < T; ++t) {
+    const int k4 = key0 + 16 * t + 4 * kq;
+#pragma unroll
+    for (int i = 0; i < 4; ++i) {
+      s[t][i] = (float)acc[t][i] / sqrt_d;
+      if (k4 + i < count) m = fmaxf(m, s[t][i]);
+    }
+    if (r < g && k4 < count)  // rows are padded to 4 scores
+      *reinterpret_cast<float4*>(scores + (int64_t)h * cs + k4) = make_float4(s[t][0], s[t][1], s[t][2], s[t][3]);
+  }
+  m = fmaxf(m, __shfl_xor(m, 16));
+  m = fmaxf(m, __shfl_xor(m, 32));
+  if (kq == 0) wm[wave][r] = m;
+  __syncthreads();
+  m = wm[0][r];
+  for (int w = 1; w < kAttnThreads / kWave; ++w) m = fmaxf(m, wm[w][r]);
+  // a block of -inf scores adds nothing (and NaN stays NaN)
+  const float base = m == -INFINITY ? 0.f : m;
+  double l = 0.0;
+#pragma unroll
+  for (int t = 0; t < T; ++t)
+#pragma unroll
+    for (int i = 0; i < 4; ++i)
+      if (key0 + 16 * t + 4 * kq + i < count) l += (double)expf(s[t][i] - base);
+  l += __shfl_xor(l, 16);
+  l += __shfl_xor(l, 32);
+  if (kq == 0) wl[wave][r] = l;
+  __syncthreads();
+  if ((int)threadIdx.x < g) {
+    double sum = 0.0;
+    for (int w = 0; w < kAttnThreads / kWave; ++w) sum += wl[w][r];
+    const int64_t at = (int64_t)h * gridDim.y + blk;
+    stat_m[at] = m;
+    stat_l[at] = sum;
+  }
 }
 
-int64_t attn_splits(int64_t count) { return (count + kPvKeys - 1) / kPvKeys; }
+// partial[h][split][d] = sum over the split's keys of p * v for the heads of
+// one KV head (blockIdx.x), p = exp(score - max) / sum rounded to the cache
+// type.  Each value row is read once per 4 heads: thread (8 dims, block of 4
+// heads, key slot).  The head's max and sum come from the score blocks'
+// (a few KB instead of all its scores): 186 -> 18.8 us at 32,768 keys.
+template <bool kF16>
+__global__ __launch_bounds__(kAttnThreads) void attn_pv_kernel(
+    const float* __restrict__ scores, const float* __restrict__ stat_m, const double* __restrict__ stat_l, int nblk,
+    const uint16_t* __restrict__ sinks, const uint16_t* __restrict__ v_cache, float* __restrict__ partial, int64_t cap,
+    int64_t first, int count, int cs, int ks_log2, int nh, int nkv, int d) {
+  const int ks = 1 << ks_log2;
+  // p [key][heads, 16-byte blocks, one spare to spread the banks], then, past
+  // a barrier, the slots' sums [slot][head][d]
+  constexpr int kRed = kAttnThreads * 32;
+  __shared__ __align__(16) float lds[kRed];
+  static_assert(kPvKeys * (kMaxGroup + 4) <= kRed, "p fits");
+  __shared__ float head_m[kMaxGroup], head_l[kMaxGroup];
+  float* const p = lds;
+  float* const red = lds;
+  const int g = nh / nkv, kvh = blockIdx.x, split = blockIdx.y;
+  const int k0 = split * ks, nk = min(ks, count - k0);
+  const int dl = d / 8, hb = (g + 3) / 4, slots = kAttnThreads / (dl * hb);
+  const int dq = threadIdx.x % dl, hblk = threadIdx.x / dl % hb, slot = threadIdx.x / (dl * hb);
+  const bool live = slot < slots;
+  auto vrow = [&](int i) {
+    return *reinterpret_cast<const uint4*>(v_cache + (ring_slot(first, k0 + i, cap) * nkv + kvh) * d + 8 * dq);
+  };
+  // the first value rows are on their way while the statistics are taken
+  constexpr int kAhead = 8;
+  uint4 v[kAhead];
+#pragma unroll
+  for (int j = 0; j < kAhead; ++j) v[j] = vrow(min(slot + j * slots, nk - 1));
+
+  // 16 to 256 lanes a head take its statistics, every head at once
+  const int lanes = g > 8 ? 16 : g > 4 ? 32 : 64;
+  {
+    const int hh = threadIdx.x / lanes, ln = threadIdx.x % lanes;
+    const int h = kvh * g + min(hh, g - 1);
+    const float* sm = stat_m + (int64_t)h * nblk;
+    const double* sl = stat_l + (int64_t)h * nblk;
+    const float sink = sinks != nullptr ? bf(sinks[h]) : -INFINITY;
+    constexpr int kHold = 4;
+    float bm[kHold];
+    double bl[kHold];
+#pragma unroll
+    for (int j = 0; j < kHold; ++j) {
+      const int b = ln + j * lanes;
+      bm[j] = b < nblk ? sm[b] : -INFINITY;
+      bl[j] = b < nblk ? sl[b] : 0.0;
+    }
+    float m = sink;
+#pragma unroll
+    for (int j = 0; j < kHold; ++j) m = fmaxf(m, bm[j]);
+    for (int b = ln + kHold * lanes; b < nblk; b += lanes) m = fmaxf(m, sm[b]);
+    for (int off = lanes / 2; off > 0; off >>= 1) m = fmaxf(m, __shfl_xor(m, off));
+    double l = 0.0;
+#pragma unroll
+    for (int j = 0; j < kHold; ++j)
+      if (ln + j * lanes < nblk) l += bl[j] * (double)expf(bm[j] - m);
+    for (int b = ln + kHold * lanes; b < nblk; b += lanes) l += sl[b] * (double)expf(sm[b] - m);
+    for (int off = lanes / 2; off > 0; off >>= 1) l += __shfl_xor(l, off);
+    if (sinks != nullptr) l += (double)expf(sink - m);
+    if (ln == 0 && hh < g) head_m[hh] = m, head_l[hh] = (float)l;
+  }
+  const int stride = 4 * hb + 4;
+  __syncthreads();
+#pragma unroll 4
+  for (int i = threadIdx.x; i < ks * 4 * hb; i += kAttnThreads) {
+    const int hh = i >> ks_log2, key = i & (ks - 1);
+    float w = 0.f;
+    if (hh < g && key < nk)
+      w = rkv(expf(scores[(int64_t)(kvh * g + hh) * cs + k0 + key] - head_m[hh]) / head_l[hh], kF16);
+    p[key * stride + hh] = w;
+  }
+  __syncthreads();
+  float a[4][8] = {};
+  if (live) {
+    for (int i0 = slot; i0 < nk; i0 += kAhead * slots) {
+      if (i0 != slot) {
+#pragma unroll
+        for (int j = 0; j < kAhead; ++j) v[j] = vrow(min(i0 + j * slots, nk - 1));
+      }
+#pragma unroll
+      for (int j = 0; j < kAhead; ++j) {
+        if (i0 + j * slots >= nk) break;
+        const float4 w = *reinterpret_cast<const float4*>(p + (i0 + j * slots) * stride + 4 * hblk);
+#pragma unroll
+        for (int e = 0; e < 8; ++e) {
+          const uint32_t x = e < 2 ? v[j].x : e < 4 ? v[j].y : e < 6 ? v[j].z : v[j].w;
+          const float f = kv_f((uint16_t)((e & 1) ? x >> 16 : x & 0xffffu), kF16);
+          a[0][e] = fmaf(w.x, f, a[0][e]);
+          a[1][e] = fmaf(w.y, f, a[1][e]);
+          a[2][e] = fmaf(w.z, f, a[2][e]);
+          a[3][e] = fmaf(w.w, f, a[3][e]);
+        }
+      }
+    }
+  }
+  __syncthreads();
+  if (live) {
+#pragma unroll
+    for (int hh = 0; hh < 4; ++hh) {
+      float4* dst = reinterpret_cast<float4*>(red + ((slot * hb + hblk) * 4 + hh) * d + 8 * dq);
+      dst[0] = make_float4(a[hh][0], a[hh][1], a[hh][2], a[hh][3]);
+      dst[1] = make_float4(a[hh][4], a[hh][5], a[hh][6], a[hh][7]);
+    }
+  }
+  __syncthreads();
+  for (int i = threadIdx.x; i < g * d; i += kAttnThreads) {
+    float t = 0.f;
+    for (int s = 0; s < slots; ++s) t += red[s * hb * 4 * d + i];
+    partial[((int64_t)(kvh * g + i / d) * gridDim.y + split) * d + i % d] = t;
+  }
+}
+
+// context[h][d] = bf16(sum over splits of partial[h][split][d]): one
+// workgroup per head, thread (4 dims, group of splits), summed in float64.
+__global__ __launch_bounds__(kAttnThreads) void attn_combine_kernel(const float* __restrict__ partial, int splits,
+                                                                    int d, uint16_t* __restrict__ context, bool f16) {
+  __shared__ double red[kAttnThreads * 4];
+  const int h = blockIdx.x, quads = d / 4, groups = kAttnThreads / quads;
+  const int dq = threadIdx.x % quads, grp = threadIdx.x / quads;
+  const float* src = partial + (int64_t)h * splits * d + 4 * dq;
+  if (grp < groups) {
+    double t[4] = {0.0, 0.0, 0.0, 0.0};
+    constexpr int kAhead = 8;
+    for (int s0 = grp; s0 < splits; s0 += kAhead * groups) {
+      float4 x[kAhead];
+#pragma unroll
+      for (int j = 0; j < kAhead; ++j)
+        x[j] = *reinterpret_cast<const float4*>(src + (int64_t)min(s0 + j * groups, splits - 1) * d);
+#pragma unroll
+      for (int j = 0; j < kAhead; ++j)
+        if (s0 + j * groups < splits) t[0] += x[j].x, t[1] += x[j].y, t[2] += x[j].z, t[3] += x[j].w;
+    }
+#pragma unroll
+    for (int e = 0; e < 4; ++e) red[grp * d + 4 * dq + e] = t[e];
+  }
+  __syncthreads();
+  if ((int)threadIdx.x < d) {
+    double t = 0.0;
+    for (int s = 0; s < groups; ++s) t += red[s * d + threadIdx.x];
+    context[(int64_t)h * d + threadIdx.x] = to_bf(rkv((float)t, f16));  // the cache type's einsum result, then bfloat16
+  }
+}
+
+// Scratch of klc_attn_decode past one window: scores [heads][count rounded
+// up to 4], value partials [heads][splits][head_dim], then the score blocks'
+// sums (float64) and maxima.
+struct AttnPlan {
+  int64_t cs, score_keys, nblk, split_keys, splits;
+};
+AttnPlan attn_plan(int64_t count) {
+  AttnPlan a;
+  a.cs = (count + 3) / 4 * 4;
+  // 64 keys a workgroup keep the chip busy on shorter contexts; past 8,192
+  // keys 256 (fewer block statistics for every value workgroup to read)
+  a.score_keys = count <= 8192 ? 64 : 256;
+  a.nblk = (count + a.score_keys - 1) / a.score_keys;
+  a.split_keys = count <= 8192 ? 128 : kPvKeys;
+  a.splits = (count + a.split_keys - 1) / a.split_keys;
+  return a;
+}
 
 }  // namespace
 }  // namespace klc
@@ -331,7 +526,9 @@ extern "C" int klc_rope_append(const void* q, const void* k, const void* v, cons
 extern "C" int64_t klc_attn_workspace_bytes(int64_t n_heads, int64_t head_dim, int64_t count) {
   if (n_heads <= 0 || head_dim <= 0 || count <= 0)
     return set_error(KLC_ERR_ARGUMENT, "klc_attn_workspace_bytes: bad sizes");
-  return 4 * (n_heads * count + n_heads * attn_splits(count) * head_dim);
+  if (count <= kPvKeys) return 4 * n_heads * (count + head_dim);
+  const AttnPlan a = attn_plan(count);
+  return n_heads * (4 * a.cs + 12 * a.nblk + 4 * a.splits * head_dim);
 }
 
 extern "C" int klc_attn_decode(const void* q, const void* k_cache, const void* v_cache, const void* sinks,
@@ -355,9 +552,6 @@ extern "C" int klc_attn_decode(const void* q, const void* k_cache, const void* v
   const int64_t need = klc_attn_workspace_bytes(n_heads, head_dim, count);
   KLC_REQUIRE(workspace_bytes >= need, KLC_ERR_ARGUMENT, "klc_attn_decode: workspace of %lld bytes, need %lld",
               (long long)workspace_bytes, (long long)need);
-  float* scores = static_cast<float*>(workspace);
-  float* partial = scores + n_heads * count;
-  const int splits = (int)attn_splits(count);
   hipStream_t st = as_stream(stream);
   const uint16_t* qb = static_cast<const uint16_t*>(q);
   const uint16_t* kb = static_cast<const uint16_t*>(k_cache);
@@ -365,20 +559,29 @@ extern "C" int klc_attn_decode(const void* q, const void* k_cache, const void* v
   const uint16_t* sk = static_cast<const uint16_t*>(sinks);
   uint16_t* ctx = static_cast<uint16_t*>(context);
   const float sqrt_d = sqrtf((float)head_dim);
-  if (splits == 1) {  // a window of at most 256 keys: one launch, one workgroup per query head
+  const int n = (int)count, nh = (int)n_heads, nkv = (int)n_kv, d = (int)head_dim;
+  if (count <= kPvKeys) {  // a window: one launch, one workgroup per query head
     static_assert(kPvKeys == kAttnThreads, "one key per thread");
     attn_window_kernel<<<(unsigned)n_heads, kAttnThreads, 0, st>>>(
-        qb, kb, sk, vb, partial, ctx, cap, first, (int)count, (int)n_heads, (int)n_kv, (int)head_dim, sqrt_d, f16);
+        qb, kb, sk, vb, static_cast<float*>(workspace), ctx, cap, first, n, nh, nkv, d, sqrt_d, f16);
     return check_launch("attn_window_kernel");
   }
-  attn_scores_kernel<<<dim3((unsigned)n_kv, (unsigned)((count + kScoreKeys - 1) / kScoreKeys)), kAttnThreads, 0, st>>>(
-      qb, kb, scores, cap, first, (int)count, (int)n_heads, (int)n_kv, (int)head_dim, sqrt_d, f16);
+  const AttnPlan a = attn_plan(count);
+  float* scores = static_cast<float*>(workspace);
+  float* partial = scores + n_heads * a.cs;
+  double* stat_l = reinterpret_cast<double*>(partial + n_heads * a.splits * head_dim);
+  float* stat_m = reinterpret_cast<float*>(stat_l + n_heads * a.nblk);
+  const dim3 sgrid((unsigned)n_kv, (unsigned)a.nblk), vgrid((unsigned)n_kv, (unsigned)a.splits);
+  auto run_scores = a.score_keys == 64 ? (f16 ? attn_scores_kernel<1, true> : attn_scores_kernel<1, false>)
+                                       : (f16 ? attn_scores_kernel<4, true> : attn_scores_kernel<4, false>);
+  run_scores<<<sgrid, kAttnThreads, 0, st>>>(qb, kb, scores, stat_m, stat_l, cap, first, n, (int)a.cs, nh, nkv, d,
+                                             sqrt_d);
   int rc = check_launch("attn_scores_kernel");
   if (rc) return rc;
-  attn_pv_kernel<<<dim3((unsigned)n_heads, (unsigned)splits), kAttnThreads, 0, st>>>(
-      scores, sk, vb, partial, ctx, cap, first, (int)count, (int)n_heads, (int)n_kv, (int)head_dim, f16);
+  auto run_pv = f16 ? attn_pv_kernel<true> : attn_pv_kernel<false>;
+  run_pv<<<vgrid, kAttnThreads, 0, st>>>(scores, stat_m, stat_l, (int)a.nblk, sk, vb, partial, cap, first, n,
+                                         (int)a.cs, a.split_keys == 128 ? 7 : 8, nh, nkv, d);
   if ((rc = check_launch("attn_pv_kernel"))) return rc;
-  attn_combine_kernel<<<(unsigned)((n_heads * head_dim + kAttnThreads - 1) / kAttnThreads), kAttnThreads, 0, st>>>(
-      partial, splits, (int)n_heads, (int)head_dim, static_cast<uint16_t*>(context), f16);
+  attn_combine_kernel<<<(unsigned)n_heads, kAttnThreads, 0, st>>>(partial, (int)a.splits, d, ctx, f16);
   return check_launch("attn_combine_kernel");
 }

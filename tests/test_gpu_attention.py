@@ -193,6 +193,60 @@ def test_other_head_shapes(gpu, nh, nkv, d, window):
     assert np.all(np.abs(got - ref) <= context_tolerance(ref, "bf16")), np.abs(got - ref).max()
 
 
+def decode_direct(gpu, q, k, v, sk, cap, first, count, kv):
+    """klc_attn_decode on ready tensors with a workspace of exactly the stated size, dirty."""
+    (nh, d), nkv = q.shape, k.shape[1]
+    ws = torch.full((_native.call("klc_attn_workspace_bytes", nh, d, count),), 255, dtype=torch.uint8, device=gpu)
+    ctx = torch.empty((nh, d), dtype=torch.bfloat16, device=gpu)
+    _native.call("klc_attn_decode", P(q.data_ptr()), P(k.data_ptr()), P(v.data_ptr()),
+                 P(0 if sk is None else sk.data_ptr()), cap, first, count, nh, nkv, d, 1 if kv == "fp16" else 0,
+                 P(ws.data_ptr()), ws.numel(), P(ctx.data_ptr()), P(torch.cuda.current_stream(gpu).cuda_stream))
+    return ctx
+
+
+@pytest.mark.parametrize("nh,nkv,d,count,kv", [
+    (64, 8, 64, 257, "fp16"), (64, 8, 64, 321, "bf16"), (64, 8, 64, 8192, "fp16"), (64, 8, 64, 8193, "fp16"),
+    (32, 2, 128, 8449, "bf16"), (32, 2, 128, 400, "fp16"), (12, 4, 24, 1000, "bf16"), (5, 1, 40, 8195, "fp16"),
+    (8, 8, 8, 700, "bf16"), (3, 3, 104, 9001, "bf16")])
+def test_split_decode_matches_oracle(gpu, nh, nkv, d, count, kv):
+    """Both score-block and value-split sizes (the line is at 8,192 keys), partial blocks, group
+    sizes 1 to 16, head dims that leave dim quarters and threads idle, a wrapped span."""
+    g = torch.Generator(device=gpu).manual_seed(count + d)
+    dt = torch.float16 if kv == "fp16" else torch.bfloat16
+    cap, first = count + 9, count - 3  # the span wraps after 12 keys
+    q = torch.randn(nh, d, generator=g, device=gpu).to(torch.bfloat16)
+    k, v = (torch.randn(cap, nkv, d, generator=g, device=gpu).to(dt) for _ in range(2))
+    sk = torch.randn(nh, generator=g, device=gpu).to(torch.bfloat16)
+    ctx = decode_direct(gpu, q, k, v, sk, cap, first, count, kv)
+    idx = (torch.arange(count, device=gpu) + first) % cap
+    kd, vd = k[idx].double(), v[idx].double()
+    s = torch.einsum("gjd,tgd->gjt", q.double().cpu().view(nkv, nh // nkv, d), kd.cpu()).reshape(nh, count)
+    s = torch.cat((s.float() / np.float32(np.sqrt(d)), sk.float().cpu()[:, None]), dim=1)
+    p = torch.softmax(s.double(), dim=1)[:, :-1].float().to(dt).double().view(nkv, nh // nkv, count)
+    ref = torch.einsum("gjt,tgd->gjd", p, vd.cpu()).reshape(nh, d)
+    ref = ref.float().to(dt).to(torch.bfloat16).float().numpy()
+    got = ctx.float().cpu().numpy()
+    assert np.all(np.abs(got - ref) <= context_tolerance(ref, kv)), np.abs(got - ref).max()
+
+
+def test_split_decode_infinite_scores(gpu):
+    """A score block that is -inf throughout weighs nothing; a NaN key makes its KV head's queries NaN."""
+    nh, nkv, d, count = 16, 2, 64, 600
+    g = torch.Generator(device=gpu).manual_seed(1)
+    q = torch.full((nh, d), 3e38, device=gpu).to(torch.bfloat16)
+    k = torch.zeros(count, nkv, d, device=gpu, dtype=torch.bfloat16)
+    k[64:256] = -3e38
+    v = torch.randn(count, nkv, d, generator=g, device=gpu).to(torch.bfloat16)
+    ctx = decode_direct(gpu, q, k, v, None, count, 0, count, "bf16").float()
+    keep = torch.cat((v[:64], v[256:])).float()
+    p = torch.tensor(1.0 / keep.shape[0]).to(torch.bfloat16).item()
+    ref = (p * keep.sum(dim=0)).repeat_interleave(nh // nkv, dim=0)
+    assert torch.allclose(ctx, ref, rtol=2.0 ** -7, atol=2.0 ** -9)
+    k[300, 1, 5] = float("nan")
+    ctx = decode_direct(gpu, q, k, v, None, count, 0, count, "bf16").float()
+    assert torch.isfinite(ctx[: nh // 2]).all() and torch.isnan(ctx[nh // 2:]).all()
+
+
 def test_attention_rejects_bad_shapes(gpu):
     x = torch.zeros(4096, dtype=torch.bfloat16, device=gpu)
     ws = torch.zeros(1 << 16, dtype=torch.uint8, device=gpu)
