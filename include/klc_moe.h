@@ -442,6 +442,34 @@ int klc_attn_decode(const void* q, const void* k_cache, const void* v_cache, con
                     int64_t first, int64_t count, int64_t n_heads, int64_t n_kv, int64_t head_dim, int kv_dtype,
                     void* workspace, int64_t workspace_bytes, void* context, void* stream);
 
+/* One decode token of StreamedAttention.forward (streamed_attention.py:101-152)
+ * in one call: q, k, v = bf16(x . w + bias) (correctly rounded sums), RoPE
+ * with the position's angles (float32 inv_freq[j] * position; cos and sin
+ * times rope_scale, rounded to bfloat16), the append of k and v to ring slot
+ * `slot`, klc_attn_decode over `count` keys from slot `first` (the appended
+ * one included), and out = bf16(context . o_weight + o_bias).  host_record
+ * (pinned host memory, or NULL): 9 words the device writes while the step
+ * runs: float32 norms |q|, |k| before RoPE, |q|, |k| after it, |q after - q|,
+ * |k after - k|, int32 counts of non-finite q and k values after it, then
+ * `tag` (not 0; the caller clears that word first).  Biases and sinks may be
+ * NULL.  hidden_size and n_heads * head_dim multiples of 8, at most 4096;
+ * hidden, weights, caches and workspace 16-byte aligned; other limits as
+ * klc_attn_decode's. */
+typedef struct klc_attn_step_args {
+  const void *hidden;                          /* bfloat16 [hidden_size] */
+  const void *q_weight, *q_bias;               /* bfloat16 [n_heads * head_dim][hidden_size], [n_heads * head_dim] */
+  const void *k_weight, *k_bias, *v_weight, *v_bias; /* [n_kv * head_dim][hidden_size], [n_kv * head_dim] */
+  const void *o_weight, *o_bias;               /* [out_size][n_heads * head_dim], [out_size] */
+  const void *sinks;                           /* bfloat16 [n_heads] */
+  const void *inv_freq;                        /* float32 [head_dim / 2], on the device */
+  void *k_cache, *v_cache;                     /* [cap][n_kv][head_dim] of kv_dtype */
+  void *workspace, *out, *host_record;
+  int64_t hidden_size, out_size, n_heads, n_kv, head_dim, cap, slot, first, count, kv_dtype, workspace_bytes, tag;
+  double position, rope_scale;
+} klc_attn_step_args;
+int64_t klc_attn_step_workspace_bytes(int64_t n_heads, int64_t n_kv, int64_t head_dim, int64_t count);
+int klc_attn_step(const klc_attn_step_args* args, void* stream);
+
 /* ---- Synthetic inputs -------------------------------------------------------
  * Counter-based SplitMix64 stream, identical to klcquant_amd/synth.py:
  * mode 0: n random bytes; mode 1: n bytes uniform in [lo, hi]. */

@@ -37,6 +37,7 @@ constexpr int kAttnThreads = 256;
 constexpr int kPvKeys = 256;     // most keys of a value workgroup, and of a one-launch window
 constexpr int kMaxHeadDim = 128;
 constexpr int kMaxGroup = 16;    // query heads per KV head
+constexpr int kMaxRow = 8 * 8 * kWave;  // longest projection input: 8 chunks of 16 bytes a lane
 typedef double f64x4_t __attribute__((ext_vector_type(4)));
 
 __device__ __forceinline__ float bf(uint16_t b) { return __uint_as_float((uint32_t)b << 16); }
@@ -75,6 +76,206 @@ __global__ __launch_bounds__(kAttnThreads) void rope_append_kernel(
       v_cache[slot * nkv * d + e] = f16 ? to_kv(bf(v[e]), true) : v[e];
     }
   }
+}
+
+// ---- one decode step's projections ------------------------------------------
+
+// Dot products of two bfloat16 rows with the bfloat16 x [k], by one wave: lane
+// l takes the 16-byte chunks l, l + 64, ...; all 3 J loads are issued by
+// load(), so a caller can work under them.  A product of two bfloat16 values
+// is exact in float64 and the sum is taken there, so what the caller rounds
+// is the correctly rounded dot product (the float64 work rides under the
+// weight stream).  Lanes past a row's end read zeros.  Every lane gets both
+// sums.
+template <int J>
+struct TwoRows {
+  u32x4_t xv[J], v0[J], v1[J];
+
+  __device__ __forceinline__ void load(const uint16_t* w0, const uint16_t* w1, const uint16_t* x, int k) {
+    const int lane = threadIdx.x % kWave;
+    const __amdgpu_buffer_rsrc_t xb = __builtin_amdgcn_make_buffer_rsrc((void*)x, (short)0, k * 2, kBufferWord3);
+    const __amdgpu_buffer_rsrc_t b0 = __builtin_amdgcn_make_buffer_rsrc((void*)w0, (short)0, k * 2, kBufferWord3);
+    const __amdgpu_buffer_rsrc_t b1 = __builtin_amdgcn_make_buffer_rsrc((void*)w1, (short)0, k * 2, kBufferWord3);
+#pragma unroll
+    for (int j = 0; j < J; ++j) {
+      const uint32_t at = (uint32_t)(lane + kWave * j) * 16u;
+      v0[j] = __builtin_amdgcn_raw_buffer_load_b128(b0, at, 0, kStreamPolicy);
+      v1[j] = __builtin_amdgcn_raw_buffer_load_b128(b1, at, 0, kStreamPolicy);
+      xv[j] = __builtin_amdgcn_raw_buffer_load_b128(xb, at, 0, 0);
+    }
+  }
+
+  __device__ __forceinline__ void dot(double& sum0, double& sum1) const {
+    double a0[2] = {0.0, 0.0}, a1[2] = {0.0, 0.0};
+#pragma unroll
+    for (int j = 0; j < J; ++j) {
+#pragma unroll
+      for (int i = 0; i < 4; ++i) {
+        const double xl = (double)__uint_as_float(xv[j][i] << 16), xh = (double)__uint_as_float(xv[j][i] & 0xffff0000u);
+        a0[0] = fma((double)__uint_as_float(v0[j][i] << 16), xl, a0[0]);
+        a1[0] = fma((double)__uint_as_float(v1[j][i] << 16), xl, a1[0]);
+        a0[1] = fma((double)__uint_as_float(v0[j][i] & 0xffff0000u), xh, a0[1]);
+        a1[1] = fma((double)__uint_as_float(v1[j][i] & 0xffff0000u), xh, a1[1]);
+      }
+    }
+    sum0 = a0[0] + a0[1];
+    sum1 = a1[0] + a1[1];
+#pragma unroll
+    for (int off = kWave / 2; off > 0; off >>= 1) {
+      sum0 += __shfl_xor(sum0, off);
+      sum1 += __shfl_xor(sum1, off);
+    }
+  }
+};
+
+__device__ __forceinline__ float bias_at(const uint16_t* bias, int row) {
+  return bias != nullptr ? bf(bias[row]) : 0.f;
+}
+__device__ __forceinline__ uint16_t biased_bf(double sum, float bias) { return to_bf((float)(sum + (double)bias)); }
+
+struct QkvArgs {
+  const uint16_t *x, *qw, *qb, *kw, *kb, *vw, *vb;
+  const float* inv_freq;      // [d / 2]
+  uint16_t *pre, *rot;        // [nh + nkv][d] queries then keys, before and after RoPE
+  uint16_t *k_cache, *v_cache;
+  int64_t slot;
+  int hidden, nh, nkv, d;
+  float position, rope_scale;
+  bool f16;
+};
+
+// q, k and v projections of one token with RoPE and the append in the
+// epilogue: a wave owns the two rows of one rotated pair (dims j and j +
+// d / 2 of a head), or two value rows, so the rotation needs nothing from
+// another wave and the step has no launch for it.  cos and sin are taken
+// while the rows are on their way, with torch's rounding points (float32
+// angle, float32 product with the scaling, bfloat16).
+template <int J>
+__global__ __launch_bounds__(kAttnThreads) void attn_qkv_kernel(QkvArgs a) {
+  const int half = a.d / 2, pairs = (a.nh + a.nkv) * half;
+  const int p = blockIdx.x * (kAttnThreads / kWave) + __builtin_amdgcn_readfirstlane(threadIdx.x / kWave);
+  if (p >= pairs + a.nkv * half) return;
+  TwoRows<J> rows;
+  double s0, s1;
+  if (p >= pairs) {
+    const int r0 = 2 * (p - pairs);
+    const uint16_t* w = a.vw + (int64_t)r0 * a.hidden;
+    rows.load(w, w + a.hidden, a.x, a.hidden);
+    const float b0 = bias_at(a.vb, r0), b1 = bias_at(a.vb, r0 + 1);
+    rows.dot(s0, s1);
+    if (threadIdx.x % kWave == 0) {
+      uint16_t* dst = a.v_cache + a.slot * a.nkv * a.d + r0;
+      const uint16_t v0 = biased_bf(s0, b0), v1 = biased_bf(s1, b1);
+      dst[0] = a.f16 ? to_kv(bf(v0), true) : v0;
+      dst[1] = a.f16 ? to_kv(bf(v1), true) : v1;
+    }
+    return;
+  }
+  const int head = p / half, j = p - head * half;
+  const bool is_q = head < a.nh;
+  const int row = (is_q ? head : head - a.nh) * a.d + j;
+  const uint16_t* w = (is_q ? a.qw : a.kw) + (int64_t)row * a.hidden;
+  rows.load(w, w + (int64_t)half * a.hidden, a.x, a.hidden);
+  const uint16_t* b = is_q ? a.qb : a.kb;
+  const float b0 = bias_at(b, row), b1 = bias_at(b, row + half);
+  const float angle = __fmul_rn(a.inv_freq[j], a.position);
+  const float c = rbf(__fmul_rn(cosf(angle), a.rope_scale)), s = rbf(__fmul_rn(sinf(angle), a.rope_scale));
+  rows.dot(s0, s1);
+  if (threadIdx.x % kWave == 0) {
+    const uint16_t pl = biased_bf(s0, b0), ph = biased_bf(s1, b1);
+    const float x0 = bf(pl), x1 = bf(ph);
+    const float lo = rbf(rbf(x0 * c) - rbf(x1 * s)), hi = rbf(rbf(x1 * c) + rbf(x0 * s));  // bfloat16 rotation
+    const int at = head * a.d + j;
+    a.pre[at] = pl;
+    a.pre[at + half] = ph;
+    a.rot[at] = to_bf(lo);
+    a.rot[at + half] = to_bf(hi);
+    if (!is_q) {
+      uint16_t* dst = a.k_cache + a.slot * a.nkv * a.d + row;
+      dst[0] = to_kv(lo, a.f16);
+      dst[half] = to_kv(hi, a.f16);
+    }
+  }
+}
+
+// out[r] = bf16(x . w[r] + bias[r]) for a bfloat16 weight [rows][k]: two rows a wave
+template <int J>
+__global__ __launch_bounds__(kAttnThreads) void attn_out_kernel(const uint16_t* __restrict__ w,
+                                                                const uint16_t* __restrict__ bias,
+                                                                const uint16_t* __restrict__ x,
+                                                                uint16_t* __restrict__ out, int rows, int k) {
+  const int r0 = 2 * (blockIdx.x * (kAttnThreads / kWave) + __builtin_amdgcn_readfirstlane(threadIdx.x / kWave));
+  if (r0 >= rows) return;
+  const int r1 = min(r0 + 1, rows - 1);
+  TwoRows<J> two;
+  two.load(w + (int64_t)r0 * k, w + (int64_t)r1 * k, x, k);
+  const float b0 = bias_at(bias, r0), b1 = bias_at(bias, r1);
+  double s0, s1;
+  two.dot(s0, s1);
+  if (threadIdx.x % kWave == 0) {
+    out[r0] = biased_bf(s0, b0);
+    if (r1 > r0) out[r1] = biased_bf(s1, b1);
+  }
+}
+
+// What the host reads back from a step: the norms of q and k before RoPE,
+// after it and of the difference, the non-finite values after it, and a tag
+// word written last, all in pinned host memory.
+struct StepRecord {
+  const uint16_t *pre, *rot;  // [nh + nkv][d]
+  uint32_t* host;             // NULL: no record
+  uint32_t tag;
+};
+
+// One workgroup: sums of squares in float64 and the record.  It runs beside
+// the score workgroups of the same launch.
+__device__ __forceinline__ void write_record(const StepRecord& rec, int nh, int nkv, int d) {
+  __shared__ double sums[kAttnThreads / kWave][6];
+  __shared__ int bad[kAttnThreads / kWave][2];
+  const int lane = threadIdx.x % kWave, wave = threadIdx.x / kWave;
+  double t[6] = {};
+  int n[2] = {0, 0};
+  auto take = [&](int which, int from, int to) {
+    double pre = 0.0, post = 0.0, delta = 0.0;
+    int count = 0;
+    for (int i = from + threadIdx.x; i < to; i += kAttnThreads) {
+      const float x = bf(rec.pre[i]), y = bf(rec.rot[i]), z = y - x;
+      pre += (double)x * x;
+      post += (double)y * y;
+      delta += (double)z * z;
+      count += !isfinite(y);
+    }
+    t[which] = pre, t[2 + which] = post, t[4 + which] = delta, n[which] = count;
+  };
+  take(0, 0, nh * d);
+  take(1, nh * d, (nh + nkv) * d);
+#pragma unroll
+  for (int e = 0; e < 6; ++e)
+    for (int off = kWave / 2; off > 0; off >>= 1) t[e] += __shfl_xor(t[e], off);
+#pragma unroll
+  for (int e = 0; e < 2; ++e)
+    for (int off = kWave / 2; off > 0; off >>= 1) n[e] += __shfl_xor(n[e], off);
+  if (lane == 0) {
+    for (int e = 0; e < 6; ++e) sums[wave][e] = t[e];
+    for (int e = 0; e < 2; ++e) bad[wave][e] = n[e];
+  }
+  __syncthreads();
+  if (wave != 0) return;
+  if (lane < 8) {
+    uint32_t word;
+    if (lane < 6) {
+      double v = 0.0;
+      for (int w = 0; w < kAttnThreads / kWave; ++w) v += sums[w][lane];
+      word = __float_as_uint((float)sqrt(v));
+    } else {
+      int v = 0;
+      for (int w = 0; w < kAttnThreads / kWave; ++w) v += bad[w][lane - 6];
+      word = (uint32_t)v;
+    }
+    rec.host[lane] = word;
+  }
+  __threadfence_system();  // one wave wrote the record: its tag follows it
+  if (lane == 0) __hip_atomic_store(rec.host + 8, rec.tag, __ATOMIC_RELEASE, __HIP_MEMORY_SCOPE_SYSTEM);
 }
 
 // Query head h's m = max(scores, sink) and l = sum exp(x - m) over [scores,
@@ -191,7 +392,11 @@ __device__ __forceinline__ void pv_body(const float* __restrict__ s_head, const 
 __global__ __launch_bounds__(kAttnThreads) void attn_window_kernel(
     const uint16_t* __restrict__ q, const uint16_t* __restrict__ k_cache, const uint16_t* __restrict__ sinks,
     const uint16_t* __restrict__ v_cache, float* __restrict__ partial, uint16_t* __restrict__ context, int64_t cap,
-    int64_t first, int count, int nh, int nkv, int d, float sqrt_d, bool f16) {
+    int64_t first, int count, int nh, int nkv, int d, float sqrt_d, bool f16, StepRecord rec) {
+  if ((int)blockIdx.x == nh) {
+    write_record(rec, nh, nkv, d);
+    return;
+  }
   __shared__ float qs[kMaxHeadDim];
   __shared__ float sc[kPvKeys];
   const int h = blockIdx.x, kvh = h / (nh / nkv);
@@ -249,8 +454,12 @@ __device__ __forceinline__ double kv_d(const uint4& v, int i) {
 template <int T, bool kF16>
 __global__ __launch_bounds__(kAttnThreads) void attn_scores_kernel(
     const uint16_t* __restrict__ q, const uint16_t* __restrict__ k_cache, float* __restrict__ scores,
-    float* __restrict__ stat_m, double* __restrict__ stat_l, int64_t cap, int64_t first, int count, int cs, int nh,
-    int nkv, int d, float sqrt_d) {
+    float* __restrict__ stat_m, double* __restrict__ stat_l, int64_t cap, int64_t first, int count, int cs, int nblk,
+    int nh, int nkv, int d, float sqrt_d, StepRecord rec) {
+  if ((int)blockIdx.y == nblk) {
+    if (blockIdx.x == 0) write_record(rec, nh, nkv, d);
+    return;
+  }
   __shared__ __align__(16) uint16_t qs[kMaxGroup][kMaxHeadDim + 8];
   __shared__ float wm[kAttnThreads / kWave][kMaxGroup];
   __shared__ double wl[kAttnThreads / kWave][kMaxGroup];
@@ -324,7 +533,7 @@ __global__ __launch_bounds__(kAttnThreads) void attn_scores_kernel(
   if ((int)threadIdx.x < g) {
     double sum = 0.0;
     for (int w = 0; w < kAttnThreads / kWave; ++w) sum += wl[w][r];
-    const int64_t at = (int64_t)h * gridDim.y + blk;
+    const int64_t at = (int64_t)h * nblk + blk;
     stat_m[at] = m;
     stat_l[at] = sum;
   }
@@ -494,6 +703,63 @@ AttnPlan attn_plan(int64_t count) {
   return a;
 }
 
+// Scores to context of one token (klc_attn_decode's kernels), with a step's
+// record when rec.host is given.
+int attn_core(const uint16_t* qb, const uint16_t* kb, const uint16_t* vb, const uint16_t* sk, int64_t cap,
+              int64_t first, int n, int nh, int nkv, int d, bool f16, void* workspace, uint16_t* ctx,
+              const StepRecord& rec, hipStream_t st) {
+  const float sqrt_d = sqrtf((float)d);
+  const unsigned extra = rec.host != nullptr ? 1 : 0;  // the record's workgroup (one per KV head in the score grid)
+  if (n <= kPvKeys) {  // a window: one launch, one workgroup per query head
+    static_assert(kPvKeys == kAttnThreads, "one key per thread");
+    attn_window_kernel<<<(unsigned)nh + extra, kAttnThreads, 0, st>>>(
+        qb, kb, sk, vb, static_cast<float*>(workspace), ctx, cap, first, n, nh, nkv, d, sqrt_d, f16, rec);
+    return check_launch("attn_window_kernel");
+  }
+  const AttnPlan a = attn_plan(n);
+  float* scores = static_cast<float*>(workspace);
+  float* partial = scores + (int64_t)nh * a.cs;
+  double* stat_l = reinterpret_cast<double*>(partial + (int64_t)nh * a.splits * d);
+  float* stat_m = reinterpret_cast<float*>(stat_l + (int64_t)nh * a.nblk);
+  const dim3 sgrid((unsigned)nkv, (unsigned)a.nblk + extra), vgrid((unsigned)nkv, (unsigned)a.splits);
+  auto run_scores = a.score_keys == 64 ? (f16 ? attn_scores_kernel<1, true> : attn_scores_kernel<1, false>)
+                                       : (f16 ? attn_scores_kernel<4, true> : attn_scores_kernel<4, false>);
+  run_scores<<<sgrid, kAttnThreads, 0, st>>>(qb, kb, scores, stat_m, stat_l, cap, first, n, (int)a.cs, (int)a.nblk,
+                                             nh, nkv, d, sqrt_d, rec);
+  int rc = check_launch("attn_scores_kernel");
+  if (rc) return rc;
+  auto run_pv = f16 ? attn_pv_kernel<true> : attn_pv_kernel<false>;
+  run_pv<<<vgrid, kAttnThreads, 0, st>>>(scores, stat_m, stat_l, (int)a.nblk, sk, vb, partial, cap, first, n,
+                                         (int)a.cs, a.split_keys == 128 ? 7 : 8, nh, nkv, d);
+  if ((rc = check_launch("attn_pv_kernel"))) return rc;
+  attn_combine_kernel<<<(unsigned)nh, kAttnThreads, 0, st>>>(partial, (int)a.splits, d, ctx, f16);
+  return check_launch("attn_combine_kernel");
+}
+
+int64_t attn_bytes(int64_t n_heads, int64_t head_dim, int64_t count) {
+  if (count <= kPvKeys) return 4 * n_heads * (count + head_dim);
+  const AttnPlan a = attn_plan(count);
+  return n_heads * (4 * a.cs + 12 * a.nblk + 4 * a.splits * head_dim);
+}
+
+// Scratch of klc_attn_step before the core's: q and k before and after RoPE, the context
+int64_t step_rows_bytes(int64_t nh, int64_t nkv, int64_t d) { return (2 * (2 * (nh + nkv) + nh) * d + 15) / 16 * 16; }
+
+template <int J>
+int launch_qkv(const QkvArgs& a, hipStream_t st) {
+  const int waves = (a.nh + 2 * a.nkv) * (a.d / 2), per = kAttnThreads / kWave;
+  attn_qkv_kernel<J><<<(unsigned)((waves + per - 1) / per), kAttnThreads, 0, st>>>(a);
+  return check_launch("attn_qkv_kernel");
+}
+
+template <int J>
+int launch_out(const uint16_t* w, const uint16_t* bias, const uint16_t* x, uint16_t* out, int rows, int k,
+               hipStream_t st) {
+  const int per = 2 * kAttnThreads / kWave;
+  attn_out_kernel<J><<<(unsigned)((rows + per - 1) / per), kAttnThreads, 0, st>>>(w, bias, x, out, rows, k);
+  return check_launch("attn_out_kernel");
+}
+
 }  // namespace
 }  // namespace klc
 
@@ -526,9 +792,7 @@ extern "C" int klc_rope_append(const void* q, const void* k, const void* v, cons
 extern "C" int64_t klc_attn_workspace_bytes(int64_t n_heads, int64_t head_dim, int64_t count) {
   if (n_heads <= 0 || head_dim <= 0 || count <= 0)
     return set_error(KLC_ERR_ARGUMENT, "klc_attn_workspace_bytes: bad sizes");
-  if (count <= kPvKeys) return 4 * n_heads * (count + head_dim);
-  const AttnPlan a = attn_plan(count);
-  return n_heads * (4 * a.cs + 12 * a.nblk + 4 * a.splits * head_dim);
+  return attn_bytes(n_heads, head_dim, count);
 }
 
 extern "C" int klc_attn_decode(const void* q, const void* k_cache, const void* v_cache, const void* sinks,
@@ -552,36 +816,80 @@ extern "C" int klc_attn_decode(const void* q, const void* k_cache, const void* v
   const int64_t need = klc_attn_workspace_bytes(n_heads, head_dim, count);
   KLC_REQUIRE(workspace_bytes >= need, KLC_ERR_ARGUMENT, "klc_attn_decode: workspace of %lld bytes, need %lld",
               (long long)workspace_bytes, (long long)need);
-  hipStream_t st = as_stream(stream);
-  const uint16_t* qb = static_cast<const uint16_t*>(q);
-  const uint16_t* kb = static_cast<const uint16_t*>(k_cache);
-  const uint16_t* vb = static_cast<const uint16_t*>(v_cache);
-  const uint16_t* sk = static_cast<const uint16_t*>(sinks);
-  uint16_t* ctx = static_cast<uint16_t*>(context);
-  const float sqrt_d = sqrtf((float)head_dim);
-  const int n = (int)count, nh = (int)n_heads, nkv = (int)n_kv, d = (int)head_dim;
-  if (count <= kPvKeys) {  // a window: one launch, one workgroup per query head
-    static_assert(kPvKeys == kAttnThreads, "one key per thread");
-    attn_window_kernel<<<(unsigned)n_heads, kAttnThreads, 0, st>>>(
-        qb, kb, sk, vb, static_cast<float*>(workspace), ctx, cap, first, n, nh, nkv, d, sqrt_d, f16);
-    return check_launch("attn_window_kernel");
+  return attn_core(static_cast<const uint16_t*>(q), static_cast<const uint16_t*>(k_cache),
+                   static_cast<const uint16_t*>(v_cache), static_cast<const uint16_t*>(sinks), cap, first, (int)count,
+                   (int)n_heads, (int)n_kv, (int)head_dim, f16, workspace, static_cast<uint16_t*>(context),
+                   StepRecord{}, as_stream(stream));
+}
+
+extern "C" int64_t klc_attn_step_workspace_bytes(int64_t n_heads, int64_t n_kv, int64_t head_dim, int64_t count) {
+  if (n_heads <= 0 || n_kv <= 0 || head_dim <= 0 || count <= 0)
+    return set_error(KLC_ERR_ARGUMENT, "klc_attn_step_workspace_bytes: bad sizes");
+  return step_rows_bytes(n_heads, n_kv, head_dim) + attn_bytes(n_heads, head_dim, count);
+}
+
+extern "C" int klc_attn_step(const klc_attn_step_args* args, void* stream) {
+  KLC_REQUIRE(args != nullptr, KLC_ERR_ARGUMENT, "klc_attn_step: null pointer");
+  const klc_attn_step_args& a = *args;
+  KLC_REQUIRE(a.hidden && a.q_weight && a.k_weight && a.v_weight && a.o_weight && a.inv_freq && a.k_cache &&
+                  a.v_cache && a.workspace && a.out,
+              KLC_ERR_ARGUMENT, "klc_attn_step: null pointer");
+  const int64_t nh = a.n_heads, nkv = a.n_kv, d = a.head_dim, h = a.hidden_size;
+  KLC_REQUIRE(nh > 0 && nkv > 0 && nh % nkv == 0 && nh / nkv <= kMaxGroup && d >= 8 && d % 8 == 0 &&
+                  d <= kMaxHeadDim && nh * d <= kMaxRow && h > 0 && h % 8 == 0 && h <= kMaxRow && a.out_size > 0 &&
+                  a.out_size < (1 << 30),
+              KLC_ERR_SHAPE,
+              "klc_attn_step: heads %lld / %lld (group <= %d) x %lld (8..%d, multiple of 8; at most %d in all), hidden "
+              "%lld (a multiple of 8, at most %d), out %lld",
+              (long long)nh, (long long)nkv, kMaxGroup, (long long)d, kMaxHeadDim, kMaxRow, (long long)h, kMaxRow,
+              (long long)a.out_size);
+  KLC_REQUIRE(a.cap > 0 && a.count > 0 && a.count <= a.cap && a.first >= 0 && a.first < a.cap &&
+                  a.count <= (1 << 22) && nh * a.count < ((int64_t)1 << 31) && a.slot >= 0 && a.slot < a.cap,
+              KLC_ERR_ARGUMENT, "klc_attn_step: slot %lld, %lld keys from slot %lld of a %lld-slot ring",
+              (long long)a.slot, (long long)a.count, (long long)a.first, (long long)a.cap);
+  KLC_REQUIRE(((uintptr_t)a.hidden | (uintptr_t)a.q_weight | (uintptr_t)a.k_weight | (uintptr_t)a.v_weight |
+               (uintptr_t)a.o_weight | (uintptr_t)a.k_cache | (uintptr_t)a.v_cache | (uintptr_t)a.workspace) %
+                      16 ==
+                  0,
+              KLC_ERR_ARGUMENT, "klc_attn_step: hidden, weights, caches and workspace must be 16-byte aligned");
+  KLC_REQUIRE(a.kv_dtype == KLC_DTYPE_BF16 || a.kv_dtype == KLC_DTYPE_F16, KLC_ERR_UNSUPPORTED,
+              "klc_attn_step: kv_dtype %lld (bfloat16 or float16)", (long long)a.kv_dtype);
+  const int64_t need = klc_attn_step_workspace_bytes(nh, nkv, d, a.count);
+  KLC_REQUIRE(a.workspace_bytes >= need, KLC_ERR_ARGUMENT, "klc_attn_step: workspace of %lld bytes, need %lld",
+              (long long)a.workspace_bytes, (long long)need);
+  StepRecord rec{};
+  if (a.host_record != nullptr) {
+    KLC_REQUIRE(a.tag != 0, KLC_ERR_ARGUMENT, "klc_attn_step: tag 0 (the caller clears the tag word to 0)");
+    hipPointerAttribute_t attr;
+    const hipError_t e = hipPointerGetAttributes(&attr, a.host_record);
+    KLC_REQUIRE(e == hipSuccess && attr.devicePointer != nullptr, KLC_ERR_ARGUMENT,
+                "klc_attn_step: host_record is not pinned host memory");
+    rec.host = static_cast<uint32_t*>(attr.devicePointer);
+    rec.tag = (uint32_t)a.tag;
   }
-  const AttnPlan a = attn_plan(count);
-  float* scores = static_cast<float*>(workspace);
-  float* partial = scores + n_heads * a.cs;
-  double* stat_l = reinterpret_cast<double*>(partial + n_heads * a.splits * head_dim);
-  float* stat_m = reinterpret_cast<float*>(stat_l + n_heads * a.nblk);
-  const dim3 sgrid((unsigned)n_kv, (unsigned)a.nblk), vgrid((unsigned)n_kv, (unsigned)a.splits);
-  auto run_scores = a.score_keys == 64 ? (f16 ? attn_scores_kernel<1, true> : attn_scores_kernel<1, false>)
-                                       : (f16 ? attn_scores_kernel<4, true> : attn_scores_kernel<4, false>);
-  run_scores<<<sgrid, kAttnThreads, 0, st>>>(qb, kb, scores, stat_m, stat_l, cap, first, n, (int)a.cs, nh, nkv, d,
-                                             sqrt_d);
-  int rc = check_launch("attn_scores_kernel");
+  hipStream_t st = as_stream(stream);
+  uint16_t* pre = static_cast<uint16_t*>(a.workspace);
+  uint16_t* rot = pre + (nh + nkv) * d;
+  uint16_t* ctx = rot + (nh + nkv) * d;
+  rec.pre = pre;
+  rec.rot = rot;
+  auto in = [](const void* p) { return static_cast<const uint16_t*>(p); };
+  const bool f16 = a.kv_dtype == KLC_DTYPE_F16;
+  const QkvArgs qkv{in(a.hidden), in(a.q_weight), in(a.q_bias), in(a.k_weight), in(a.k_bias), in(a.v_weight),
+                    in(a.v_bias), static_cast<const float*>(a.inv_freq), pre, rot,
+                    static_cast<uint16_t*>(a.k_cache), static_cast<uint16_t*>(a.v_cache), a.slot, (int)h, (int)nh,
+                    (int)nkv, (int)d, (float)a.position, (float)a.rope_scale, f16};
+  using QkvFn = int (*)(const QkvArgs&, hipStream_t);
+  static constexpr QkvFn kQkv[] = {launch_qkv<1>, launch_qkv<2>, launch_qkv<3>, launch_qkv<4>,
+                                   launch_qkv<5>, launch_qkv<6>, launch_qkv<7>, launch_qkv<8>};
+  int rc = kQkv[(h / 8 + kWave - 1) / kWave - 1](qkv, st);
   if (rc) return rc;
-  auto run_pv = f16 ? attn_pv_kernel<true> : attn_pv_kernel<false>;
-  run_pv<<<vgrid, kAttnThreads, 0, st>>>(scores, stat_m, stat_l, (int)a.nblk, sk, vb, partial, cap, first, n,
-                                         (int)a.cs, a.split_keys == 128 ? 7 : 8, nh, nkv, d);
-  if ((rc = check_launch("attn_pv_kernel"))) return rc;
-  attn_combine_kernel<<<(unsigned)n_heads, kAttnThreads, 0, st>>>(partial, (int)a.splits, d, ctx, f16);
-  return check_launch("attn_combine_kernel");
+  rc = attn_core(rot, in(a.k_cache), in(a.v_cache), in(a.sinks), a.cap, a.first, (int)a.count, (int)nh, (int)nkv,
+                 (int)d, f16, static_cast<char*>(a.workspace) + step_rows_bytes(nh, nkv, d), ctx, rec, st);
+  if (rc) return rc;
+  using OutFn = int (*)(const uint16_t*, const uint16_t*, const uint16_t*, uint16_t*, int, int, hipStream_t);
+  static constexpr OutFn kOut[] = {launch_out<1>, launch_out<2>, launch_out<3>, launch_out<4>,
+                                   launch_out<5>, launch_out<6>, launch_out<7>, launch_out<8>};
+  return kOut[(nh * d / 8 + kWave - 1) / kWave - 1](in(a.o_weight), in(a.o_bias), ctx, static_cast<uint16_t*>(a.out),
+                                                    (int)a.out_size, (int)(nh * d), st);
 }

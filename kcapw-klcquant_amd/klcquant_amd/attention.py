@@ -8,22 +8,31 @@ StreamedAttention) and kv_cache_manager.py (KVCacheManager's methods, here
 * the cache is a preallocated ring per layer in HBM ([cap, n_kv, head_dim] of
   the cache type); ``append`` writes one slot and ``get`` only builds the
   stacked view the reference API returns;
-* ``StreamedAttention.forward`` with a ``DeviceKVCache`` runs RoPE + append in
-  one kernel (klc_rope_append) and the scores / softmax with sinks / value
-  sum over the window in klc_attn_decode; the q/k/v/o projections stay
-  torch's ``F.linear`` (plain library GEMVs), so they are the reference's.
+* ``StreamedAttention.forward`` with a ``DeviceKVCache`` is one library call
+  (klc_attn_step): q/k/v projections with RoPE and the append in their
+  epilogue, scores / softmax with sinks / value sum over the window, the
+  output projection; the diagnostics come back through a pinned host record
+  that the device writes while the step runs.  What that call does not take
+  (autograd, autocast, tensor subclasses, other layouts) runs as torch's
+  ``F.linear`` with klc_rope_append and klc_attn_decode between.
 """
 
 from __future__ import annotations
 
 import ctypes
 import math
+import struct
+import time
 from dataclasses import dataclass
 
+import numpy as np
 import torch
+from torch.autograd import forward_ad
 
 from . import _native
 
+# klc_attn_step_args: pointers, sizes, then position and RoPE scaling
+_STEP = struct.Struct("=16Q12q2d")
 _KV_DTYPES = {"fp16": (torch.float16, 1), "bf16": (torch.bfloat16, 0)}  # KLC_DTYPE_F16 = 1, KLC_DTYPE_BF16 = 0
 
 
@@ -200,6 +209,51 @@ class DeviceKVCache:
         self.layers.clear()
 
 
+class _HostRecord:
+    """klc_attn_step's record in pinned host memory: 6 norms, 2 counts, tag."""
+
+    def __init__(self) -> None:
+        self._held = torch.zeros(16, dtype=torch.int32, pin_memory=True)
+        self.words = self._held.numpy()
+        self.floats = self.words.view(np.float32)
+        self.ptr = self._held.data_ptr()
+
+    def wait(self, dev: torch.device, limit_s: float) -> None:
+        """Spins until the device has written the tag; past ``limit_s`` it synchronises the current
+        stream instead, which raises if the device failed."""
+        words, spins, deadline = self.words, 0, None
+        while words[8] != 1:
+            spins += 1
+            if spins & 1023 == 0:
+                now = time.perf_counter()
+                if deadline is None:
+                    deadline = now + limit_s
+                elif now > deadline:
+                    torch.cuda.current_stream(dev).synchronize()
+                    if words[8] != 1:
+                        raise RuntimeError("the attention step finished without its host record")
+                    return
+
+
+_TENSORS = (torch.Tensor, torch.nn.Parameter)
+
+
+def _plain(t, dev: torch.device, shape: tuple) -> bool:
+    """A contiguous bfloat16 tensor of ``shape`` on ``dev``, no subclass."""
+    return (type(t) in _TENSORS and t.dtype is torch.bfloat16 and t.shape == shape and t.device == dev
+            and t.is_contiguous())
+
+
+def _intercepted() -> bool:
+    """Something watches or replaces torch calls here (modes, function transforms, forward-mode AD,
+    autocast, tracing, stream capture): F.linear has to be seen by it."""
+    c = torch._C
+    return bool(c._len_torch_dispatch_stack() or c._len_torch_function_stack()
+                or c._functorch.peek_interpreter_stack() is not None or forward_ad._current_level >= 0
+                or torch.is_autocast_enabled("cuda") or c._get_tracing_state() is not None
+                or torch.compiler.is_compiling() or torch.cuda.is_current_stream_capturing())
+
+
 class StreamedAttention:
     """StreamedAttention (streamed_attention.py:101-152)."""
 
@@ -207,6 +261,8 @@ class StreamedAttention:
         self.config = config
         self._tables: dict = {}
         self._workspace: torch.Tensor | None = None
+        self._inv_freq: dict = {}
+        self._records: list = []  # pinned host records of klc_attn_step not in use
 
     def _cos_sin(self, position: int, device: torch.device) -> tuple[torch.Tensor, torch.Tensor]:
         key = (int(position), str(device))
@@ -218,10 +274,104 @@ class StreamedAttention:
             self._tables[key] = t
         return t
 
+    def _device_inv_freq(self, device: torch.device) -> torch.Tensor:
+        c = self.config
+        key = (device, c.head_dim, c.rope_theta, c.rope_factor, c.rope_beta_fast, c.rope_beta_slow,
+               c.rope_original_max_position_embeddings, c.rope_truncate)
+        t = self._inv_freq.get(key)
+        if t is None:
+            t = yarn_inv_freq(c, device)
+            torch.cuda.current_stream(device).synchronize()  # any stream may read it from here on
+            self._inv_freq[key] = t
+        return t
+
+    # A record the GPU has not written after this long is waited for by a
+    # synchronisation of the stream.
+    _RECORD_WAIT_S = 2.0
+
+    def _step(self, layer_idx: int, prefix: str, hidden: torch.Tensor, tensors: dict, position: int, kv_cache,
+              sliding_window: int | None):
+        """One klc_attn_step call, or None for what that call does not take (the caller's general path)."""
+        cfg = self.config
+        dev = hidden.device
+        nh, nkv, d = cfg.num_heads, cfg.num_kv_heads, cfg.head_dim
+        size = hidden.shape[-1] if hidden.dim() else 0
+        q, kv = nh * d, nkv * d
+        if (type(hidden) is not torch.Tensor or hidden.dtype is not torch.bfloat16 or dev.type != "cuda"
+                or not isinstance(kv_cache, DeviceKVCache) or kv_cache.device.type != "cuda"
+                or size == 0 or size % 8 or size > 4096 or hidden.numel() != size or not hidden.is_contiguous()
+                or d % 8 or d > 128 or q > 4096 or nh % nkv or nh // nkv > 16 or _intercepted()):
+            return None
+        get = tensors.get
+        weights = [get(f"{prefix}.{n}_proj.weight") for n in "qkvo"]
+        biases = [get(f"{prefix}.{n}_proj.bias") for n in "qkvo"]
+        sinks = get(f"{prefix}.sinks")
+        o_size = weights[3].shape[0] if isinstance(weights[3], torch.Tensor) and weights[3].dim() == 2 else 0
+        rows = (q, kv, kv, o_size)
+        for w, b, n, k in zip(weights, biases, rows, (size, size, size, q)):
+            if not (_plain(w, dev, (n, k)) and _plain(b, dev, (n,))):
+                return None
+        if o_size == 0 or (sinks is not None and not _plain(sinks, dev, (nh,))):
+            return None
+        held = [hidden, *weights, *biases] if sinks is None else [hidden, *weights, *biases, sinks]
+        if torch.is_grad_enabled() and any(t.requires_grad for t in held):
+            return None
+        ptr = [t.data_ptr() for t in held]
+        if (ptr[0] | ptr[1] | ptr[2] | ptr[3] | ptr[4]) % 16:
+            return None
+        window = sliding_window if sliding_window is not None else cfg.sliding_window
+        inv_freq = self._device_inv_freq(dev)
+        scaling = yarn_attention_scaling(cfg)
+        ring, slot = kv_cache.next_slot(layer_idx, nkv, d)
+        keys, values = ring["k"], ring["v"]
+        if keys.device != dev or keys.shape[1:] != (nkv, d) or values.shape != keys.shape:
+            return None
+        total = ring["total"] + 1
+        count = min(total, ring["cap"])
+        if window:
+            count = min(count, window)
+        lib = _native.load()
+        need = lib.klc_attn_step_workspace_bytes(nh, nkv, d, count)
+        workspace = torch.empty(max(need, 16), dtype=torch.uint8, device=dev)
+        out = torch.empty(o_size, dtype=torch.bfloat16, device=dev)
+        record = self._records.pop() if self._records else _HostRecord()
+        words = record.words
+        words[8] = 0
+        rc = lib.klc_attn_step(
+            _STEP.pack(ptr[0], ptr[1], ptr[5], ptr[2], ptr[6], ptr[3], ptr[7], ptr[4], ptr[8],
+                       0 if sinks is None else ptr[9], inv_freq.data_ptr(), keys.data_ptr(), values.data_ptr(),
+                       workspace.data_ptr(), out.data_ptr(), record.ptr, size, o_size, nh, nkv, d, ring["cap"], slot,
+                       (total - count) % ring["cap"], count, kv_cache.kv_code, workspace.numel(), 1, float(position),
+                       scaling), torch._C._cuda_getCurrentRawStream(dev.index))
+        if rc < 0:
+            raise _native.KlcError("klc_attn_step", int(rc), _native.last_error())
+        ring["total"] = total
+        record.wait(dev, self._RECORD_WAIT_S)
+        norms = record.floats[:6].tolist()
+        diagnostics = {
+            "rope_position": int(position),
+            "rope_attention_scaling": float(scaling),
+            "sliding_window": sliding_window,
+            "q_pre_rope_norm": norms[0],
+            "k_pre_rope_norm": norms[1],
+            "q_post_rope_norm": norms[2],
+            "k_post_rope_norm": norms[3],
+            "q_rope_delta_norm": norms[4],
+            "k_rope_delta_norm": norms[5],
+            "q_post_rope_nonfinite_count": int(words[6]),
+            "k_post_rope_nonfinite_count": int(words[7]),
+        }
+        if len(self._records) < 16:
+            self._records.append(record)
+        return out, diagnostics
+
     def forward(self, layer_idx: int, hidden: torch.Tensor, tensors: dict, position: int, kv_cache,
                 sliding_window: int | None = None):
         cfg = self.config
         prefix = f"model.layers.{layer_idx}.self_attn"
+        stepped = self._step(layer_idx, prefix, hidden, tensors, position, kv_cache, sliding_window)
+        if stepped is not None:
+            return stepped
         lin = torch.nn.functional.linear
         q = lin(hidden, tensors[f"{prefix}.q_proj.weight"], tensors[f"{prefix}.q_proj.bias"]).view(cfg.num_heads, cfg.head_dim)
         k = lin(hidden, tensors[f"{prefix}.k_proj.weight"], tensors[f"{prefix}.k_proj.bias"]).view(cfg.num_kv_heads, cfg.head_dim)

@@ -247,6 +247,97 @@ def test_split_decode_infinite_scores(gpu):
     assert torch.isfinite(ctx[: nh // 2]).all() and torch.isnan(ctx[nh // 2:]).all()
 
 
+def step_tensors(gpu, g, nh, nkv, d, h, rows, pre, sinks=True):
+    def w(*s, scale=0.02):
+        return (torch.randn(s, generator=g, device=gpu) * scale).to(torch.bfloat16)
+
+    t = {f"{pre}.{n}_proj.weight": w(r, c) for n, r, c in (("q", nh * d, h), ("k", nkv * d, h), ("v", nkv * d, h),
+                                                           ("o", rows, nh * d))}
+    t |= {f"{pre}.{n}_proj.bias": w(r) for n, r in (("q", nh * d), ("k", nkv * d), ("v", nkv * d), ("o", rows))}
+    if sinks:
+        t[f"{pre}.sinks"] = w(nh, scale=1.0)
+    return t
+
+
+@pytest.mark.parametrize("nh,nkv,d,h,rows,count,position,kv,sinks", [
+    (64, 8, 64, 2880, 2880, 128, 131071, "fp16", True), (64, 8, 64, 2880, 2880, 900, 0, "bf16", True),
+    (4, 4, 8, 8, 1, 1, 5, "fp16", False), (32, 2, 128, 4096, 33, 257, 99999, "bf16", True),
+    (6, 2, 24, 520, 77, 300, 4095, "fp16", True), (16, 1, 40, 1544, 512, 256, 70000, "bf16", False)])
+def test_attention_step_matches_oracle(gpu, nh, nkv, d, h, rows, count, position, kv, sinks):
+    """klc_attn_step's stages, each exactly from the one before: correctly rounded projections (the
+    float64 sum rounded to float32 and bfloat16), RoPE with torch's own tables and the stored key and
+    value bit for bit, the context and output within their bounds, the diagnostics."""
+    g = torch.Generator(device=gpu).manual_seed(nh * d + h)
+    pre = "model.layers.3.self_attn"
+    cfg = AttentionConfig(hidden_size=h, num_heads=nh, num_kv_heads=nkv, head_dim=d, rope_factor=32.0)
+    t = step_tensors(gpu, g, nh, nkv, d, h, rows, pre, sinks)
+    x = torch.randn(h, generator=g, device=gpu).to(torch.bfloat16)
+    cache = DeviceKVCache(gpu, max_tokens=count, precision=kv)
+    ring, _ = cache.next_slot(3, nkv, d)
+    ring["k"].copy_(torch.randn(ring["k"].shape, generator=g, device=gpu))
+    ring["v"].copy_(torch.randn(ring["v"].shape, generator=g, device=gpu))
+    ring["total"] = count + 1  # the token goes to slot 1 % count
+    attn = StreamedAttention(cfg)
+    assert attn._step(3, pre, x, t, position, cache, None) is not None, "the one-call path did not take these tensors"
+    ring["total"] = count + 1
+    out, diag = attn.forward(3, x, t, position, cache)
+    assert ring["total"] == count + 2
+
+    def proj(n, heads):
+        y = t[f"{pre}.{n}_proj.weight"].double().cpu() @ x.double().cpu() + t[f"{pre}.{n}_proj.bias"].double().cpu()
+        return f32_to_bf16(y.float().numpy()).reshape(heads, d)
+
+    q, k, v = proj("q", nh), proj("k", nkv), proj("v", nkv)
+    cos, sin = rope_cos_sin(cfg, position, gpu, torch.bfloat16)
+    q_rot, k_rot = oat.rope_rotate(q, bits(cos), bits(sin)), oat.rope_rotate(k, bits(cos), bits(sin))
+    slot = (count + 1) % count
+    assert np.array_equal(ring["k"][slot].float().cpu().numpy(), oat.to_kv(bf16_to_f32(k_rot), kv))
+    assert np.array_equal(ring["v"][slot].float().cpu().numpy(), oat.to_kv(bf16_to_f32(v), kv))
+    order = [(slot + 1 + i) % count for i in range(count)]  # the appended token last
+    sk = t[f"{pre}.sinks"] if sinks else None
+    ctx = decode_direct(gpu, dev(q_rot, gpu), ring["k"], ring["v"], sk, count, order[0], count, kv)
+    want = t[f"{pre}.o_proj.weight"].double() @ ctx.reshape(-1).double() + t[f"{pre}.o_proj.bias"].double()
+    assert torch.equal(out, want.float().to(torch.bfloat16))
+    ref = {"q_pre_rope_norm": q, "k_pre_rope_norm": k, "q_post_rope_norm": q_rot, "k_post_rope_norm": k_rot}
+    for name, rows_ in ref.items():
+        assert np.isclose(diag[name], np.linalg.norm(bf16_to_f32(rows_).astype(np.float64)), rtol=1e-6)
+    for name, a, b in (("q_rope_delta_norm", q_rot, q), ("k_rope_delta_norm", k_rot, k)):
+        assert np.isclose(diag[name], np.linalg.norm((bf16_to_f32(a) - bf16_to_f32(b)).astype(np.float64)), rtol=1e-6)
+    assert diag["q_post_rope_nonfinite_count"] == diag["k_post_rope_nonfinite_count"] == 0
+    assert diag["rope_position"] == position and diag["sliding_window"] is None
+
+
+def test_attention_step_and_general_path_agree(gpu):
+    """The same step through the one call and, with gradients asked for, through F.linear; non-finite
+    values are counted by both."""
+    nh, nkv, d, h = 64, 8, 64, 2880
+    g = torch.Generator(device=gpu).manual_seed(5)
+    pre = "model.layers.0.self_attn"
+    t = step_tensors(gpu, g, nh, nkv, d, h, h, pre)
+    cfg = AttentionConfig(**CFG, sliding_window=4)
+    for poison in (False, True):
+        x = torch.randn(h, generator=g, device=gpu).to(torch.bfloat16)
+        if poison:
+            x[7] = float("inf")
+        outs, diags = [], []
+        for grad in (False, True):
+            w = {n: v.clone().requires_grad_(grad and n.endswith("o_proj.weight")) for n, v in t.items()}
+            cache = DeviceKVCache(gpu, precision="fp16", capacity=4)
+            attn = StreamedAttention(cfg)
+            assert (attn._step(0, pre, x, w, 3, DeviceKVCache(gpu, capacity=4), None) is None) == grad
+            for pos in range(3):
+                out, diag = attn.forward(0, x, w, pos, cache)
+            outs.append(out)
+            diags.append(diag)
+        assert outs[1].requires_grad and not outs[0].requires_grad
+        assert torch.allclose(outs[0].float(), outs[1].float(), rtol=2e-2, atol=1e-2, equal_nan=True)
+        assert diags[0].keys() == diags[1].keys()
+        for name in diags[0]:
+            assert diags[0][name] == diags[1][name] or np.isclose(diags[0][name], diags[1][name], rtol=1e-4, equal_nan=True)
+        if poison:
+            assert diags[0]["q_post_rope_nonfinite_count"] > 0
+
+
 def test_attention_rejects_bad_shapes(gpu):
     x = torch.zeros(4096, dtype=torch.bfloat16, device=gpu)
     ws = torch.zeros(1 << 16, dtype=torch.uint8, device=gpu)
