@@ -34,6 +34,7 @@ namespace klc {
 namespace {
 
 constexpr int kAttnThreads = 256;
+constexpr int kProjThreads = 128;  // projection kernels: 64, 128 and 256 measured alike (2880 rows: 6.9, 6.7, 7.6 us)
 constexpr int kPvKeys = 256;     // most keys of a value workgroup, and of a one-launch window
 constexpr int kMaxHeadDim = 128;
 constexpr int kMaxGroup = 16;    // query heads per KV head
@@ -128,8 +129,12 @@ struct TwoRows {
   }
 };
 
+// bias[row], 0 without a bias (an empty buffer), with no branch; loaded before
+// the rows, so that nothing waits for it alone
 __device__ __forceinline__ float bias_at(const uint16_t* bias, int row) {
-  return bias != nullptr ? bf(bias[row]) : 0.f;
+  const __amdgpu_buffer_rsrc_t b = __builtin_amdgcn_make_buffer_rsrc((void*)bias, (short)0,
+                                                                     bias != nullptr ? 2 * (row + 1) : 0, kBufferWord3);
+  return bf((uint16_t)__builtin_amdgcn_raw_buffer_load_b16(b, 2 * row, 0, 0));
 }
 __device__ __forceinline__ uint16_t biased_bf(double sum, float bias) { return to_bf((float)(sum + (double)bias)); }
 
@@ -149,19 +154,21 @@ struct QkvArgs {
 // d / 2 of a head), or two value rows, so the rotation needs nothing from
 // another wave and the step has no launch for it.  cos and sin are taken
 // while the rows are on their way, with torch's rounding points (float32
-// angle, float32 product with the scaling, bfloat16).
+// angle, float32 product with the scaling, bfloat16).  HBM bound: 29.5 MB for
+// 5120 rows of 2880 in 8.5 us (10.4 with the biases read through a branch,
+// which waited for every row in flight).
 template <int J>
-__global__ __launch_bounds__(kAttnThreads) void attn_qkv_kernel(QkvArgs a) {
+__global__ __launch_bounds__(kProjThreads) void attn_qkv_kernel(QkvArgs a) {
   const int half = a.d / 2, pairs = (a.nh + a.nkv) * half;
-  const int p = blockIdx.x * (kAttnThreads / kWave) + __builtin_amdgcn_readfirstlane(threadIdx.x / kWave);
+  const int p = blockIdx.x * (kProjThreads / kWave) + __builtin_amdgcn_readfirstlane(threadIdx.x / kWave);
   if (p >= pairs + a.nkv * half) return;
   TwoRows<J> rows;
   double s0, s1;
   if (p >= pairs) {
     const int r0 = 2 * (p - pairs);
     const uint16_t* w = a.vw + (int64_t)r0 * a.hidden;
-    rows.load(w, w + a.hidden, a.x, a.hidden);
     const float b0 = bias_at(a.vb, r0), b1 = bias_at(a.vb, r0 + 1);
+    rows.load(w, w + a.hidden, a.x, a.hidden);
     rows.dot(s0, s1);
     if (threadIdx.x % kWave == 0) {
       uint16_t* dst = a.v_cache + a.slot * a.nkv * a.d + r0;
@@ -175,10 +182,10 @@ __global__ __launch_bounds__(kAttnThreads) void attn_qkv_kernel(QkvArgs a) {
   const bool is_q = head < a.nh;
   const int row = (is_q ? head : head - a.nh) * a.d + j;
   const uint16_t* w = (is_q ? a.qw : a.kw) + (int64_t)row * a.hidden;
-  rows.load(w, w + (int64_t)half * a.hidden, a.x, a.hidden);
   const uint16_t* b = is_q ? a.qb : a.kb;
-  const float b0 = bias_at(b, row), b1 = bias_at(b, row + half);
-  const float angle = __fmul_rn(a.inv_freq[j], a.position);
+  const float b0 = bias_at(b, row), b1 = bias_at(b, row + half), freq = a.inv_freq[j];
+  rows.load(w, w + (int64_t)half * a.hidden, a.x, a.hidden);
+  const float angle = __fmul_rn(freq, a.position);
   const float c = rbf(__fmul_rn(cosf(angle), a.rope_scale)), s = rbf(__fmul_rn(sinf(angle), a.rope_scale));
   rows.dot(s0, s1);
   if (threadIdx.x % kWave == 0) {
@@ -198,18 +205,19 @@ __global__ __launch_bounds__(kAttnThreads) void attn_qkv_kernel(QkvArgs a) {
   }
 }
 
-// out[r] = bf16(x . w[r] + bias[r]) for a bfloat16 weight [rows][k]: two rows a wave
+// out[r] = bf16(x . w[r] + bias[r]) for a bfloat16 weight [rows][k]: two rows
+// a wave.  HBM bound: 23.6 MB (2880 rows of 4096) in 6.7 us.
 template <int J>
-__global__ __launch_bounds__(kAttnThreads) void attn_out_kernel(const uint16_t* __restrict__ w,
+__global__ __launch_bounds__(kProjThreads) void attn_out_kernel(const uint16_t* __restrict__ w,
                                                                 const uint16_t* __restrict__ bias,
                                                                 const uint16_t* __restrict__ x,
                                                                 uint16_t* __restrict__ out, int rows, int k) {
-  const int r0 = 2 * (blockIdx.x * (kAttnThreads / kWave) + __builtin_amdgcn_readfirstlane(threadIdx.x / kWave));
+  const int r0 = 2 * (blockIdx.x * (kProjThreads / kWave) + __builtin_amdgcn_readfirstlane(threadIdx.x / kWave));
   if (r0 >= rows) return;
   const int r1 = min(r0 + 1, rows - 1);
   TwoRows<J> two;
-  two.load(w + (int64_t)r0 * k, w + (int64_t)r1 * k, x, k);
   const float b0 = bias_at(bias, r0), b1 = bias_at(bias, r1);
+  two.load(w + (int64_t)r0 * k, w + (int64_t)r1 * k, x, k);
   double s0, s1;
   two.dot(s0, s1);
   if (threadIdx.x % kWave == 0) {
@@ -228,27 +236,51 @@ struct StepRecord {
 };
 
 // One workgroup: sums of squares in float64 and the record.  It runs beside
-// the score workgroups of the same launch.
+// the score workgroups of the same launch and must not outlast them: 16-byte
+// loads, all in flight (2-byte ones made a 4,096-key score launch 10.2 us
+// instead of 6.7).
 __device__ __forceinline__ void write_record(const StepRecord& rec, int nh, int nkv, int d) {
   __shared__ double sums[kAttnThreads / kWave][6];
   __shared__ int bad[kAttnThreads / kWave][2];
   const int lane = threadIdx.x % kWave, wave = threadIdx.x / kWave;
   double t[6] = {};
   int n[2] = {0, 0};
-  auto take = [&](int which, int from, int to) {
-    double pre = 0.0, post = 0.0, delta = 0.0;
-    int count = 0;
-    for (int i = from + threadIdx.x; i < to; i += kAttnThreads) {
-      const float x = bf(rec.pre[i]), y = bf(rec.rot[i]), z = y - x;
-      pre += (double)x * x;
-      post += (double)y * y;
-      delta += (double)z * z;
-      count += !isfinite(y);
+  const int chunks = (nh + nkv) * d / 8, q_chunks = nh * d / 8;
+  constexpr int kAhead = 3;
+  for (int c0 = threadIdx.x; c0 < chunks; c0 += kAhead * kAttnThreads) {
+    uint4 x[kAhead], y[kAhead];
+#pragma unroll
+    for (int i = 0; i < kAhead; ++i) {
+      const int c = min(c0 + i * kAttnThreads, chunks - 1);
+      x[i] = reinterpret_cast<const uint4*>(rec.pre)[c];
+      y[i] = reinterpret_cast<const uint4*>(rec.rot)[c];
     }
-    t[which] = pre, t[2 + which] = post, t[4 + which] = delta, n[which] = count;
-  };
-  take(0, 0, nh * d);
-  take(1, nh * d, (nh + nkv) * d);
+#pragma unroll
+    for (int i = 0; i < kAhead; ++i) {
+      const int c = c0 + i * kAttnThreads;
+      if (c >= chunks) break;
+      double pre = 0.0, post = 0.0, delta = 0.0;
+      int count = 0;
+      auto add = [&](uint32_t xa, uint32_t ya) {
+        const float u = bf((uint16_t)xa), v = bf((uint16_t)ya), z = v - u;
+        pre += (double)u * u;
+        post += (double)v * v;
+        delta += (double)z * z;
+        count += !isfinite(v);
+      };
+      const uint32_t xs[4] = {x[i].x, x[i].y, x[i].z, x[i].w}, ys[4] = {y[i].x, y[i].y, y[i].z, y[i].w};
+#pragma unroll
+      for (int e = 0; e < 4; ++e) {
+        add(xs[e] & 0xffffu, ys[e] & 0xffffu);
+        add(xs[e] >> 16, ys[e] >> 16);
+      }
+      const bool is_q = c < q_chunks;
+      t[0] += is_q ? pre : 0.0, t[1] += is_q ? 0.0 : pre;
+      t[2] += is_q ? post : 0.0, t[3] += is_q ? 0.0 : post;
+      t[4] += is_q ? delta : 0.0, t[5] += is_q ? 0.0 : delta;
+      n[0] += is_q ? count : 0, n[1] += is_q ? 0 : count;
+    }
+  }
 #pragma unroll
   for (int e = 0; e < 6; ++e)
     for (int off = kWave / 2; off > 0; off >>= 1) t[e] += __shfl_xor(t[e], off);
@@ -747,16 +779,16 @@ int64_t step_rows_bytes(int64_t nh, int64_t nkv, int64_t d) { return (2 * (2 * (
 
 template <int J>
 int launch_qkv(const QkvArgs& a, hipStream_t st) {
-  const int waves = (a.nh + 2 * a.nkv) * (a.d / 2), per = kAttnThreads / kWave;
-  attn_qkv_kernel<J><<<(unsigned)((waves + per - 1) / per), kAttnThreads, 0, st>>>(a);
+  const int waves = (a.nh + 2 * a.nkv) * (a.d / 2), per = kProjThreads / kWave;
+  attn_qkv_kernel<J><<<(unsigned)((waves + per - 1) / per), kProjThreads, 0, st>>>(a);
   return check_launch("attn_qkv_kernel");
 }
 
 template <int J>
 int launch_out(const uint16_t* w, const uint16_t* bias, const uint16_t* x, uint16_t* out, int rows, int k,
                hipStream_t st) {
-  const int per = 2 * kAttnThreads / kWave;
-  attn_out_kernel<J><<<(unsigned)((rows + per - 1) / per), kAttnThreads, 0, st>>>(w, bias, x, out, rows, k);
+  const int per = 2 * kProjThreads / kWave;
+  attn_out_kernel<J><<<(unsigned)((rows + per - 1) / per), kProjThreads, 0, st>>>(w, bias, x, out, rows, k);
   return check_launch("attn_out_kernel");
 }
 
