@@ -603,7 +603,15 @@ int resolve_layer_path(int path, int64_t n_tok, int64_t hidden, int64_t inter, i
     }
     return fused ? KLC_PATH_FUSED : -1;
   }
-  return n_tok * k >= 8 * n_exp ? KLC_PATH_GEMM : KLC_PATH_GEMV;
+  // The GEMV stages 8 (gate_up) or 4 (down) pairs a pass, so an expert's
+  // weights are read again every few pairs; the GEMM's 16-token units read
+  // them once, on half as many workgroups.  Layer, GEMV against GEMM: 64
+  // tokens of 128 experts (2 pairs each) 269 / 265 us, 100 (3.1) 307 / 292,
+  // 200 (6.3) 433 / 322; of 64 experts 32 (2) 141 / 147, 48 (3) 163 / 158; of
+  // 32 experts 16 (2) 80 / 90, 32 (4) 99 / 95; of 16 experts 16 (4) 63 / 65,
+  // 24 (6) 72 / 74.
+  const int64_t pairs = n_tok * k;
+  return pairs >= 8 * n_exp || (pairs >= 3 * n_exp && pairs >= 128) ? KLC_PATH_GEMM : KLC_PATH_GEMV;
 }
 
 

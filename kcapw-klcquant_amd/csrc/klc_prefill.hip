@@ -55,13 +55,14 @@ constexpr int kWaveTiles = KLC_GEMM_WAVE_TILES;     // 64-row packed tiles per w
 constexpr int kRb = 4 * kWaveTiles;                 // 16-row MFMA blocks per wave
 constexpr int kGemmThreads = kGemmWaves * kWave;
 constexpr int kGemmRows = kGemmWaves * kWaveTiles * kTileRows;  // output rows per workgroup
-constexpr int kBRowsPerWave = kUnitTokensGemm / kGemmWaves;  // token rows each wave stages per step
-constexpr int kBInstr = kBRowsPerWave / 4;          // LDS-DMA instructions per wave, plane and step (4 rows each)
-static_assert(kBInstr >= 1 && kBRowsPerWave % 4 == 0, "token rows split evenly over the waves");
 constexpr int kYStride = kGemmRows / 2 + 1;         // gate_up epilogue: floats per token row (odd: spreads the banks)
-constexpr int kGemmCb = kUnitTokensGemm / 16;       // 4 column blocks of 16 tokens
+constexpr int kGemmCb = kUnitTokensGemm / 16;       // 4 column blocks of 16 tokens: the widest kernel's
 template <int N>
 struct ColumnBlocks {
+  static constexpr int value = N;
+};
+template <int N>
+struct WeightPolicy {
   static constexpr int value = N;
 };
 constexpr int kXcds = 8;  // accelerator complex dies of an MI355X, each with its own L2
@@ -105,29 +106,78 @@ __device__ __forceinline__ void ring_barrier() {
 // kPl: activation planes of B (gate_up 1; down 2 = hi + lo of the float32
 // SwiGLU output, or 1 = its bfloat16 rounding, which is exactly the
 // bfloat16-precision input, so the lo plane's zero products are skipped).
-template <bool kDown, int kPl>
-__host__ __device__ constexpr int gemm_ring() { return kDown && kPl == 2 ? KLC_GEMM_RING_DOWN : KLC_GEMM_RING_UP; }
-template <bool kDown, int kPl>
-__host__ __device__ constexpr int gemm_stage_bytes() { return kPl * kUnitTokensGemm * 256; }
+template <bool kDown, int kPl, int kCb>
+__host__ __device__ constexpr int gemm_ring() {
+  if (kCb < kGemmCb) return kCb == 1 ? 3 : 2;
+  return kDown && kPl == 2 ? KLC_GEMM_RING_DOWN : KLC_GEMM_RING_UP;
+}
+template <int kPl, int kCb>
+__host__ __device__ constexpr int gemm_stage_bytes() { return kPl * 16 * kCb * 256; }
 // Each wave's tile of scale records copied into LDS (the packed layout,
 // [S / 8][64 rows][4 quarters][8 bytes], at most 6 KiB for inputs <= 3072),
 // where two workgroups of a CU still fit (not beside the two-plane down
 // ring: that one keeps the records in registers).
 constexpr int kScaleTileLds = kTileRows * 4 * 24;
 constexpr int kScaleLdsBytes = kGemmWaves * kWaveTiles * kScaleTileLds;
-template <bool kDown, int kPl>
-__host__ __device__ constexpr bool gemm_scales_in_lds() { return !(kDown && kPl == 2); }
+template <bool kDown, int kPl, int kCb>
+__host__ __device__ constexpr bool gemm_scales_in_lds() { return kCb < kGemmCb || !(kDown && kPl == 2); }
 // LDS of one workgroup: the B ring, or the gate_up epilogue's output tile if
 // larger, then the staged scales.
-template <bool kDown, int kPl>
+template <bool kDown, int kPl, int kCb>
 __host__ __device__ constexpr int gemm_lds_bytes() {
-  const int ring = gemm_ring<kDown, kPl>() * gemm_stage_bytes<kDown, kPl>();
-  const int tile = kDown ? 0 : kUnitTokensGemm * kYStride * 4;
-  return (ring > tile ? ring : tile) + (gemm_scales_in_lds<kDown, kPl>() ? kScaleLdsBytes : 0);
+  const int ring = gemm_ring<kDown, kPl, kCb>() * gemm_stage_bytes<kPl, kCb>();
+  const int tile = kDown ? 0 : 16 * kCb * kYStride * 4;
+  return (ring > tile ? ring : tile) + (gemm_scales_in_lds<kDown, kPl, kCb>() ? kScaleLdsBytes : 0);
 }
-static_assert(2 * gemm_lds_bytes<false, 1>() <= 160 * 1024 && 2 * gemm_lds_bytes<true, 1>() <= 160 * 1024 &&
-                  2 * gemm_lds_bytes<true, 2>() <= 160 * 1024,
+static_assert(2 * gemm_lds_bytes<false, 1, kGemmCb>() <= 160 * 1024 &&
+                  2 * gemm_lds_bytes<true, 1, kGemmCb>() <= 160 * 1024 &&
+                  2 * gemm_lds_bytes<true, 2, kGemmCb>() <= 160 * 1024,
               "two workgroups per CU");
+
+// Unit u of the runs of kTok pairs of each expert, in expert order, from the
+// expert offsets alone (the dispatch lists 64-token units): each wave scans
+// the experts' unit counts, 4 experts a lane (n_exp <= 256).  All results
+// uniform; false past the last unit.
+template <int kTok>
+__device__ __forceinline__ bool find_unit(const int32_t* __restrict__ offsets, int n_exp, int u, int& e, int& pb,
+                                          int& tc, int& ne) {
+  const int lane = threadIdx.x & 63;
+  int at[5];
+#pragma unroll
+  for (int i = 0; i < 5; ++i) at[i] = offsets[min(4 * lane + i, n_exp)];
+  int n[4], sum = 0;
+#pragma unroll
+  for (int i = 0; i < 4; ++i) {
+    n[i] = (at[i + 1] - at[i] + kTok - 1) / kTok;
+    sum += n[i];
+  }
+  int incl = sum;
+#pragma unroll
+  for (int off = 1; off < kWave; off <<= 1) {
+    const int v = __shfl_up(incl, off);
+    if (lane >= off) incl += v;
+  }
+  const uint64_t past = __ballot(incl > u);
+  if (past == 0) return false;
+  const int src = __builtin_amdgcn_readfirstlane(__builtin_ctzll(past));
+  int r = u - __builtin_amdgcn_readlane(incl - sum, src), i = 0;
+#pragma unroll
+  for (int j = 0; j < 3; ++j) {
+    const int c = __builtin_amdgcn_readlane(n[j], src);
+    if (i == j && r >= c) {
+      r -= c;
+      ++i;
+    }
+  }
+  const int a0 = __builtin_amdgcn_readlane(at[0], src), a1 = __builtin_amdgcn_readlane(at[1], src),
+            a2 = __builtin_amdgcn_readlane(at[2], src), a3 = __builtin_amdgcn_readlane(at[3], src),
+            a4 = __builtin_amdgcn_readlane(at[4], src);
+  e = 4 * src + i;
+  pb = i == 0 ? a0 : i == 1 ? a1 : i == 2 ? a2 : a3;
+  tc = r * kTok;
+  ne = (i == 0 ? a1 : i == 1 ? a2 : i == 2 ? a3 : a4) - pb;
+  return true;
+}
 
 // One GEMM unit x one 256-row tile.  gate_up: act = bfloat16 hidden state
 // [n_tok][in], one plane; writes the down input as hi/lo bfloat16 planes
@@ -135,20 +185,24 @@ static_assert(2 * gemm_lds_bytes<false, 1>() <= 160 * 1024 && 2 * gemm_lds_bytes
 // act = those planes (rows by pair); writes float32 expert outputs.
 // kWide: activation planes past 2 GiB (rows addressed with 64-bit pointers
 // instead of a buffer's 32-bit offsets).
-template <bool kDown, int kPl, bool kWide>
+template <bool kDown, int kPl, int kCb, bool kWide>
 __device__ __forceinline__ void moe_gemm_body(
     const uint8_t* const* __restrict__ wptr, const uint16_t* __restrict__ bias, const uint16_t* __restrict__ act,
     int64_t act_plane, float* __restrict__ out, uint16_t* __restrict__ out_split, int64_t out_plane,
     float* __restrict__ out_raw, const int32_t* __restrict__ offsets, const int32_t* __restrict__ pairs,
     const int32_t* __restrict__ units, const int32_t* __restrict__ n_units, int rows, int groups, int k_top,
-    float limit, int precision, int row_wgs, int units_per_xcd) {
+    float limit, int precision, int row_wgs, int units_per_xcd, int n_exp) {
   static_assert(kPl == 1 || (kDown && kPl == 2), "gate_up reads one plane, down one or two");
   constexpr int kPlanes = kPl;
-  constexpr int kRing = gemm_ring<kDown, kPl>();
-  constexpr int kStage = gemm_stage_bytes<kDown, kPl>();  // one step: 64 token rows x 256 bytes per plane
+  constexpr int kTok = 16 * kCb;                  // tokens of this kernel's units
+  constexpr int kBRowsPerWave = kTok / kGemmWaves;  // token rows each wave stages per step
+  constexpr int kBInstr = kBRowsPerWave / 4;      // LDS-DMA instructions per wave, plane and step (4 rows each)
+  static_assert(kBInstr >= 1 && kBRowsPerWave % 4 == 0, "token rows split evenly over the waves");
+  constexpr int kRing = gemm_ring<kDown, kPl, kCb>();
+  constexpr int kStage = gemm_stage_bytes<kPl, kCb>();  // one step: kTok token rows x 256 bytes per plane
   constexpr int kPlaneStage = kStage / kPlanes;
   constexpr int kLoadsPerStep = kRb + kBInstr * kPlanes;  // A: a chunk per row block; B: kBInstr per plane
-  constexpr bool kScLds = gemm_scales_in_lds<kDown, kPl>();
+  constexpr bool kScLds = gemm_scales_in_lds<kDown, kPl, kCb>();
   static_assert((kRing - 2) * kLoadsPerStep <= 63, "the ring's outstanding loads fit the vmcnt field");
   extern __shared__ __align__(16) uint8_t stage[];    // kRing x kStage
 
@@ -159,12 +213,25 @@ __device__ __forceinline__ void moe_gemm_body(
   const int j0 = blockIdx.x / kXcds;
   const int u = xcd + kXcds * (j0 / row_wgs);
   const int row_wg = j0 % row_wgs;
-  if (j0 >= units_per_xcd * row_wgs || u >= *n_units) return;
-  const int32_t unit = units[u];
-  const int e = unit_expert(unit);
-  const int pb = offsets[e];
-  const int tc = unit_pass(unit) * kUnitTokensGemm;
-  const int nt = min(kUnitTokensGemm, offsets[e + 1] - pb - tc);
+  if (j0 >= units_per_xcd * row_wgs) return;
+  int e, pb, tc, nt, ne;
+  if constexpr (kCb == kGemmCb) {
+    if (u >= *n_units) return;
+    const int32_t unit = units[u];
+    e = unit_expert(unit);
+    pb = offsets[e];
+    tc = unit_pass(unit) * kTok;
+    ne = offsets[e + 1] - pb;
+  } else {
+    if (!find_unit<kTok>(offsets, n_exp, u, e, pb, tc, ne)) return;
+  }
+  nt = min(kTok, ne - tc);
+  // In the narrow kernels an expert of one unit streams its weights past the
+  // caches (B = 64 layer 302 -> 265 us, 300 tokens 352 -> 329, of 128
+  // experts), while the units of a larger one find each other's lines there.
+  // The 64-token kernel gains nothing at its loads (777 tokens of 32 experts
+  // 288 -> 295 us, 2000 of 128 716 -> 728 with the second copy of its loops).
+  const bool only_unit = ne <= kTok;
   const int ncb = (nt + 15) >> 4;
   const int tid = threadIdx.x;
   const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
@@ -249,9 +316,9 @@ __device__ __forceinline__ void moe_gemm_body(
     const int row0 = wtile[rb >> 2] * kTileRows + (rb & 3) * 16 + 4 * lq;
     bias4[rb] = *reinterpret_cast<const u32x2_t*>(bias + (int64_t)e * rows + row0);
   }
-  int pcol[kGemmCb];
+  int pcol[kCb];
 #pragma unroll
-  for (int i = 0; i < kGemmCb; ++i) {
+  for (int i = 0; i < kCb; ++i) {
     // gate_up: the store loop's token c = tid / 16 + 16 i; down: column c = 16 i + lr
     const int c = kDown ? 16 * i + lr : (tid >> 4) + 16 * i;
     pcol[i] = pairs[pb + tc + min(c, nt - 1)];
@@ -281,7 +348,7 @@ __device__ __forceinline__ void moe_gemm_body(
   // round trip, so no wait); lane (lr, lq) of row block rb finds step s at
   // sc_lane[rb * 512 + (s / 8) * 2048 + s % 8].
   static_assert(kWaveTiles == 1, "one scale tile per wave");
-  uint8_t* sc_lds = stage + (gemm_lds_bytes<kDown, kPl>() - kScaleLdsBytes) + wave * kScaleTileLds;
+  uint8_t* sc_lds = stage + (gemm_lds_bytes<kDown, kPl, kCb>() - kScaleLdsBytes) + wave * kScaleTileLds;
   const uint8_t* sc_lane = sc_lds + (lr * 4 + lq) * 8;
   if constexpr (kScLds) {
     // (inputs <= 3072 wide, checked by check_gemv_shapes: rec <= 24)
@@ -299,17 +366,17 @@ __device__ __forceinline__ void moe_gemm_body(
   const __amdgpu_buffer_rsrc_t abuf = __builtin_amdgcn_make_buffer_rsrc(
       (void*)(wptr[e] + tile_off[0]), (short)0, tile_live[0] ? groups * 1024 : 0, kBufferWord3);
   const uint32_t aoff = (uint32_t)(lq * 1024 + lr * 16);
-  auto a_load = [&](int s, u32x4_t (&a)[kRb]) {
+  auto a_load = [&](auto policy, int s, u32x4_t (&a)[kRb]) {
     const uint32_t v = aoff + 4096u * (uint32_t)s;
 #pragma unroll
-    for (int rb = 0; rb < kRb; ++rb) a[rb] = __builtin_amdgcn_raw_buffer_load_b128(abuf, v, (uint32_t)(rb * 256), 0);
+    for (int rb = 0; rb < kRb; ++rb) a[rb] = __builtin_amdgcn_raw_buffer_load_b128(abuf, v, (uint32_t)(rb * 256), decltype(policy)::value);
   };
 
-  f32x4_t acc[kRb][kGemmCb];
+  f32x4_t acc[kRb][kCb];
 #pragma unroll
   for (int rb = 0; rb < kRb; ++rb)
 #pragma unroll
-    for (int cb = 0; cb < kGemmCb; ++cb) acc[rb][cb] = f32x4_t{0.0f, 0.0f, 0.0f, 0.0f};
+    for (int cb = 0; cb < kCb; ++cb) acc[rb][cb] = f32x4_t{0.0f, 0.0f, 0.0f, 0.0f};
 
   // B read offsets: lane (lr, lq) reads piece 4 lq + j of row 16 cb + lr
   // (kept as LDS pointers, one register each: every read of a step is then
@@ -381,7 +448,7 @@ __device__ __forceinline__ void moe_gemm_body(
 #pragma unroll
           for (int rb = 0; rb < kRb; ++rb)
             acc[rb][cb] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(a[rb], bq[j & 1][cb][pl], acc[rb][cb], 0, 0, 0);
-      if constexpr (kDown && kPlanes == 2) {
+      if constexpr (kDown && kPlanes == 2 && kCb == kGemmCb) {
         // down (two planes): each quarter's B read, its kRb MFMAs and kRb VALU
         // instructions as one group, in order (330 against 345 us on the
         // 2048-token layer; the same grouping made gate_up spill and slower)
@@ -396,11 +463,6 @@ __device__ __forceinline__ void moe_gemm_body(
   };
 
   u32x4_t a_ring[kRing][kRb];
-#pragma unroll
-  for (int i = 0; i < kRing - 1; ++i) {
-    a_load(i, a_ring[i]);
-    b_dma(i, i);
-  }
 
   // step s: wait for its own loads (the kRing - 2 later steps' stay in
   // flight), barrier (every wave's B rows of step s have landed and every
@@ -413,7 +475,12 @@ __device__ __forceinline__ void moe_gemm_body(
   // step starts a new dword (s % 4 == 0); with kRing dividing 4 every group
   // starts at a multiple of kRing and needs only the first pick.
   const int steps_pad = (steps + kRing - 1) / kRing * kRing;
-  auto run = [&](auto ncb_c) {
+  auto run_as = [&](auto ncb_c, auto policy) {
+#pragma unroll
+    for (int i = 0; i < kRing - 1; ++i) {
+      a_load(policy, i, a_ring[i]);
+      b_dma(i, i);
+    }
     for (int s0 = 0; s0 < steps_pad; s0 += kRing) {
       uint32_t word[kRb];
 #pragma unroll
@@ -421,18 +488,33 @@ __device__ __forceinline__ void moe_gemm_body(
         const int s = s0 + uu;
         if (!kScLds && (uu == 0 || (4 % kRing != 0 && (s & 3) == 0))) scale_words(s, word);
         ring_barrier<(kRing - 2) * kLoadsPerStep>();
-        a_load(s + kRing - 1, a_ring[(uu + kRing - 1) % kRing]);
+        a_load(policy, s + kRing - 1, a_ring[(uu + kRing - 1) % kRing]);
         b_dma(s + kRing - 1, (uu + kRing - 1) % kRing);
         if (wave_live) compute(ncb_c, s, uu, a_ring[uu], word);
       }
     }
   };
+  auto run = [&](auto ncb_c) {
+    if (kCb < kGemmCb && only_unit)
+      run_as(ncb_c, WeightPolicy<kStreamPolicy>{});
+    else
+      run_as(ncb_c, WeightPolicy<0>{});
+  };
   static_assert(kGemmCb == 4, "one loop per column-block count");
-  switch (ncb) {  // uniform over the workgroup
-    case 1: run(ColumnBlocks<1>{}); break;
-    case 2: run(ColumnBlocks<2>{}); break;
-    case 3: run(ColumnBlocks<3>{}); break;
-    default: run(ColumnBlocks<4>{}); break;
+  if constexpr (kCb == 1) {
+    run(ColumnBlocks<1>{});
+  } else if constexpr (kCb == 2) {
+    if (ncb == 1)
+      run(ColumnBlocks<1>{});
+    else
+      run(ColumnBlocks<2>{});
+  } else {
+    switch (ncb) {  // uniform over the workgroup
+      case 1: run(ColumnBlocks<1>{}); break;
+      case 2: run(ColumnBlocks<2>{}); break;
+      case 3: run(ColumnBlocks<3>{}); break;
+      default: run(ColumnBlocks<4>{}); break;
+    }
   }
   __builtin_amdgcn_s_waitcnt(vmcnt_imm(0));  // no LDS-DMA may outlive the workgroup
 
@@ -441,12 +523,12 @@ __device__ __forceinline__ void moe_gemm_body(
     // SwiGLU outputs of the workgroup (128 columns x up to 64 tokens) go
     // through LDS (the ring is idle now), so each token's 128 outputs leave
     // as 16-byte stores instead of 2-byte ones scattered over 16 rows
-    static_assert(kUnitTokensGemm * kYStride * 4 <= gemm_lds_bytes<false, 1>(), "the output tile fits in the LDS");
+    static_assert(kTok * kYStride * 4 <= gemm_lds_bytes<false, 1, kCb>(), "the output tile fits in the LDS");
     float* ytile = reinterpret_cast<float*>(stage);
     __syncthreads();  // every wave is done reading the ring
     if (wave_live) {
 #pragma unroll
-      for (int cb = 0; cb < kGemmCb; ++cb) {
+      for (int cb = 0; cb < kCb; ++cb) {
         if (cb >= ncb) continue;
         const int c = cb * 16 + lr;
 #pragma unroll
@@ -473,9 +555,9 @@ __device__ __forceinline__ void moe_gemm_body(
     const int col0 = row_wg * (kGemmRows / 2);
     const int ncols = min(kGemmRows / 2, half - col0);
     constexpr int kPieces = kGemmRows / 16;  // 8-column pieces of a token's outputs
-    static_assert(kPieces == 16 && kUnitTokensGemm * kPieces == kGemmCb * kGemmThreads, "thread i covers token i / 16 + 16 it");
+    static_assert(kPieces == 16 && kTok * kPieces == kCb * kGemmThreads, "thread i covers token i / 16 + 16 it");
 #pragma unroll
-    for (int it = 0; it < kGemmCb; ++it) {  // (token, 8-column piece)
+    for (int it = 0; it < kCb; ++it) {  // (token, 8-column piece)
       const int i = tid + it * kGemmThreads;
       const int c = i / kPieces;
       const int ch = (i % kPieces) * 8;
@@ -507,7 +589,7 @@ __device__ __forceinline__ void moe_gemm_body(
   } else {
     if (!wave_live) return;
 #pragma unroll
-    for (int cb = 0; cb < kGemmCb; ++cb) {
+    for (int cb = 0; cb < kCb; ++cb) {
       if (cb >= ncb) continue;
       const int c = cb * 16 + lr;
       if (c >= nt) continue;
@@ -533,26 +615,51 @@ __device__ __forceinline__ void moe_gemm_body(
 #ifndef KLC_GEMM_WAVES_PER_EU
 #define KLC_GEMM_WAVES_PER_EU 2
 #endif
-// The kernels: planes below 2 GiB (every layer call) and past it.
-template <bool kDown, int kPl>
-__global__ __launch_bounds__(kGemmThreads) __attribute__((amdgpu_waves_per_eu(KLC_GEMM_WAVES_PER_EU))) void moe_gemm_kernel(
-    const uint8_t* const* __restrict__ wptr, const uint16_t* __restrict__ bias, const uint16_t* __restrict__ act,
-    int64_t act_plane, float* __restrict__ out, uint16_t* __restrict__ out_split, int64_t out_plane,
-    float* __restrict__ out_raw, const int32_t* __restrict__ offsets, const int32_t* __restrict__ pairs,
-    const int32_t* __restrict__ units, const int32_t* __restrict__ n_units, int rows, int groups, int k_top,
-    float limit, int precision, int row_wgs, int units_per_xcd) {
-  moe_gemm_body<kDown, kPl, false>(wptr, bias, act, act_plane, out, out_split, out_plane, out_raw, offsets, pairs,
-                                   units, n_units, rows, groups, k_top, limit, precision, row_wgs, units_per_xcd);
+// Waves per SIMD: two for the 64-token kernels (their accumulators fill the
+// registers), more for the narrow ones.
+template <int kCb>
+__host__ __device__ constexpr int gemm_waves_per_eu() {
+  return kCb == 1 ? 4 : kCb == 2 ? 3 : KLC_GEMM_WAVES_PER_EU;
 }
-template <bool kDown, int kPl>
-__global__ __launch_bounds__(kGemmThreads) __attribute__((amdgpu_waves_per_eu(KLC_GEMM_WAVES_PER_EU))) void moe_gemm_wide_kernel(
+// The kernels: planes below 2 GiB (every layer call) and past it.
+template <bool kDown, int kPl, int kCb, bool kWide>
+__global__ __launch_bounds__(kGemmThreads) __attribute__((amdgpu_waves_per_eu(gemm_waves_per_eu<kCb>()))) void moe_gemm_kernel(
     const uint8_t* const* __restrict__ wptr, const uint16_t* __restrict__ bias, const uint16_t* __restrict__ act,
     int64_t act_plane, float* __restrict__ out, uint16_t* __restrict__ out_split, int64_t out_plane,
     float* __restrict__ out_raw, const int32_t* __restrict__ offsets, const int32_t* __restrict__ pairs,
     const int32_t* __restrict__ units, const int32_t* __restrict__ n_units, int rows, int groups, int k_top,
-    float limit, int precision, int row_wgs, int units_per_xcd) {
-  moe_gemm_body<kDown, kPl, true>(wptr, bias, act, act_plane, out, out_split, out_plane, out_raw, offsets, pairs,
-                                  units, n_units, rows, groups, k_top, limit, precision, row_wgs, units_per_xcd);
+    float limit, int precision, int row_wgs, int units_per_xcd, int n_exp) {
+  moe_gemm_body<kDown, kPl, kCb, kWide>(wptr, bias, act, act_plane, out, out_split, out_plane, out_raw, offsets, pairs,
+                                        units, n_units, rows, groups, k_top, limit, precision, row_wgs, units_per_xcd, n_exp);
+}
+
+// Tokens per unit (in 16-token column blocks) by the call's mean pairs per
+// expert.  Below ~22 pairs an expert's weights are read for few tokens and the
+// layer is a weight stream: 16- and 32-token units leave registers and LDS for
+// 4 and 3 waves per SIMD instead of 2.  Layer times of 128 experts, float32
+// (16 / 32 / 64 tokens per unit): 100 tokens (3.1 pairs) 292 / 299 / 315 us,
+// 200 (6.3) 322 / 321 / 340, 300 (9.4) 345 / 330 / 355, 450 (14) 398 / 354 /
+// 386, 700 (22) 501 / 426 / 435, 1000 (31) 620 / 500 / 478; 32 experts, 200
+// tokens (25) 174 / 151 / 150.  Skewed loads split their hot experts over
+// more units: 300 tokens at Zipf 1.1 372 / 372 / 403.
+int gemm_column_blocks(int64_t n_pairs, int64_t n_exp, bool wide) {
+  if (wide) return kGemmCb;
+  if (n_pairs <= 5 * n_exp) return 1;
+  if (n_pairs <= 23 * n_exp) return 2;
+  return kGemmCb;
+}
+
+template <bool kDown, int kPl, int kCb, bool kWide>
+void run_gemm(int64_t n_pairs, int64_t n_exp, int row_wgs, hipStream_t stream, const uint8_t* const* w,
+              const uint16_t* bias, const uint16_t* act, int64_t act_plane, float* out, uint16_t* out_split,
+              int64_t out_plane, float* out_raw, const int32_t* offsets, const int32_t* pairs, const int32_t* units,
+              const int32_t* n_units, int rows, int groups, int k_top, float limit, int precision) {
+  const int per_xcd = (int)((units_capacity(n_pairs, n_exp, 16 * kCb) + kXcds - 1) / kXcds);
+  const unsigned grid = (unsigned)(kXcds * per_xcd * row_wgs);
+  moe_gemm_kernel<kDown, kPl, kCb, kWide>
+      <<<grid, kGemmThreads, gemm_lds_bytes<kDown, kPl, kCb>(), stream>>>(w, bias, act, act_plane, out, out_split, out_plane, out_raw, offsets,
+                                                                 pairs, units, n_units, rows, groups, k_top, limit,
+                                                                 precision, row_wgs, per_xcd, (int)n_exp);
 }
 
 }  // namespace
@@ -564,16 +671,16 @@ int launch_gemm_gate_up(const void* const* w, const void* bias, const void* x, i
   const int64_t n_pairs = n_tok * k;
   const int64_t rows = 2 * inter;
   const int row_wgs = (int)((rows + kGemmRows - 1) / kGemmRows);
-  const int per_xcd = (int)((units_capacity(n_pairs, n_exp, kUnitTokensGemm) + kXcds - 1) / kXcds);
-  const dim3 grid((unsigned)(kXcds * per_xcd * row_wgs));
   const int groups = (int)(hidden / 32);
-  // activation planes past 2 GiB take the 64-bit-pointer form
-  auto kernel = n_tok * hidden * 2 > 0x7fffffff ? moe_gemm_wide_kernel<false, 1> : moe_gemm_kernel<false, 1>;
-  kernel<<<grid, kGemmThreads, gemm_lds_bytes<false, 1>(), stream>>>(
-      reinterpret_cast<const uint8_t* const*>(w), static_cast<const uint16_t*>(bias), static_cast<const uint16_t*>(x),
-      0, nullptr, static_cast<uint16_t*>(gated_split), n_pairs * inter, gated_raw, offsets, pairs,
-      units + units_offset_gemm(n_pairs, n_exp), units + 2, (int)rows, groups, (int)k, limit, precision,
-      row_wgs, per_xcd);
+  const bool wide = n_tok * hidden * 2 > 0x7fffffff;
+  const int cb = gemm_column_blocks(n_pairs, n_exp, wide);
+  auto run = cb == 1 ? run_gemm<false, 1, 1, false> : cb == 2 ? run_gemm<false, 1, 2, false>
+             : wide  ? run_gemm<false, 1, kGemmCb, true>
+                     : run_gemm<false, 1, kGemmCb, false>;
+  run(n_pairs, n_exp, row_wgs, stream, reinterpret_cast<const uint8_t* const*>(w), static_cast<const uint16_t*>(bias),
+      static_cast<const uint16_t*>(x), 0, nullptr, static_cast<uint16_t*>(gated_split), n_pairs * inter, gated_raw,
+      offsets, pairs, units + units_offset_gemm(n_pairs, n_exp), units + 2, (int)rows, groups, (int)k, limit,
+      precision);
   return check_launch("moe_gemm_kernel<gate_up>");
 }
 
@@ -581,20 +688,18 @@ int launch_gemm_down(const void* const* w, const void* bias, const void* gated_s
                      const int32_t* offsets, const int32_t* pairs, const int32_t* units, int64_t hidden, int64_t inter,
                      int precision, float* eo, hipStream_t stream) {
   const int row_wgs = (int)((hidden + kGemmRows - 1) / kGemmRows);
-  const int per_xcd = (int)((units_capacity(n_pairs, n_exp, kUnitTokensGemm) + kXcds - 1) / kXcds);
-  const dim3 grid((unsigned)(kXcds * per_xcd * row_wgs));
   const int groups = (int)(inter / 32);
-  // bfloat16 precision: the input is the hi plane alone (its lo plane is zero)
-  // activation planes past 2 GiB take the 64-bit-pointer form
   const bool wide = n_pairs * inter * 2 > 0x7fffffff;
-  auto kernel = precision == KLC_PRECISION_BF16 ? (wide ? moe_gemm_wide_kernel<true, 1> : moe_gemm_kernel<true, 1>)
-                                                : (wide ? moe_gemm_wide_kernel<true, 2> : moe_gemm_kernel<true, 2>);
-  const int lds = precision == KLC_PRECISION_BF16 ? gemm_lds_bytes<true, 1>() : gemm_lds_bytes<true, 2>();
-  kernel<<<grid, kGemmThreads, lds, stream>>>(
-      reinterpret_cast<const uint8_t* const*>(w), static_cast<const uint16_t*>(bias),
+  const int cb = gemm_column_blocks(n_pairs, n_exp, wide);
+  // bfloat16 precision: the input is the hi plane alone (its lo plane is zero)
+  const bool one = precision == KLC_PRECISION_BF16;
+  auto run = cb == 1   ? (one ? run_gemm<true, 1, 1, false> : run_gemm<true, 2, 1, false>)
+             : cb == 2 ? (one ? run_gemm<true, 1, 2, false> : run_gemm<true, 2, 2, false>)
+             : wide    ? (one ? run_gemm<true, 1, kGemmCb, true> : run_gemm<true, 2, kGemmCb, true>)
+                       : (one ? run_gemm<true, 1, kGemmCb, false> : run_gemm<true, 2, kGemmCb, false>);
+  run(n_pairs, n_exp, row_wgs, stream, reinterpret_cast<const uint8_t* const*>(w), static_cast<const uint16_t*>(bias),
       static_cast<const uint16_t*>(gated_split), n_pairs * inter, eo, nullptr, 0, nullptr, offsets, pairs,
-      units + units_offset_gemm(n_pairs, n_exp), units + 2, (int)hidden, groups, 1, 0.0f, precision,
-      row_wgs, per_xcd);
+      units + units_offset_gemm(n_pairs, n_exp), units + 2, (int)hidden, groups, 1, 0.0f, precision);
   return check_launch("moe_gemm_kernel<down>");
 }
 

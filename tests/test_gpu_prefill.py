@@ -74,6 +74,40 @@ def test_gemm_units_span_hot_experts(gpu):
     assert_final_close(bf16_bits(det["out"]), ref)
 
 
+@pytest.mark.parametrize("n_tok,k,n_exp,hot,precision", [
+    (1, 1, 1, 0, "fp32"), (5, 1, 1, 0, "bf16"), (23, 1, 1, 0, "fp32"), (20, 4, 16, 0, "fp32"), (21, 4, 16, 0, "bf16"),
+    (60, 4, 64, 3, "fp32"), (33, 2, 66, 1, "bf16"), (90, 4, 255, 2, "fp32"), (92, 4, 16, 0, "fp32"),
+    (93, 4, 16, 0, "fp32"), (97, 4, 17, 2, "bf16"), (250, 4, 256, 4, "fp32")])
+def test_gemm_narrow_units_match_oracle(gpu, n_tok, k, n_exp, hot, precision):
+    """The 16-token kernels (up to 5 pairs per expert), the 32-token ones (up to 23) and the line to the
+    64-token ones; `hot` experts take every token (several units each, found by the scan of the offsets
+    anywhere among up to 256 experts), the rest are spread or empty.  Every kernel sums a product in the
+    same order, so repeating the tokens until the 64-token kernel runs gives the same bits.  Against the
+    oracle in float32 only: in bfloat16 mode a SwiGLU value that two float32 sums round to neighbouring
+    bfloat16 values moves an output by its unit (2^-8 of it) times a weight (up to 6 x 2^-3), past the
+    bound for outputs that are small by cancellation (1 of 99,328 here)."""
+    bias = None
+    if hot:
+        bias = np.zeros(n_exp, dtype=np.uint16)
+        bias[[(i * 97 + n_exp - 1) % n_exp for i in range(hot)]] = 0x42C8  # +100.0
+    host, dev_w, x = build(gpu, 600 + n_tok + n_exp, 256, 320, n_exp, n_tok, bias_override=bias)
+    layer = moe.MoELayer(dev_w, k, precision=precision, path="gemm")
+    xt = bf16_tensor(x, gpu)
+    det = layer.forward_detailed(xt)
+    fused = layer.forward(xt)
+    wide = layer.forward_detailed(xt.repeat(24 * n_exp // (n_tok * k) + 1, 1))
+    for name in ("ids", "gated", "expert_out", "out"):
+        got = det[name].reshape(n_tok, -1)
+        assert torch.equal(got, wide[name].reshape(wide["out"].shape[0], -1)[:n_tok]), name
+    assert torch.equal(fused, det["out"])
+    ref = oracle_layer(host, x, k, precision)
+    assert np.array_equal(det["ids"].cpu().numpy(), ref["ids"])
+    assert_close(det["gated"].cpu().numpy().reshape(n_tok, k, -1), ref["gated"], "SwiGLU output", precision)
+    if precision == "fp32":
+        assert_close(det["expert_out"].cpu().numpy().reshape(n_tok, k, -1), ref["expert_out"], "expert output")
+        assert_final_close(bf16_bits(det["out"]), ref, precision)
+
+
 def test_gemm_and_gemv_paths_agree(gpu):
     host, dev_w, x = build(gpu, 55, 256, 128, 16, 24)
     xt = bf16_tensor(x, gpu)
