@@ -2,15 +2,16 @@
 //
 // Dequant is HBM bound (1 byte of codes + 1/32 byte of scale in, 2 or 4 bytes
 // out per value), and the transposed [in, out] output sets its pace: each
-// output row is one input column of the checkpoint, so what counts is that a
-// workgroup writes long runs of every output row it touches and that there
-// are enough workgroups for the chip however few matrices a call has.
-// Measured against workgroups that own 64 output columns for all groups:
-// 1 x 5760 x 90 groups to float16 25.0 -> 10.4 us, 16 x 2880 x 90 75 -> 73,
-// 100 x 2880 x 90 to float32 1,386 -> 749 (5.0 TB/s, a copy's rate), 32 x 2881
-// x 90 to bfloat16 468 -> 171 (odd rows: one unaligned 16-byte store instead
-// of eight 2-byte ones), one packed 5760 x 90 to bfloat16 24.7 -> 8.9; 128 x
-// 2880 x 90 to bfloat16 stays at 502 us (5.35 TB/s).  Values come from
+// output row is one input column of the checkpoint, so workgroups write runs
+// of every output row they touch, of a length that follows the call's size,
+// and there are enough of them for the chip however few matrices it has.
+// Measured against one workgroup per 64 output columns and all groups (and
+// 768 columns x 4 groups for bfloat16 of 64-row multiples): 1 x 5760 x 90
+// groups to float16 24.4 -> 9.5 us, 16 x 2880 x 90 59 -> 54, 100 x 2880 x 90
+// to float32 1,386 -> 733 (5.1 TB/s, a copy's rate), 32 x 2881 x 90 to
+// bfloat16 468 -> 171 (odd rows: one unaligned 16-byte store instead of eight
+// 2-byte ones), one packed 5760 x 90 24.7 -> 8.8, 128 x 2880 x 90 to bfloat16
+// 507 -> 469 (5.7 TB/s).  Values come from
 // gfx950's scaled E2M1 conversions (v_cvt_scalef32_pk_{bf16,f16,f32}_fp4),
 // exact for every scale byte below 255; the MX NaN scale 255 takes an integer
 // path (mxfp4_f32_bits) that reproduces the reference's +-inf / NaN.
@@ -71,14 +72,14 @@ __device__ __forceinline__ void store_piece(void* dst, u32x4_t v) {
   }
 }
 
-// MXFP4 -> dense [in, out] in long output runs: workgroup (matrix, column
-// block, group quad) stages 4 groups' code chunks and scale bytes of up to
+// MXFP4 -> dense [in, out]: workgroup (matrix, column block, part of the
+// groups) stages up to kGroups groups' code chunks and scale bytes of up to
 // kCols checkpoint rows (= output columns) in LDS, word-major (word w of row
-// r at sw[w * kCols + r]), and writes output rows 128 q .. 128 q + 127 at its
-// columns.  In the checkpoint layout the 4 groups are a 64-byte run of each
-// row, and the two quads that share a 128-byte line of each row run side by
-// side on one XCD (workgroups go to the XCDs round-robin), so that line is
-// fetched once; in the packed layout a group's chunks of 64 rows are
+// r at sw[w * kCols + r]), and writes its 32 x groups output rows at its
+// columns.  In the checkpoint layout a row's chunks of the part are
+// contiguous, and the two parts that share a 128-byte line of each row run
+// side by side on one XCD (workgroups go to the XCDs round-robin), so that
+// line is fetched once; in the packed layout a group's chunks of 64 rows are
 // contiguous.  A task is 8 output rows (a band: one word of one group's
 // chunks) x 16 bytes of output columns; the threads take consecutive tasks,
 // so a task's 8 stores are, across the workgroup, runs of consecutive 16-byte
@@ -88,7 +89,6 @@ __device__ __forceinline__ void store_piece(void* dst, u32x4_t v) {
 // tasks are written again with the exact integer path (mxfp4_f32_bits) after
 // the main loop, by the thread that wrote them (program order), so the main
 // loop has no branch for it.
-constexpr int kDqGroups = 4;  // groups per workgroup
 
 // Column block cb of nb over rows: nearly equal widths, multiples of 64 columns but for the last
 __host__ __device__ inline int dq_col0(int rows, int nb, int cb) {
@@ -96,31 +96,33 @@ __host__ __device__ inline int dq_col0(int rows, int nb, int cb) {
   return col < rows ? col : rows;
 }
 
-template <int kDtype, bool kPacked, bool kAligned, int kThreads, int kCols>
+template <int kDtype, bool kPacked, bool kAligned, int kThreads, int kCols, int kGroups>
 __global__ __launch_bounds__(kThreads) void dequant_kernel(const uint8_t* __restrict__ blocks,
                                                            const uint8_t* __restrict__ scales, uint8_t* __restrict__ out,
                                                            int n_mat, int rows, int groups, int nb,
                                                            int64_t packed_stride) {
   constexpr int kElem = kDtype == KLC_DTYPE_F32 ? 4 : 2;
   constexpr int kPiece = 16 / kElem;                     // output columns of a 16-byte piece
-  constexpr int kRounds = kCols * kDqGroups / kThreads;  // 16-byte loads per thread
-  static_assert(kCols * kDqGroups % kThreads == 0, "whole load rounds");
-  __shared__ __align__(16) uint32_t sw[4 * kDqGroups * kCols];
-  __shared__ __align__(16) uint8_t ss[kDqGroups * kCols];
+  constexpr int kRounds = kCols * kGroups / kThreads;  // 16-byte loads per thread
+  static_assert(kCols * kGroups % kThreads == 0, "whole load rounds");
+  __shared__ __align__(16) uint32_t sw[4 * kGroups * kCols];
+  __shared__ __align__(16) uint8_t ss[kGroups * kCols];
   // workgroup -> (pair of quads P, half h): P's two workgroups are 8 apart in a window of 16
-  const int quads = (groups + kDqGroups - 1) / kDqGroups;
-  const int pairs = (quads + 1) / 2;
+  const int parts = (groups + kGroups - 1) / kGroups;
+  const int pairs = (parts + 1) / 2;
   const int b = blockIdx.x;
   const int pair = (b >> 4) * 8 + (b & 7);
-  const int quad = 2 * (pair % pairs) + ((b >> 3) & 1);
+  const int part = 2 * (pair % pairs) + ((b >> 3) & 1);
   const int mcb = pair / pairs;  // (matrix, column block)
-  if (quad >= quads || mcb >= n_mat * nb) return;
+  if (part >= parts || mcb >= n_mat * nb) return;
   const int m = mcb / nb;
   const int cb = mcb - m * nb;
   const int col0 = dq_col0(rows, nb, cb);
   const int ncols = dq_col0(rows, nb, cb + 1) - col0;
-  const int g0 = quad * kDqGroups;
-  const int ng = min(kDqGroups, groups - g0);
+  // parts of nearly equal size (17 groups in parts of 8, 8 and 1 leave a third of the workgroups idle);
+  // 4-group parts stay whole 64-byte runs
+  const int g0 = kGroups > 4 ? (int)((int64_t)groups * part / parts) : part * kGroups;
+  const int ng = (kGroups > 4 ? (int)((int64_t)groups * (part + 1) / parts) : min(groups, g0 + kGroups)) - g0;
   const int tid = threadIdx.x;
   // Load i of this thread is chunk c of row r; rows and groups past the end
   // read the last one again (the line is there already), so no load is
@@ -128,11 +130,11 @@ __global__ __launch_bounds__(kThreads) void dequant_kernel(const uint8_t* __rest
   auto where = [&](int i, int& r, int& c) {
     const int idx = tid + i * kThreads;
     if constexpr (kPacked) {  // a wave reads one group's 64-row tile
-      r = (idx & 63) + (idx >> 8) * 64;
-      c = (idx >> 6) & 3;
+      r = (idx & 63) + idx / (64 * kGroups) * 64;
+      c = (idx >> 6) % kGroups;
     } else {
-      r = idx >> 2;
-      c = idx & 3;
+      r = idx / kGroups;
+      c = idx % kGroups;
     }
   };
   u32x4_t v[kRounds];
@@ -391,42 +393,54 @@ int launch_pack(const uint8_t* blocks, const uint8_t* scales, uint8_t* out_block
 
 namespace {
 
-// One launch with workgroups of kThreads over column blocks of at most kCols.
-template <int kDtype, bool kPacked, int kThreads, int kCols>
+// One launch: workgroups of kThreads over nb column blocks of at most kCols
+// columns and parts of at most kGroups groups.
+template <int kDtype, bool kPacked, bool kAligned, int kThreads, int kCols, int kGroups>
 int launch_dequant_shape(const uint8_t* blocks, const uint8_t* scales, uint8_t* out, int64_t n_mat, int64_t rows,
-                         int64_t groups, int64_t nb, int64_t packed_stride, hipStream_t stream) {
-  const int64_t pairs = ((groups + kDqGroups - 1) / kDqGroups + 1) / 2;
+                         int64_t groups, int64_t packed_stride, hipStream_t stream) {
+  const int64_t pairs = ((groups + kGroups - 1) / kGroups + 1) / 2;
+  // narrower blocks (down to 128 columns) until there are 768 workgroups
+  const int64_t least = (rows + kCols - 1) / kCols, most = std::max(least, rows / 128);
+  const int64_t nb = std::clamp((768 + 2 * n_mat * pairs - 1) / (2 * n_mat * pairs), least, most);
   const int64_t grid = (n_mat * nb * pairs + 7) / 8 * 16;
   KLC_REQUIRE(grid <= 0x7fffffff, KLC_ERR_UNSUPPORTED, "dequant: too many matrices (%lld)", (long long)n_mat);
-  if (rows % (kDtype == KLC_DTYPE_F32 ? 4 : 8) == 0) {
-    dequant_kernel<kDtype, kPacked, true, kThreads, kCols><<<(unsigned)grid, kThreads, 0, stream>>>(
-        blocks, scales, out, (int)n_mat, (int)rows, (int)groups, (int)nb, packed_stride);
-  } else if constexpr (!kPacked) {  // packed matrices have whole 64-row tiles
-    dequant_kernel<kDtype, kPacked, false, kThreads, kCols><<<(unsigned)grid, kThreads, 0, stream>>>(
-        blocks, scales, out, (int)n_mat, (int)rows, (int)groups, (int)nb, packed_stride);
-  }
+  dequant_kernel<kDtype, kPacked, kAligned, kThreads, kCols, kGroups><<<(unsigned)grid, kThreads, 0, stream>>>(
+      blocks, scales, out, (int)n_mat, (int)rows, (int)groups, (int)nb, packed_stride);
   return check_launch("dequant_kernel");
 }
 
-// The workgroup shape: long runs (1024 columns, two workgroups per CU) once
-// they give 2048 workgroups, else 384 columns, and fewer (down to 128) until
-// there are 768 workgroups.  Measured, wide against 384 columns: 128 x 2880 x
-// 90 groups to bfloat16 502 against 509 us, 32 x 2881 x 90 (2,304 wide
-// workgroups) 171 against 193; 16 x 2880 x 90 (1,152) packed 66 against 62, 4
-// x 2880 x 90 21.8 against 17.4, 1 x 2880 x 90 8.2 against 6.0 (6.6 without
-// the narrower blocks).
+// The workgroup shape.  16-bit outputs of aligned rows: calls whose input and
+// output fit the 256 MB memory-side cache about twice over read whole 16-group
+// pieces of 64 rows; larger ones write longer runs (128 columns x 8 groups).
+// Measured, 64 x 16 against 128 x 8 (us): 57 x 4160 x 17 groups 51 / 56, 57 x
+// 4160 x 20 59 / 65, 16 x 2880 x 90 54 / 58; 64 x 2880 x 90 266 / 238, 128 x
+// 2880 x 90 534 / 469.  float32 (its runs are twice as long): 384 x 4; 20 x
+// 5760 x 45 125 against 129 with 128 x 8.  Odd row lengths want long runs,
+// since each run's ends share lines with its neighbours': 1024 x 4 once that
+// gives 2048 workgroups (32 x 2881 x 90 171 against 193 us with 384 x 4).
 template <int kDtype, bool kPacked>
 int launch_dequant_as(const uint8_t* blocks, const uint8_t* scales, uint8_t* out, int64_t n_mat, int64_t rows,
                       int64_t groups, int64_t packed_stride, hipStream_t stream) {
-  const int64_t per_block = n_mat * ((groups + 2 * kDqGroups - 1) / (2 * kDqGroups)) * 2;  // workgroups
-  const int64_t wide = (rows + 1023) / 1024;
-  if (per_block * wide >= 2048)
-    return launch_dequant_shape<kDtype, kPacked, 512, 1024>(blocks, scales, out, n_mat, rows, groups, wide,
-                                                            packed_stride, stream);
-  const int64_t most = std::max((rows + 383) / 384, rows / 128);
-  const int64_t nb = std::clamp((768 + per_block - 1) / per_block, (rows + 383) / 384, most);
-  return launch_dequant_shape<kDtype, kPacked, 256, 384>(blocks, scales, out, n_mat, rows, groups, nb, packed_stride,
-                                                         stream);
+  if constexpr (!kPacked) {  // packed matrices have whole 64-row tiles
+    if (rows % (kDtype == KLC_DTYPE_F32 ? 4 : 8) != 0) {
+      if (n_mat * ((groups + 7) / 8) * 2 * ((rows + 1023) / 1024) >= 2048)
+        return launch_dequant_shape<kDtype, false, false, 512, 1024, 4>(blocks, scales, out, n_mat, rows, groups, 0,
+                                                                        stream);
+      return launch_dequant_shape<kDtype, false, false, 256, 384, 4>(blocks, scales, out, n_mat, rows, groups, 0,
+                                                                     stream);
+    }
+  }
+  if constexpr (kDtype == KLC_DTYPE_F32) {
+    return launch_dequant_shape<kDtype, kPacked, true, 256, 384, 4>(blocks, scales, out, n_mat, rows, groups,
+                                                                    packed_stride, stream);
+  } else {
+    const int64_t bytes = n_mat * rows * groups * (17 + 64);
+    if (bytes >= (int64_t)512 << 20)
+      return launch_dequant_shape<kDtype, kPacked, true, 256, 128, 8>(blocks, scales, out, n_mat, rows, groups,
+                                                                      packed_stride, stream);
+    return launch_dequant_shape<kDtype, kPacked, true, 256, 64, 16>(blocks, scales, out, n_mat, rows, groups,
+                                                                    packed_stride, stream);
+  }
 }
 
 template <bool kPacked>

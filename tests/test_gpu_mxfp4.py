@@ -70,10 +70,12 @@ def test_dequant_seeded_matches_oracle(gpu, n_mat, out_dim, groups):
 @pytest.mark.parametrize("dtype,kind", [(torch.bfloat16, "bf16"), (torch.float16, "f16"), (torch.float32, "f32")])
 @pytest.mark.parametrize("n_mat,out_dim,groups", [(1, 1, 1), (2, 7, 5), (1, 63, 9), (3, 65, 4), (1, 385, 8), (1, 770, 3),
                                                    (2, 1028, 1), (5, 129, 11), (1, 5760, 3), (64, 33, 128),
-                                                   (64, 36, 125), (256, 64, 31), (1, 1029, 4093)])
+                                                   (64, 36, 125), (256, 64, 31), (1, 1029, 4093), (2, 72, 17),
+                                                   (1, 136, 90), (3, 200, 33), (17, 2880, 9)])
 def test_dequant_shapes_match_oracle(gpu, n_mat, out_dim, groups, dtype, kind):
-    """Both workgroup shapes (the last four calls take the wide one) over odd and aligned row
-    lengths, partial group quads and column blocks, every scale byte: bit-exact."""
+    """The workgroup shapes of aligned rows (64 x 16, float32 384 x 4) and odd ones (384 x 4, and
+    1024 x 4 where that gives 2048 workgroups: the 33- and 1029-row calls) over partial parts and
+    column blocks, every scale byte: bit-exact.  (128 x 8 starts at 512 MB of input and output.)"""
     blocks, scales = synth.mxfp4_expert_tensors(out_dim, groups, n_mat, out_dim, groups * 32, 0, 255)
     got = ops.mxfp4_dequant(torch.from_numpy(blocks).to(gpu), torch.from_numpy(scales).to(gpu), dtype)
     g = bf16_bits(got) if kind == "bf16" else got.cpu().numpy()
@@ -82,6 +84,25 @@ def test_dequant_shapes_match_oracle(gpu, n_mat, out_dim, groups, dtype, kind):
         packed = ops.mxfp4_pack(torch.from_numpy(blocks).to(gpu), torch.from_numpy(scales).to(gpu))
         again = ops.mxfp4_dequant_packed(packed, out_dim, groups, dtype)
         assert torch.equal(again.view(torch.uint8), got.view(torch.uint8))
+
+
+def test_dequant_large_call_equals_its_halves(gpu):
+    """160 x 2888 x 90 groups to bfloat16 (3.4 GB) takes the large-call shape, 2 matrices the small
+    one: the same bits, checkpoint and (2,880 rows) packed layout."""
+    g = torch.Generator(device=gpu).manual_seed(9)
+    for rows in (2888, 2880):
+        blocks = torch.randint(0, 256, (20, rows, 90, 16), dtype=torch.uint8, device=gpu, generator=g)
+        scales = torch.randint(0, 256, (20, rows, 90), dtype=torch.uint8, device=gpu, generator=g)
+        packed = ops.mxfp4_pack(blocks, scales) if rows == 2880 else None
+        big = ops.mxfp4_dequant(blocks.repeat(8, 1, 1, 1), scales.repeat(8, 1, 1)).view(torch.int16)
+        for i in range(0, 20, 2):
+            part = ops.mxfp4_dequant(blocks[i:i + 2], scales[i:i + 2]).view(torch.int16)
+            assert torch.equal(big[i:i + 2], part) and torch.equal(big[140 + i:142 + i], part)
+        if packed is not None:
+            again = ops.mxfp4_dequant_packed(packed.repeat(8, 1), rows, 90).view(torch.int16)
+            assert torch.equal(again, big)
+        del big, part
+        torch.cuda.empty_cache()
 
 
 def test_dequant_single_matrix_shape_and_errors(gpu):
