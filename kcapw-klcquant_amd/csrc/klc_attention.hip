@@ -17,15 +17,15 @@
 // rounded to the cache's type and then to bfloat16 (o_proj's input type).
 //
 // Kernels per step: scores with per-block maxima and sums (workgroup = one KV
-// head x 64 or 256 keys, its whole query group), probabilities x values
+// head x 64 to 256 keys, its whole query group), probabilities x values
 // (workgroup = one KV head x 128 or 256 keys), and the sum of the splits; a
 // window of at most 256 keys runs as one launch, scores to context, one
 // workgroup per query head.  Measured for 64 / 8 heads x 64, float16 (cold
-// rings): 4,096 keys 23.7 -> 17.6 us, 8,192 40.2 -> 21.2, 16,384 81.6 ->
-// 29.8, 32,768 200 -> 43.2 against value workgroups per query head that each
-// took their head's statistics over all its scores (quadratic in the
-// context: 186 of the 200 us) and vector float64 dot products per query head
-// (38 us -> 20).
+// rings): 128 keys 7.7 -> 6.0 us, 4,096 23.7 -> 16.5, 8,192 40.2 -> 20.5,
+// 16,384 81.6 -> 27.6, 32,768 200 -> 42.7 against value workgroups per query
+// head that each took their head's statistics over all its scores (quadratic
+// in the context: 186 of the 200 us) and vector float64 dot products per
+// query head (38 us -> 20).
 #include <math.h>
 
 #include "klc_common.h"
@@ -310,155 +310,6 @@ __device__ __forceinline__ void write_record(const StepRecord& rec, int nh, int 
   if (lane == 0) __hip_atomic_store(rec.host + 8, rec.tag, __ATOMIC_RELEASE, __HIP_MEMORY_SCOPE_SYSTEM);
 }
 
-// Query head h's m = max(scores, sink) and l = sum exp(x - m) over [scores,
-// sink], l summed in float64 and rounded once; each reduction is a wave
-// shuffle tree plus one exchange of the 4 waves' values.  Every thread of
-// the workgroup calls it and gets both.
-__device__ __forceinline__ void head_stats(const float* __restrict__ s, int count, const uint16_t* __restrict__ sinks,
-                                           int h, float& m_out, float& l_out) {
-  __shared__ float wm[kAttnThreads / kWave];
-  __shared__ double wl[kAttnThreads / kWave];
-  const int lane = threadIdx.x % kWave, wave = threadIdx.x / kWave;
-  // both passes issue 8 loads before using them (a thread's scores are
-  // otherwise a chain of dependent L2 round trips); the sum keeps the
-  // thread's order i, i + 256, ...
-  constexpr int kAhead = 8;
-  float m = sinks != nullptr ? bf(sinks[h]) : -INFINITY;
-  int i = threadIdx.x;
-  for (; i + (kAhead - 1) * kAttnThreads < count; i += kAhead * kAttnThreads) {
-    float x[kAhead];
-#pragma unroll
-    for (int j = 0; j < kAhead; ++j) x[j] = s[i + j * kAttnThreads];
-#pragma unroll
-    for (int j = 0; j < kAhead; ++j) m = fmaxf(m, x[j]);
-  }
-  for (; i < count; i += kAttnThreads) m = fmaxf(m, s[i]);
-  for (int off = kWave / 2; off > 0; off >>= 1) m = fmaxf(m, __shfl_xor(m, off));
-  if (lane == 0) wm[wave] = m;
-  __syncthreads();
-  m = wm[0];
-  for (int w = 1; w < kAttnThreads / kWave; ++w) m = fmaxf(m, wm[w]);
-  double l = 0.0;
-  i = threadIdx.x;
-  for (; i + (kAhead - 1) * kAttnThreads < count; i += kAhead * kAttnThreads) {
-    float x[kAhead];
-#pragma unroll
-    for (int j = 0; j < kAhead; ++j) x[j] = s[i + j * kAttnThreads];
-#pragma unroll
-    for (int j = 0; j < kAhead; ++j) l += (double)expf(x[j] - m);
-  }
-  for (; i < count; i += kAttnThreads) l += (double)expf(s[i] - m);
-  if (threadIdx.x == 0 && sinks != nullptr) l += (double)expf(bf(sinks[h]) - m);
-  for (int off = kWave / 2; off > 0; off >>= 1) l += __shfl_xor(l, off);
-  if (lane == 0) wl[wave] = l;
-  __syncthreads();
-  double t = 0.0;
-  for (int w = 0; w < kAttnThreads / kWave; ++w) t += wl[w];
-  m_out = m;
-  l_out = (float)t;
-}
-
-// The value half of a window workgroup: the context of query head
-// h = blockIdx.x whose `count` <= 256 scores s_head (LDS) holds; p rounded to
-// the cache type, the slices' float32 sums in `partial` [h][d].
-__device__ __forceinline__ void pv_body(const float* __restrict__ s_head, const uint16_t* __restrict__ sinks,
-                                        const uint16_t* __restrict__ v_cache, float* __restrict__ partial,
-                                        uint16_t* __restrict__ context, int64_t cap, int64_t first, int count, int nh,
-                                        int nkv, int d, bool f16) {
-  __shared__ float p[kPvKeys];
-  __shared__ float acc_s[kAttnThreads / 32][kMaxHeadDim];
-  const int h = blockIdx.x, g = nh / nkv, kvh = h / g;
-  const int nk = count;
-  float m, l;
-  head_stats(s_head, count, sinks, h, m, l);
-  for (int i = threadIdx.x; i < nk; i += kAttnThreads) p[i] = rkv(expf(s_head[i] - m) / l, f16);
-  __syncthreads();
-  // thread (slice, four dims): slices of keys; each thread issues the 8-byte
-  // loads of four keys before their multiply-adds, so L2 round trips overlap
-  const int quads = d / 4, slices = kAttnThreads / quads;
-  const int dq = threadIdx.x % quads, sl = threadIdx.x / quads;
-  float a[4] = {0.f, 0.f, 0.f, 0.f};
-  auto vrow = [&](int i) {
-    return *reinterpret_cast<const uint2*>(v_cache + (((first + i) % cap) * nkv + kvh) * d + 4 * dq);
-  };
-  auto add = [&](float pi, uint2 w) {
-    a[0] = fmaf(pi, kv_f((uint16_t)(w.x & 0xffffu), f16), a[0]);
-    a[1] = fmaf(pi, kv_f((uint16_t)(w.x >> 16), f16), a[1]);
-    a[2] = fmaf(pi, kv_f((uint16_t)(w.y & 0xffffu), f16), a[2]);
-    a[3] = fmaf(pi, kv_f((uint16_t)(w.y >> 16), f16), a[3]);
-  };
-  if (sl < slices) {
-    int i = sl;
-    for (; i + 3 * slices < nk; i += 4 * slices) {
-      const uint2 w0 = vrow(i), w1 = vrow(i + slices), w2 = vrow(i + 2 * slices), w3 = vrow(i + 3 * slices);
-      add(p[i], w0);
-      add(p[i + slices], w1);
-      add(p[i + 2 * slices], w2);
-      add(p[i + 3 * slices], w3);
-    }
-    for (; i < nk; i += slices) add(p[i], vrow(i));
-  }
-  // sum the slices, kAttnThreads / 32 of them at a time through LDS
-  for (int base = 0; base < slices; base += kAttnThreads / 32) {
-    if (sl >= base && sl < base + kAttnThreads / 32) {
-#pragma unroll
-      for (int e = 0; e < 4; ++e) acc_s[sl - base][4 * dq + e] = a[e];
-    }
-    __syncthreads();
-    if ((int)threadIdx.x < d) {
-      float t = 0.f;
-      for (int s2 = 0; s2 < min(kAttnThreads / 32, slices - base); ++s2) t += acc_s[s2][threadIdx.x];
-      float* out = partial + (int64_t)h * d + threadIdx.x;
-      *out = base == 0 ? t : *out + t;
-    }
-    __syncthreads();
-  }
-  if ((int)threadIdx.x < d)
-    context[(int64_t)h * d + threadIdx.x] = to_bf(rkv(partial[(int64_t)h * d + threadIdx.x], f16));
-}
-
-// A window of at most 256 keys in one launch: workgroup = query head
-// blockIdx.x.  Its scores (the same float64 dot products as
-// attn_scores_kernel, one key per thread) go to LDS, then the value body
-// takes the max, the sum and the context.
-__global__ __launch_bounds__(kAttnThreads) void attn_window_kernel(
-    const uint16_t* __restrict__ q, const uint16_t* __restrict__ k_cache, const uint16_t* __restrict__ sinks,
-    const uint16_t* __restrict__ v_cache, float* __restrict__ partial, uint16_t* __restrict__ context, int64_t cap,
-    int64_t first, int count, int nh, int nkv, int d, float sqrt_d, bool f16, StepRecord rec) {
-  if ((int)blockIdx.x == nh) {
-    write_record(rec, nh, nkv, d);
-    return;
-  }
-  __shared__ float qs[kMaxHeadDim];
-  __shared__ float sc[kPvKeys];
-  const int h = blockIdx.x, kvh = h / (nh / nkv);
-  const int key = threadIdx.x;
-  const bool live = key < count;
-  uint4 kr[kMaxHeadDim / 8] = {};
-  const uint16_t* krow = k_cache + (((first + (live ? key : 0)) % cap) * nkv + kvh) * d;
-#pragma unroll
-  for (int c = 0; c < kMaxHeadDim / 8; ++c)
-    if (live && c * 8 < d) kr[c] = *reinterpret_cast<const uint4*>(krow + c * 8);
-  for (int i = threadIdx.x; i < d; i += blockDim.x) qs[i] = bf(q[(int64_t)h * d + i]);
-  __syncthreads();
-  if (live) {
-    double acc = 0.0;
-#pragma unroll
-    for (int c = 0; c < kMaxHeadDim / 8; ++c) {
-      if (c * 8 >= d) break;
-      const uint32_t wd[4] = {kr[c].x, kr[c].y, kr[c].z, kr[c].w};
-#pragma unroll
-      for (int t = 0; t < 4; ++t) {
-        acc = fma((double)kv_f((uint16_t)(wd[t] & 0xffffu), f16), (double)qs[8 * c + 2 * t], acc);
-        acc = fma((double)kv_f((uint16_t)(wd[t] >> 16), f16), (double)qs[8 * c + 2 * t + 1], acc);
-      }
-    }
-    sc[key] = (float)acc / sqrt_d;
-  }
-  __syncthreads();
-  pv_body(sc, sinks, v_cache, partial, context, cap, first, count, nh, nkv, d, f16);
-}
-
 // ring slot of key i of a span starting at slot `first`
 __device__ __forceinline__ int64_t ring_slot(int64_t first, int64_t i, int64_t cap) {
   const int64_t s = first + i;
@@ -472,6 +323,127 @@ __device__ __forceinline__ double kv_d(const uint4& v, int i) {
   return (double)kv_f((uint16_t)((i & 1) ? w >> 16 : w & 0xffffu), kF16);
 }
 
+// A window of at most 256 keys in one launch: workgroup = query head
+// blockIdx.x (a KV head's group would halve the loads and leave the chip
+// idle).  It is a latency chain, so everything it will read is requested at
+// the start: a thread's key row (P threads share a row) and its value rows
+// (thread (key slot, 8 dims)).  Scores are the same correctly rounded
+// float64 dot products as attn_scores_kernel's; every wave takes the maximum
+// and the sum over all of them itself, so the reductions need no exchange
+// between waves.  Measured at 128 keys: 8.3 -> 6.1 us against statistics
+// exchanged through LDS, value loads after them and slice sums through
+// global memory.
+template <int P, int kC, bool kF16>
+__global__ __launch_bounds__(kAttnThreads) void attn_window_kernel(
+    const uint16_t* __restrict__ q, const uint16_t* __restrict__ k_cache, const uint16_t* __restrict__ sinks,
+    const uint16_t* __restrict__ v_cache, uint16_t* __restrict__ context, int64_t cap, int64_t first, int count,
+    int nh, int nkv, int d, float sqrt_d, StepRecord rec) {
+  if ((int)blockIdx.x == nh) {
+    write_record(rec, nh, nkv, d);
+    return;
+  }
+  constexpr int kDims = 64 * kC;             // head_dim <= kDims
+  constexpr int kChunks = kDims / 8 / P;     // 16-byte chunks of a key row per thread
+  __shared__ __align__(16) double qs[kDims];
+  __shared__ __align__(16) float sc[kPvKeys];
+  __shared__ float p[kPvKeys];
+  __shared__ float red[kAttnThreads * 8];    // [slot][d]
+  const int h = blockIdx.x, kvh = h / (nh / nkv);
+  const int key = threadIdx.x / P, part = threadIdx.x % P;
+  const uint16_t* krow = k_cache + (ring_slot(first, min(key, count - 1), cap) * nkv + kvh) * d;
+  uint4 kr[kChunks];
+#pragma unroll
+  for (int c = 0; c < kChunks; ++c) {
+    const int at = 8 * (P * c + part);
+    kr[c] = make_uint4(0, 0, 0, 0);
+    if (at < d) kr[c] = *reinterpret_cast<const uint4*>(krow + at);
+  }
+  const int dl = d / 8, slots = kAttnThreads / dl;
+  const int dq = threadIdx.x % dl, slot = threadIdx.x / dl;
+  constexpr int kAhead = 8;
+  uint4 v[kAhead];
+  auto vrow = [&](int i) {
+    return *reinterpret_cast<const uint4*>(v_cache + (ring_slot(first, min(i, count - 1), cap) * nkv + kvh) * d + 8 * dq);
+  };
+#pragma unroll
+  for (int j = 0; j < kAhead; ++j) {
+    v[j] = make_uint4(0, 0, 0, 0);
+    if (slot + j * slots < count) v[j] = vrow(slot + j * slots);
+  }
+  const float sink = sinks != nullptr ? bf(sinks[h]) : -INFINITY;
+  for (int i = threadIdx.x; i < kDims; i += kAttnThreads) qs[i] = i < d ? (double)bf(q[(int64_t)h * d + i]) : 0.0;
+  __syncthreads();
+  {
+    double acc[2] = {0.0, 0.0};
+#pragma unroll
+    for (int c = 0; c < kChunks; ++c) {
+      const double2* qc = reinterpret_cast<const double2*>(qs + 8 * (P * c + part));
+#pragma unroll
+      for (int e = 0; e < 4; ++e) {
+        const double2 qq = qc[e];
+        acc[0] = fma(kv_d<kF16>(kr[c], 2 * e), qq.x, acc[0]);
+        acc[1] = fma(kv_d<kF16>(kr[c], 2 * e + 1), qq.y, acc[1]);
+      }
+    }
+    double dot = acc[0] + acc[1];
+#pragma unroll
+    for (int off = 1; off < P; off <<= 1) dot += __shfl_xor(dot, off);
+    if (part == 0 && key < count) sc[key] = (float)dot / sqrt_d;
+  }
+  __syncthreads();
+  const int lane = threadIdx.x % kWave, wave = threadIdx.x / kWave;
+  float s[4], m = sink;
+  const float4 s4 = reinterpret_cast<const float4*>(sc)[lane];
+  s[0] = s4.x, s[1] = s4.y, s[2] = s4.z, s[3] = s4.w;
+#pragma unroll
+  for (int e = 0; e < 4; ++e)
+    if (4 * lane + e < count) m = fmaxf(m, s[e]);
+  for (int off = kWave / 2; off > 0; off >>= 1) m = fmaxf(m, __shfl_xor(m, off));
+  double l = 0.0;
+#pragma unroll
+  for (int e = 0; e < 4; ++e) {
+    s[e] = expf(s[e] - m);
+    if (4 * lane + e < count) l += (double)s[e];
+  }
+  for (int off = kWave / 2; off > 0; off >>= 1) l += __shfl_xor(l, off);
+  if (sinks != nullptr) l += (double)expf(sink - m);
+  const float lf = (float)l;
+  if (lane / (kWave / 4) == wave) {  // each wave writes a quarter of the probabilities
+#pragma unroll
+    for (int e = 0; e < 4; ++e) p[4 * lane + e] = 4 * lane + e < count ? rkv(s[e] / lf, kF16) : 0.f;
+  }
+  __syncthreads();
+  float a[8] = {};
+  if (slot < slots) {
+    for (int i0 = slot; i0 < count; i0 += kAhead * slots) {
+      if (i0 != slot) {
+#pragma unroll
+        for (int j = 0; j < kAhead; ++j) v[j] = vrow(i0 + j * slots);
+      }
+#pragma unroll
+      for (int j = 0; j < kAhead; ++j) {
+        if (i0 + j * slots >= count) break;
+        const float w = p[i0 + j * slots];
+#pragma unroll
+        for (int e = 0; e < 8; ++e) {
+          const uint32_t x = e < 2 ? v[j].x : e < 4 ? v[j].y : e < 6 ? v[j].z : v[j].w;
+          a[e] = fmaf(w, kv_f((uint16_t)((e & 1) ? x >> 16 : x & 0xffffu), kF16), a[e]);
+        }
+      }
+    }
+    float4* dst = reinterpret_cast<float4*>(red + slot * d + 8 * dq);
+    dst[0] = make_float4(a[0], a[1], a[2], a[3]);
+    dst[1] = make_float4(a[4], a[5], a[6], a[7]);
+  }
+  __syncthreads();
+  if ((int)threadIdx.x < d) {
+    float t = 0.f;
+#pragma unroll 8
+    for (int i = 0; i < min(slots, count); ++i) t += red[i * d + threadIdx.x];
+    context[(int64_t)h * d + threadIdx.x] = to_bf(rkv(t, kF16));
+  }
+}
+
 // Scores of one KV head's query group against 64 * T keys (blockIdx.y), and
 // per head the block's maximum and sum of exp(score - maximum).
 //
@@ -483,11 +455,11 @@ __device__ __forceinline__ double kv_d(const uint4& v, int i) {
 // row l / 16 + 4 i; tile row m holds key 4 (m % 4) + m / 4, so a lane ends up
 // with 4 consecutive keys of head l % 16 and stores them as one float4.
 // Groups of fewer than 16 heads leave MFMA columns idle.
-template <int T, bool kF16>
+template <int T, int kC, bool kF16>
 __global__ __launch_bounds__(kAttnThreads) void attn_scores_kernel(
     const uint16_t* __restrict__ q, const uint16_t* __restrict__ k_cache, float* __restrict__ scores,
     float* __restrict__ stat_m, double* __restrict__ stat_l, int64_t cap, int64_t first, int count, int cs, int nblk,
-    int nh, int nkv, int d, float sqrt_d, StepRecord rec) {
+    int nh, int nkv, int d, float sqrt_d, float inv_sqrt, StepRecord rec) {
   if ((int)blockIdx.y == nblk) {
     if (blockIdx.x == 0) write_record(rec, nh, nkv, d);
     return;
@@ -499,8 +471,7 @@ __global__ __launch_bounds__(kAttnThreads) void attn_scores_kernel(
   const int lane = threadIdx.x % kWave, wave = threadIdx.x / kWave;
   const int r = lane & 15, kq = lane >> 4;  // MFMA row / column, dim quarter
   const int key0 = (blk * (kAttnThreads / kWave) + wave) * 16 * T;
-  constexpr int kC = kMaxHeadDim / 32;
-  // dims 32 c + 8 kq of the head exist: d is a multiple of 8
+  // kC chunks of 32 dims (head_dim <= 32 kC): dims 32 c + 8 kq of the head exist: d is a multiple of 8
   uint4 kr[T][kC];
 #pragma unroll
   for (int t = 0; t < T; ++t) {
@@ -538,7 +509,8 @@ __global__ __launch_bounds__(kAttnThreads) void attn_scores_kernel(
     const int k4 = key0 + 16 * t + 4 * kq;
 #pragma unroll
     for (int i = 0; i < 4; ++i) {
-      s[t][i] = (float)acc[t][i] / sqrt_d;
+      // a power of two divides exactly as its reciprocal multiplies
+      s[t][i] = inv_sqrt != 0.f ? (float)acc[t][i] * inv_sqrt : (float)acc[t][i] / sqrt_d;
       if (k4 + i < count) m = fmaxf(m, s[t][i]);
     }
     if (r < g && k4 < count)  // rows are padded to 4 scores
@@ -604,7 +576,17 @@ __global__ __launch_bounds__(kAttnThreads) void attn_pv_kernel(
 #pragma unroll
   for (int j = 0; j < kAhead; ++j) v[j] = vrow(min(slot + j * slots, nk - 1));
 
-  // 16 to 256 lanes a head take its statistics, every head at once
+  // and so are the scores
+  constexpr int kHeldScores = kPvKeys * kMaxGroup / kAttnThreads;
+  float sc[kHeldScores];
+#pragma unroll
+  for (int j = 0; j < kHeldScores; ++j) {
+    const int i = threadIdx.x + j * kAttnThreads;
+    const int hh = i >> ks_log2, key = i & (ks - 1);
+    sc[j] = 0.f;
+    if (hh < g) sc[j] = scores[(int64_t)(kvh * g + hh) * cs + k0 + min(key, nk - 1)];
+  }
+  // 16 to 64 lanes a head take its statistics, every head at once
   const int lanes = g > 8 ? 16 : g > 4 ? 32 : 64;
   {
     const int hh = threadIdx.x / lanes, ln = threadIdx.x % lanes;
@@ -637,12 +619,13 @@ __global__ __launch_bounds__(kAttnThreads) void attn_pv_kernel(
   }
   const int stride = 4 * hb + 4;
   __syncthreads();
-#pragma unroll 4
-  for (int i = threadIdx.x; i < ks * 4 * hb; i += kAttnThreads) {
+#pragma unroll
+  for (int j = 0; j < kHeldScores; ++j) {
+    const int i = threadIdx.x + j * kAttnThreads;
     const int hh = i >> ks_log2, key = i & (ks - 1);
+    if (hh >= 4 * hb) break;
     float w = 0.f;
-    if (hh < g && key < nk)
-      w = rkv(expf(scores[(int64_t)(kvh * g + hh) * cs + k0 + key] - head_m[hh]) / head_l[hh], kF16);
+    if (hh < g && key < nk) w = rkv(expf(sc[j] - head_m[hh]) / head_l[hh], kF16);
     p[key * stride + hh] = w;
   }
   __syncthreads();
@@ -726,13 +709,34 @@ struct AttnPlan {
 AttnPlan attn_plan(int64_t count) {
   AttnPlan a;
   a.cs = (count + 3) / 4 * 4;
-  // 64 keys a workgroup keep the chip busy on shorter contexts; past 8,192
-  // keys 256 (fewer block statistics for every value workgroup to read)
-  a.score_keys = count <= 8192 ? 64 : 256;
+  // 64 keys a score workgroup keep the chip busy on shorter contexts; larger
+  // blocks leave fewer statistics for every value workgroup to read.  Core at
+  // 12,000 keys with 64 / 128 / 256: 25.8 / 24.2 / 26.4 us, 16,384 30.6 /
+  // 27.6 / 27.5, 32,768 48.6 / 42.7 / 42.9.
+  a.score_keys = count <= 8192 ? 64 : count <= 65536 ? 128 : 256;
   a.nblk = (count + a.score_keys - 1) / a.score_keys;
-  a.split_keys = count <= 8192 ? 128 : kPvKeys;
+  a.split_keys = count <= 8192 ? 128 : kPvKeys;  // 16,384 keys in splits of 128: 31.3 us against 27.6
   a.splits = (count + a.split_keys - 1) / a.split_keys;
   return a;
+}
+
+using ScoresKernel = void (*)(const uint16_t*, const uint16_t*, float*, float*, double*, int64_t, int64_t, int, int,
+                              int, int, int, int, float, float, StepRecord);
+template <int kC>
+ScoresKernel pick_scores(int64_t keys, bool f16) {
+  if (keys == 128) return f16 ? attn_scores_kernel<2, kC, true> : attn_scores_kernel<2, kC, false>;
+  if (keys == 64) return f16 ? attn_scores_kernel<1, kC, true> : attn_scores_kernel<1, kC, false>;
+  return f16 ? attn_scores_kernel<4, kC, true> : attn_scores_kernel<4, kC, false>;
+}
+
+using WindowKernel = void (*)(const uint16_t*, const uint16_t*, const uint16_t*, const uint16_t*, uint16_t*, int64_t,
+                              int64_t, int, int, int, int, float, StepRecord);
+// threads per key row: 256 threads over the window's keys
+template <int kC>
+WindowKernel pick_window(int n, bool f16) {
+  if (n <= 64) return f16 ? attn_window_kernel<4, kC, true> : attn_window_kernel<4, kC, false>;
+  if (n <= 128) return f16 ? attn_window_kernel<2, kC, true> : attn_window_kernel<2, kC, false>;
+  return f16 ? attn_window_kernel<1, kC, true> : attn_window_kernel<1, kC, false>;
 }
 
 // Scores to context of one token (klc_attn_decode's kernels), with a step's
@@ -743,9 +747,8 @@ int attn_core(const uint16_t* qb, const uint16_t* kb, const uint16_t* vb, const 
   const float sqrt_d = sqrtf((float)d);
   const unsigned extra = rec.host != nullptr ? 1 : 0;  // the record's workgroup (one per KV head in the score grid)
   if (n <= kPvKeys) {  // a window: one launch, one workgroup per query head
-    static_assert(kPvKeys == kAttnThreads, "one key per thread");
-    attn_window_kernel<<<(unsigned)nh + extra, kAttnThreads, 0, st>>>(
-        qb, kb, sk, vb, static_cast<float*>(workspace), ctx, cap, first, n, nh, nkv, d, sqrt_d, f16, rec);
+    auto run = d <= 64 ? pick_window<1>(n, f16) : pick_window<2>(n, f16);
+    run<<<(unsigned)nh + extra, kAttnThreads, 0, st>>>(qb, kb, sk, vb, ctx, cap, first, n, nh, nkv, d, sqrt_d, rec);
     return check_launch("attn_window_kernel");
   }
   const AttnPlan a = attn_plan(n);
@@ -754,10 +757,9 @@ int attn_core(const uint16_t* qb, const uint16_t* kb, const uint16_t* vb, const 
   double* stat_l = reinterpret_cast<double*>(partial + (int64_t)nh * a.splits * d);
   float* stat_m = reinterpret_cast<float*>(stat_l + (int64_t)nh * a.nblk);
   const dim3 sgrid((unsigned)nkv, (unsigned)a.nblk + extra), vgrid((unsigned)nkv, (unsigned)a.splits);
-  auto run_scores = a.score_keys == 64 ? (f16 ? attn_scores_kernel<1, true> : attn_scores_kernel<1, false>)
-                                       : (f16 ? attn_scores_kernel<4, true> : attn_scores_kernel<4, false>);
+  auto run_scores = d <= 64 ? pick_scores<2>(a.score_keys, f16) : pick_scores<4>(a.score_keys, f16);
   run_scores<<<sgrid, kAttnThreads, 0, st>>>(qb, kb, scores, stat_m, stat_l, cap, first, n, (int)a.cs, (int)a.nblk,
-                                             nh, nkv, d, sqrt_d, rec);
+                                             nh, nkv, d, sqrt_d, d == 16 || d == 64 ? 1.f / sqrt_d : 0.f, rec);
   int rc = check_launch("attn_scores_kernel");
   if (rc) return rc;
   auto run_pv = f16 ? attn_pv_kernel<true> : attn_pv_kernel<false>;
