@@ -20,6 +20,7 @@ StreamedAttention) and kv_cache_manager.py (KVCacheManager's methods, here
 from __future__ import annotations
 
 import ctypes
+import functools
 import math
 import struct
 import time
@@ -238,12 +239,6 @@ class _HostRecord:
 _TENSORS = (torch.Tensor, torch.nn.Parameter)
 
 
-def _plain(t, dev: torch.device, shape: tuple) -> bool:
-    """A contiguous bfloat16 tensor of ``shape`` on ``dev``, no subclass."""
-    return (type(t) in _TENSORS and t.dtype is torch.bfloat16 and t.shape == shape and t.device == dev
-            and t.is_contiguous())
-
-
 def _intercepted() -> bool:
     """Something watches or replaces torch calls here (modes, function transforms, forward-mode AD,
     autocast, tracing, stream capture): F.linear has to be seen by it."""
@@ -262,6 +257,8 @@ class StreamedAttention:
         self._tables: dict = {}
         self._workspace: torch.Tensor | None = None
         self._inv_freq: dict = {}
+        self._names: dict = {}  # layer -> the names of its tensors
+        self._need: dict = {}   # sizes -> klc_attn_step's workspace bytes
         self._records: list = []  # pinned host records of klc_attn_step not in use
 
     def _cos_sin(self, position: int, device: torch.device) -> tuple[torch.Tensor, torch.Tensor]:
@@ -285,11 +282,15 @@ class StreamedAttention:
             self._inv_freq[key] = t
         return t
 
+    @functools.cached_property
+    def _step_fn(self):
+        return _native.load().klc_attn_step
+
     # A record the GPU has not written after this long is waited for by a
     # synchronisation of the stream.
     _RECORD_WAIT_S = 2.0
 
-    def _step(self, layer_idx: int, prefix: str, hidden: torch.Tensor, tensors: dict, position: int, kv_cache,
+    def _step(self, layer_idx: int, hidden: torch.Tensor, tensors: dict, position: int, kv_cache,
               sliding_window: int | None):
         """One klc_attn_step call, or None for what that call does not take (the caller's general path)."""
         cfg = self.config
@@ -298,26 +299,35 @@ class StreamedAttention:
         size = hidden.shape[-1] if hidden.dim() else 0
         q, kv = nh * d, nkv * d
         if (type(hidden) is not torch.Tensor or hidden.dtype is not torch.bfloat16 or dev.type != "cuda"
-                or not isinstance(kv_cache, DeviceKVCache) or kv_cache.device.type != "cuda"
+                or not isinstance(kv_cache, DeviceKVCache)
                 or size == 0 or size % 8 or size > 4096 or hidden.numel() != size or not hidden.is_contiguous()
                 or d % 8 or d > 128 or q > 4096 or nh % nkv or nh // nkv > 16 or _intercepted()):
             return None
+        names = self._names.get(layer_idx)
+        if names is None:
+            pre = f"model.layers.{layer_idx}.self_attn"
+            names = self._names[layer_idx] = (*(f"{pre}.{n}_proj.{t}" for t in ("weight", "bias") for n in "qkvo"),
+                                              f"{pre}.sinks")
         get = tensors.get
-        weights = [get(f"{prefix}.{n}_proj.weight") for n in "qkvo"]
-        biases = [get(f"{prefix}.{n}_proj.bias") for n in "qkvo"]
-        sinks = get(f"{prefix}.sinks")
-        o_size = weights[3].shape[0] if isinstance(weights[3], torch.Tensor) and weights[3].dim() == 2 else 0
-        rows = (q, kv, kv, o_size)
-        for w, b, n, k in zip(weights, biases, rows, (size, size, size, q)):
-            if not (_plain(w, dev, (n, k)) and _plain(b, dev, (n,))):
-                return None
-        if o_size == 0 or (sinks is not None and not _plain(sinks, dev, (nh,))):
+        held = [get(n) for n in names]
+        o_weight = held[3]
+        if type(o_weight) not in _TENSORS or o_weight.dim() != 2:
             return None
-        held = [hidden, *weights, *biases] if sinks is None else [hidden, *weights, *biases, sinks]
-        if torch.is_grad_enabled() and any(t.requires_grad for t in held):
+        o_size = o_weight.shape[0]
+        index, grad = dev.index, torch.is_grad_enabled()
+        shapes = ((q, size), (kv, size), (kv, size), (o_size, q), (q,), (kv,), (kv,), (o_size,), (nh,))
+        if held[8] is None:
+            del held[8]
+        # no subclass, contiguous bfloat16 on hidden's device, nothing for autograd to see
+        for t, shape in zip(held, shapes):
+            if (type(t) not in _TENSORS or t.dtype is not torch.bfloat16 or t.shape != shape
+                    or t.get_device() != index or not t.is_contiguous() or (grad and t.requires_grad)):
+                return None
+        if o_size == 0 or (grad and hidden.requires_grad):
             return None
         ptr = [t.data_ptr() for t in held]
-        if (ptr[0] | ptr[1] | ptr[2] | ptr[3] | ptr[4]) % 16:
+        hidden_ptr = hidden.data_ptr()
+        if (hidden_ptr | ptr[0] | ptr[1] | ptr[2] | ptr[3]) % 16:
             return None
         window = sliding_window if sliding_window is not None else cfg.sliding_window
         inv_freq = self._device_inv_freq(dev)
@@ -330,19 +340,26 @@ class StreamedAttention:
         count = min(total, ring["cap"])
         if window:
             count = min(count, window)
-        lib = _native.load()
-        need = lib.klc_attn_step_workspace_bytes(nh, nkv, d, count)
-        workspace = torch.empty(max(need, 16), dtype=torch.uint8, device=dev)
+        sizes = (nh, nkv, d, count)
+        need = self._need.get(sizes)
+        if need is None:
+            if len(self._need) > 1024:
+                self._need.clear()
+            need = self._need[sizes] = _native.call("klc_attn_step_workspace_bytes", *sizes)
+        workspace = torch.empty(need, dtype=torch.uint8, device=dev)
         out = torch.empty(o_size, dtype=torch.bfloat16, device=dev)
-        record = self._records.pop() if self._records else _HostRecord()
+        try:
+            record = self._records.pop()
+        except IndexError:  # none free (or another thread took the last one)
+            record = _HostRecord()
         words = record.words
         words[8] = 0
-        rc = lib.klc_attn_step(
-            _STEP.pack(ptr[0], ptr[1], ptr[5], ptr[2], ptr[6], ptr[3], ptr[7], ptr[4], ptr[8],
-                       0 if sinks is None else ptr[9], inv_freq.data_ptr(), keys.data_ptr(), values.data_ptr(),
+        rc = self._step_fn(
+            _STEP.pack(hidden_ptr, ptr[0], ptr[4], ptr[1], ptr[5], ptr[2], ptr[6], ptr[3], ptr[7],
+                       ptr[8] if len(ptr) == 9 else 0, inv_freq.data_ptr(), keys.data_ptr(), values.data_ptr(),
                        workspace.data_ptr(), out.data_ptr(), record.ptr, size, o_size, nh, nkv, d, ring["cap"], slot,
-                       (total - count) % ring["cap"], count, kv_cache.kv_code, workspace.numel(), 1, float(position),
-                       scaling), torch._C._cuda_getCurrentRawStream(dev.index))
+                       (total - count) % ring["cap"], count, kv_cache.kv_code, need, 1, float(position), scaling),
+            torch._C._cuda_getCurrentRawStream(index))
         if rc < 0:
             raise _native.KlcError("klc_attn_step", int(rc), _native.last_error())
         ring["total"] = total
@@ -368,10 +385,10 @@ class StreamedAttention:
     def forward(self, layer_idx: int, hidden: torch.Tensor, tensors: dict, position: int, kv_cache,
                 sliding_window: int | None = None):
         cfg = self.config
-        prefix = f"model.layers.{layer_idx}.self_attn"
-        stepped = self._step(layer_idx, prefix, hidden, tensors, position, kv_cache, sliding_window)
+        stepped = self._step(layer_idx, hidden, tensors, position, kv_cache, sliding_window)
         if stepped is not None:
             return stepped
+        prefix = f"model.layers.{layer_idx}.self_attn"
         lin = torch.nn.functional.linear
         q = lin(hidden, tensors[f"{prefix}.q_proj.weight"], tensors[f"{prefix}.q_proj.bias"]).view(cfg.num_heads, cfg.head_dim)
         k = lin(hidden, tensors[f"{prefix}.k_proj.weight"], tensors[f"{prefix}.k_proj.bias"]).view(cfg.num_kv_heads, cfg.head_dim)

@@ -278,7 +278,7 @@ def test_attention_step_matches_oracle(gpu, nh, nkv, d, h, rows, count, position
     ring["v"].copy_(torch.randn(ring["v"].shape, generator=g, device=gpu))
     ring["total"] = count + 1  # the token goes to slot 1 % count
     attn = StreamedAttention(cfg)
-    assert attn._step(3, pre, x, t, position, cache, None) is not None, "the one-call path did not take these tensors"
+    assert attn._step(3, x, t, position, cache, None) is not None, "the one-call path did not take these tensors"
     ring["total"] = count + 1
     out, diag = attn.forward(3, x, t, position, cache)
     assert ring["total"] == count + 2
@@ -324,7 +324,7 @@ def test_attention_step_and_general_path_agree(gpu):
             w = {n: v.clone().requires_grad_(grad and n.endswith("o_proj.weight")) for n, v in t.items()}
             cache = DeviceKVCache(gpu, precision="fp16", capacity=4)
             attn = StreamedAttention(cfg)
-            assert (attn._step(0, pre, x, w, 3, DeviceKVCache(gpu, capacity=4), None) is None) == grad
+            assert (attn._step(0, x, w, 3, DeviceKVCache(gpu, capacity=4), None) is None) == grad
             for pos in range(3):
                 out, diag = attn.forward(0, x, w, pos, cache)
             outs.append(out)
