@@ -775,6 +775,12 @@ int64_t attn_bytes(int64_t n_heads, int64_t head_dim, int64_t count) {
   const AttnPlan a = attn_plan(count);
   return n_heads * (4 * a.cs + 12 * a.nblk + 4 * a.splits * head_dim);
 }
+// What a caller is told: the finest plan's bytes, which never shrink with the
+// count, so a workspace made for a ring's capacity serves every shorter span
+int64_t attn_bytes_up_to(int64_t n_heads, int64_t head_dim, int64_t count) {
+  if (count <= kPvKeys) return 4 * n_heads * (count + head_dim);
+  return n_heads * (4 * ((count + 3) / 4 * 4) + 12 * ((count + 63) / 64) + 4 * ((count + 127) / 128) * head_dim);
+}
 
 // Scratch of klc_attn_step before the core's: q and k before and after RoPE, the context
 int64_t step_rows_bytes(int64_t nh, int64_t nkv, int64_t d) { return (2 * (2 * (nh + nkv) + nh) * d + 15) / 16 * 16; }
@@ -826,7 +832,7 @@ extern "C" int klc_rope_append(const void* q, const void* k, const void* v, cons
 extern "C" int64_t klc_attn_workspace_bytes(int64_t n_heads, int64_t head_dim, int64_t count) {
   if (n_heads <= 0 || head_dim <= 0 || count <= 0)
     return set_error(KLC_ERR_ARGUMENT, "klc_attn_workspace_bytes: bad sizes");
-  return attn_bytes(n_heads, head_dim, count);
+  return attn_bytes_up_to(n_heads, head_dim, count);
 }
 
 extern "C" int klc_attn_decode(const void* q, const void* k_cache, const void* v_cache, const void* sinks,
@@ -847,7 +853,7 @@ extern "C" int klc_attn_decode(const void* q, const void* k_cache, const void* v
   KLC_REQUIRE(kv_dtype == KLC_DTYPE_BF16 || kv_dtype == KLC_DTYPE_F16, KLC_ERR_UNSUPPORTED,
               "klc_attn_decode: kv_dtype %d (bfloat16 or float16)", kv_dtype);
   const bool f16 = kv_dtype == KLC_DTYPE_F16;
-  const int64_t need = klc_attn_workspace_bytes(n_heads, head_dim, count);
+  const int64_t need = attn_bytes(n_heads, head_dim, count);
   KLC_REQUIRE(workspace_bytes >= need, KLC_ERR_ARGUMENT, "klc_attn_decode: workspace of %lld bytes, need %lld",
               (long long)workspace_bytes, (long long)need);
   return attn_core(static_cast<const uint16_t*>(q), static_cast<const uint16_t*>(k_cache),
@@ -859,7 +865,7 @@ extern "C" int klc_attn_decode(const void* q, const void* k_cache, const void* v
 extern "C" int64_t klc_attn_step_workspace_bytes(int64_t n_heads, int64_t n_kv, int64_t head_dim, int64_t count) {
   if (n_heads <= 0 || n_kv <= 0 || head_dim <= 0 || count <= 0)
     return set_error(KLC_ERR_ARGUMENT, "klc_attn_step_workspace_bytes: bad sizes");
-  return step_rows_bytes(n_heads, n_kv, head_dim) + attn_bytes(n_heads, head_dim, count);
+  return step_rows_bytes(n_heads, n_kv, head_dim) + attn_bytes_up_to(n_heads, head_dim, count);
 }
 
 extern "C" int klc_attn_step(const klc_attn_step_args* args, void* stream) {
@@ -888,7 +894,7 @@ extern "C" int klc_attn_step(const klc_attn_step_args* args, void* stream) {
               KLC_ERR_ARGUMENT, "klc_attn_step: hidden, weights, caches and workspace must be 16-byte aligned");
   KLC_REQUIRE(a.kv_dtype == KLC_DTYPE_BF16 || a.kv_dtype == KLC_DTYPE_F16, KLC_ERR_UNSUPPORTED,
               "klc_attn_step: kv_dtype %lld (bfloat16 or float16)", (long long)a.kv_dtype);
-  const int64_t need = klc_attn_step_workspace_bytes(nh, nkv, d, a.count);
+  const int64_t need = step_rows_bytes(nh, nkv, d) + attn_bytes(nh, d, a.count);
   KLC_REQUIRE(a.workspace_bytes >= need, KLC_ERR_ARGUMENT, "klc_attn_step: workspace of %lld bytes, need %lld",
               (long long)a.workspace_bytes, (long long)need);
   StepRecord rec{};

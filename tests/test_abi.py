@@ -98,6 +98,17 @@ def test_route_entry_argument_errors():
     assert ei.value.status == nat.KLC_ERR_ARGUMENT and "workspace" in ei.value.message
 
 
+def test_attention_workspace_never_shrinks_with_the_count():
+    """A workspace made for a ring's capacity serves every shorter span, across the lines between
+    the kernels' block sizes (256, 8,192 and 65,536 keys)."""
+    lib = nat.load()
+    for nh, nkv, d in ((64, 8, 64), (8, 8, 128), (3, 1, 8)):
+        for size in (lambda n: lib.klc_attn_workspace_bytes(nh, d, n),
+                     lambda n: lib.klc_attn_step_workspace_bytes(nh, nkv, d, n)):
+            sizes = [size(n) for n in (*range(1, 600), *range(8000, 8400), *range(65400, 65800), 1 << 20, 1 << 22)]
+            assert all(a > 0 for a in sizes) and sizes == sorted(sizes)
+
+
 def test_units_size():
     lib = nat.load()
     # 256 pairs over 128 experts: gate_up (256 + 7 * 128) // 8 = 144, down (256 + 3 * 128) // 4 = 160,
