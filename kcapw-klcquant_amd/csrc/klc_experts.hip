@@ -41,7 +41,7 @@ int64_t decode_router_partial_bytes(int64_t n_tok, int64_t hidden, int64_t n_exp
 int check_router_args(int64_t n_tok, int64_t hidden, int64_t n_exp);
 int launch_gemm_gate_up(const void* const* w, const void* bias, const void* x, int64_t n_tok, int64_t k,
                         int64_t n_exp, const int32_t* offsets, const int32_t* pairs, const int32_t* units,
-                        int64_t hidden, int64_t inter, float limit, int precision, void* gated_split,
+                        int64_t hidden, int64_t inter, float limit, int precision, bool lo_plane, void* gated_split,
                         float* gated_raw, hipStream_t stream);
 int launch_gemm_down(const void* const* w, const void* bias, const void* gated_split, int64_t n_pairs, int64_t n_exp,
                      const int32_t* offsets, const int32_t* pairs, const int32_t* units, int64_t hidden, int64_t inter,
@@ -909,8 +909,11 @@ int run_moe_layer(const void* x, const void* router_w, const void* router_b, con
   const bool gemm = route == KLC_PATH_GEMM;
   if (!gemm && (rc = check_gemv_grid(n_tokens * k, n_experts))) return rc;
   if (gemm) {
+    // in bfloat16 precision down's GEMM reads the hi plane alone: the zero lo plane is not written
+    // (47 MB at 2048 tokens: layer 640 -> 634 us; 2911 tokens, top-2, 2048 x 2048: 302 -> 296)
+    const bool lo_plane = precision != KLC_PRECISION_BF16;
     if ((rc = launch_gemm_gate_up(w_gate_up, gate_up_bias, x, n_tokens, k, n_experts, offsets, sorted, units, hidden,
-                                  inter, swiglu_limit, precision, gated, gated_raw, st)))
+                                  inter, swiglu_limit, precision, lo_plane, gated, gated_raw, st)))
       return rc;
     if ((rc = mark(4))) return rc;
     if ((rc = launch_gemm_down(w_down, down_bias, gated, n_tokens * k, n_experts, offsets, sorted, units, hidden,

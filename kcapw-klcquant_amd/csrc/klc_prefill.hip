@@ -580,7 +580,8 @@ __device__ __forceinline__ void moe_gemm_body(
       }
       const int64_t idx = (int64_t)p * half + col0 + ch;  // half % 8 == 0: 16-byte aligned
       *reinterpret_cast<u32x4_t*>(out_split + idx) = u32x4_t{hi[0], hi[1], hi[2], hi[3]};
-      *reinterpret_cast<u32x4_t*>(out_split + out_plane + idx) = u32x4_t{lo[0], lo[1], lo[2], lo[3]};
+      if (out_plane != 0)  // 0: the down kernel reads the hi plane alone
+        *reinterpret_cast<u32x4_t*>(out_split + out_plane + idx) = u32x4_t{lo[0], lo[1], lo[2], lo[3]};
       if (out_raw) {
         reinterpret_cast<float4*>(out_raw + idx)[0] = make_float4(y[0], y[1], y[2], y[3]);
         reinterpret_cast<float4*>(out_raw + idx)[1] = make_float4(y[4], y[5], y[6], y[7]);
@@ -666,7 +667,7 @@ void run_gemm(int64_t n_pairs, int64_t n_exp, int row_wgs, hipStream_t stream, c
 
 int launch_gemm_gate_up(const void* const* w, const void* bias, const void* x, int64_t n_tok, int64_t k,
                         int64_t n_exp, const int32_t* offsets, const int32_t* pairs, const int32_t* units,
-                        int64_t hidden, int64_t inter, float limit, int precision, void* gated_split,
+                        int64_t hidden, int64_t inter, float limit, int precision, bool lo_plane, void* gated_split,
                         float* gated_raw, hipStream_t stream) {
   const int64_t n_pairs = n_tok * k;
   const int64_t rows = 2 * inter;
@@ -678,7 +679,7 @@ int launch_gemm_gate_up(const void* const* w, const void* bias, const void* x, i
              : wide  ? run_gemm<false, 1, kGemmCb, true>
                      : run_gemm<false, 1, kGemmCb, false>;
   run(n_pairs, n_exp, row_wgs, stream, reinterpret_cast<const uint8_t* const*>(w), static_cast<const uint16_t*>(bias),
-      static_cast<const uint16_t*>(x), 0, nullptr, static_cast<uint16_t*>(gated_split), n_pairs * inter, gated_raw,
+      static_cast<const uint16_t*>(x), 0, nullptr, static_cast<uint16_t*>(gated_split), lo_plane ? n_pairs * inter : 0, gated_raw,
       offsets, pairs, units + units_offset_gemm(n_pairs, n_exp), units + 2, (int)rows, groups, (int)k, limit,
       precision);
   return check_launch("moe_gemm_kernel<gate_up>");
@@ -722,7 +723,7 @@ extern "C" int klc_moe_gemm_gate_up(const void* const* w_gate_up, const void* bi
   const int rc = check_gemv_shapes(hidden, inter, n_tokens * k, n_experts);
   if (rc) return rc;
   return launch_gemm_gate_up(w_gate_up, bias, x, n_tokens, k, n_experts, offsets, sorted_pairs, units, hidden, inter,
-                             swiglu_limit, precision, gated_split, gated_raw, as_stream(stream));
+                             swiglu_limit, precision, true, gated_split, gated_raw, as_stream(stream));
 }
 
 extern "C" int klc_moe_gemm_down(const void* const* w_down, const void* bias, const void* gated_split, int64_t n_pairs,
