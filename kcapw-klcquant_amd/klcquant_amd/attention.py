@@ -20,7 +20,6 @@ StreamedAttention) and kv_cache_manager.py (KVCacheManager's methods, here
 from __future__ import annotations
 
 import ctypes
-import functools
 import math
 import struct
 import time
@@ -219,6 +218,9 @@ class _HostRecord:
         self.floats = self.words.view(np.float32)
         self.ptr = self._held.data_ptr()
 
+    def __reduce__(self):
+        return _HostRecord, ()  # a copy is a record of its own, with its own memory
+
     def wait(self, dev: torch.device, limit_s: float) -> None:
         """Spins until the device has written the tag; past ``limit_s`` it synchronises the current
         stream instead, which raises if the device failed."""
@@ -281,10 +283,6 @@ class StreamedAttention:
             torch.cuda.current_stream(device).synchronize()  # any stream may read it from here on
             self._inv_freq[key] = t
         return t
-
-    @functools.cached_property
-    def _step_fn(self):
-        return _native.load().klc_attn_step
 
     # A record the GPU has not written after this long is waited for by a
     # synchronisation of the stream.
@@ -354,7 +352,7 @@ class StreamedAttention:
             record = _HostRecord()
         words = record.words
         words[8] = 0
-        rc = self._step_fn(
+        rc = _native.load().klc_attn_step(
             _STEP.pack(hidden_ptr, ptr[0], ptr[4], ptr[1], ptr[5], ptr[2], ptr[6], ptr[3], ptr[7],
                        ptr[8] if len(ptr) == 9 else 0, inv_freq.data_ptr(), keys.data_ptr(), values.data_ptr(),
                        workspace.data_ptr(), out.data_ptr(), record.ptr, size, o_size, nh, nkv, d, ring["cap"], slot,

@@ -11,6 +11,7 @@ the softmax sum is taken in another order).
 
 from __future__ import annotations
 
+import copy
 import ctypes
 
 import numpy as np
@@ -327,6 +328,7 @@ def test_attention_step_and_general_path_agree(gpu):
             assert (attn._step(0, x, w, 3, DeviceKVCache(gpu, capacity=4), None) is None) == grad
             for pos in range(3):
                 out, diag = attn.forward(0, x, w, pos, cache)
+                attn = copy.deepcopy(attn)  # with its records and tables
             outs.append(out)
             diags.append(diag)
         assert outs[1].requires_grad and not outs[0].requires_grad
