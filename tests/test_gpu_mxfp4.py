@@ -86,6 +86,22 @@ def test_dequant_shapes_match_oracle(gpu, n_mat, out_dim, groups, dtype, kind):
         assert torch.equal(again.view(torch.uint8), got.view(torch.uint8))
 
 
+@pytest.mark.parametrize("dtype,kind", [(torch.bfloat16, "bf16"), (torch.float16, "f16"), (torch.float32, "f32")])
+@pytest.mark.parametrize("n_mat,out_dim,groups", [(4100, 1, 1), (1025, 7, 3), (333, 8, 4), (67, 64, 17), (33, 72, 45),
+                                                   (19, 128, 9), (40, 5, 20), (515, 65, 5)])
+def test_dequant_many_small_matrices_match_oracle(gpu, n_mat, out_dim, groups, dtype, kind):
+    """Odd numbers of parts (1, 3, 5) of odd numbers of matrices: a pair of workgroups covers parts of
+    two matrices, and the last workgroups have none."""
+    blocks, scales = synth.mxfp4_expert_tensors(n_mat, groups, n_mat, out_dim, groups * 32, 0, 255)
+    got = ops.mxfp4_dequant(torch.from_numpy(blocks).to(gpu), torch.from_numpy(scales).to(gpu), dtype)
+    g = bf16_bits(got) if kind == "bf16" else got.cpu().numpy()
+    same_bits_nan_aware(g, omx.dequantize_batch(blocks, scales, kind), kind)
+    if out_dim % 64 == 0:
+        packed = ops.mxfp4_pack(torch.from_numpy(blocks).to(gpu), torch.from_numpy(scales).to(gpu))
+        again = ops.mxfp4_dequant_packed(packed, out_dim, groups, dtype)
+        assert torch.equal(again.view(torch.uint8), got.view(torch.uint8))
+
+
 def test_dequant_large_call_equals_its_halves(gpu):
     """160 x 2888 x 90 groups to bfloat16 (3.4 GB) takes the large-call shape, 2 matrices the small
     one: the same bits, checkpoint and (2,880 rows) packed layout."""
