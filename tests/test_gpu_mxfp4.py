@@ -73,9 +73,9 @@ def test_dequant_seeded_matches_oracle(gpu, n_mat, out_dim, groups):
                                                    (64, 36, 125), (256, 64, 31), (1, 1029, 4093), (2, 72, 17),
                                                    (1, 136, 90), (3, 200, 33), (17, 2880, 9)])
 def test_dequant_shapes_match_oracle(gpu, n_mat, out_dim, groups, dtype, kind):
-    """The workgroup shapes of aligned rows (64 x 16, float32 384 x 4) and odd ones (384 x 4, and
-    1024 x 4 where that gives 2048 workgroups: the 33- and 1029-row calls) over partial parts and
-    column blocks, every scale byte: bit-exact.  (128 x 8 starts at 512 MB of input and output.)"""
+    """The workgroup shapes of aligned rows (64 x 16, float32 384 x 4) and odd ones (384 x 4, and 1024 x 4
+    from 192 rows where that gives 2048 workgroups: the 1029-row call) over partial parts and column
+    blocks, every scale byte: bit-exact.  (256 x 4 starts at 160 MB of input and output.)"""
     blocks, scales = synth.mxfp4_expert_tensors(out_dim, groups, n_mat, out_dim, groups * 32, 0, 255)
     got = ops.mxfp4_dequant(torch.from_numpy(blocks).to(gpu), torch.from_numpy(scales).to(gpu), dtype)
     g = bf16_bits(got) if kind == "bf16" else got.cpu().numpy()
@@ -119,6 +119,23 @@ def test_dequant_large_call_equals_its_halves(gpu):
             assert torch.equal(again, big)
         del big, part
         torch.cuda.empty_cache()
+
+
+@pytest.mark.parametrize("n_mat,rows,groups", [(20, 2888, 90), (8, 5120, 61), (40, 1984, 28), (300, 392, 21)])
+@pytest.mark.parametrize("dtype", [torch.bfloat16, torch.float16])
+def test_dequant_large_call_equals_single_matrices(gpu, n_mat, rows, groups, dtype):
+    """Calls past 160 MB of input and output take the 256 x 4 shape (here over partial column blocks and
+    parts), a matrix alone the 64 x 16 one: the same bits, checkpoint and packed layout, every scale byte."""
+    g = torch.Generator(device=gpu).manual_seed(rows)
+    blocks = torch.randint(0, 256, (n_mat, rows, groups, 16), dtype=torch.uint8, device=gpu, generator=g)
+    scales = torch.randint(0, 256, (n_mat, rows, groups), dtype=torch.uint8, device=gpu, generator=g)
+    assert blocks.numel() // 16 * 81 >= 160 << 20
+    big = ops.mxfp4_dequant(blocks, scales, dtype).view(torch.int16)
+    for i in range(0, n_mat, max(1, n_mat // 20)):
+        assert torch.equal(big[i], ops.mxfp4_dequant(blocks[i], scales[i], dtype).view(torch.int16))
+    if rows % 64 == 0:
+        packed = ops.mxfp4_pack(blocks, scales)
+        assert torch.equal(ops.mxfp4_dequant_packed(packed, rows, groups, dtype).view(torch.int16), big)
 
 
 def test_dequant_single_matrix_shape_and_errors(gpu):
