@@ -218,9 +218,10 @@ int64_t klc_moe_workspace_bytes(int64_t n_tokens, int64_t hidden, int64_t inter,
  * records the first before its launch and the other six after it. */
 #define KLC_LAYER_EVENTS 7
 /* Expert path of klc_moe_layer.  AUTO picks the grouped GEMM once the batch
- * gives experts 3 or more tokens on average (n_tokens * k >= 3 * n_experts
- * and at least 128, or >= 8 * n_experts),
- * the decode GEMVs below that.  GEMV and GEMM force that expert path.  FUSED
+ * gives experts enough tokens on average: with pairs = n_tokens * k, from
+ * pairs >= 8 * n_experts, and for pairs >= 128 from 3 * n_experts when pairs *
+ * hidden * inter >= 5.5e8 or 4.5 * n_experts when it is >= 2.5e8; the decode
+ * GEMVs below that.  GEMV and GEMM force that expert path.  FUSED
  * runs the whole layer as one launch: batches of at most 16 tokens (at most
  * 64 token-slot pairs, 256 experts, k <= 16), 8-byte aligned out/residual,
  * and a stream that is not capturing a graph; other calls fail with

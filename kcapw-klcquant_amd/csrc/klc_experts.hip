@@ -605,13 +605,30 @@ int resolve_layer_path(int path, int64_t n_tok, int64_t hidden, int64_t inter, i
   }
   // The GEMV stages 8 (gate_up) or 4 (down) pairs a pass, so an expert's
   // weights are read again every few pairs; the GEMM's 16-token units read
-  // them once, on half as many workgroups.  Layer, GEMV against GEMM: 64
-  // tokens of 128 experts (2 pairs each) 269 / 265 us, 100 (3.1) 307 / 292,
-  // 200 (6.3) 433 / 322; of 64 experts 32 (2) 141 / 147, 48 (3) 163 / 158; of
-  // 32 experts 16 (2) 80 / 90, 32 (4) 99 / 95; of 16 experts 16 (4) 63 / 65,
-  // 24 (6) 72 / 74.
+  // them once, on half as many workgroups, which small layers do not fill the
+  // chip with.  So below 8 pairs an expert the GEMM is taken for enough pairs
+  // times weights: more of both at 3 pairs an expert than at 4.5.  Layer,
+  // GEMV / GEMM in us, float32, uniform routing, hidden x inter:
+  //   2880 x 2880: 128 experts 96 tokens (3 pairs) 302 / 285, 200 (6.3) 433 /
+  //   322; 64 experts 48 (3) 163 / 158; 32 experts 32 (4) 102.6 / 98.1
+  //   2048 x 2048: 64 experts 48 (3) 99.1 / 97.6; 32 experts 32 (4) 62.9 /
+  //   63.3, 36 (4.5) 68.7 / 64.6
+  //   2048 x 1024: 128 experts 96 (3) 103.6 / 101.7; 64 experts 48 (3) 64.1 /
+  //   66.3, 64 (4) 66.3 / 67.0, 72 (4.5) 71.6 / 68.4; 32 experts 32 (4) 44.6 /
+  //   45.6, 40 (5) 49.8 / 46.6
+  //   1024 x 1024: 128 experts 96 (3) 67.8 / 69.4; 32 experts 56 (7) 40.1 /
+  //   41.3; 512 x 512: 64 experts 112 (7) 37.3 / 38.4, 32 experts 32 (4) 27.8
+  //   / 33.0
+  // Skewed routing and bfloat16 favour the GEMM more (128 experts, 2880 x
+  // 2880, 96 tokens at Zipf 1.1 303 / 261; bfloat16 302 / 275; 64 experts, 2048
+  // x 1024, 48 at Zipf 0.8 in bfloat16 65.7 / 65.8).  Fewer than 128 pairs: 16
+  // experts 16 tokens (4) 63 / 65, 24 (6) 72 / 74.
   const int64_t pairs = n_tok * k;
-  return pairs >= 8 * n_exp || (pairs >= 3 * n_exp && pairs >= 128) ? KLC_PATH_GEMM : KLC_PATH_GEMV;
+  const int64_t work = pairs * hidden * inter;
+  const bool gemm = pairs >= 8 * n_exp ||
+                    (pairs >= 128 && ((pairs >= 3 * n_exp && work >= 550000000) ||
+                                      (2 * pairs >= 9 * n_exp && work >= 250000000)));
+  return gemm ? KLC_PATH_GEMM : KLC_PATH_GEMV;
 }
 
 

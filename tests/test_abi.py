@@ -98,6 +98,24 @@ def test_route_entry_argument_errors():
     assert ei.value.status == nat.KLC_ERR_ARGUMENT and "workspace" in ei.value.message
 
 
+@pytest.mark.parametrize("n_tok,hidden,inter,n_exp,k,path", [
+    (96, 2880, 2880, 128, 4, nat.PATH_GEMM), (95, 2880, 2880, 128, 4, nat.PATH_GEMV),
+    (48, 2880, 2880, 64, 4, nat.PATH_GEMM), (47, 2880, 2880, 64, 4, nat.PATH_GEMV),
+    (32, 2880, 2880, 32, 4, nat.PATH_GEMM), (31, 2880, 2880, 32, 4, nat.PATH_GEMV),
+    # small layers: the GEMV is the faster one at these loads
+    (48, 2048, 1024, 64, 4, nat.PATH_GEMV), (65, 2048, 1024, 64, 4, nat.PATH_GEMV),
+    (66, 2048, 1024, 64, 4, nat.PATH_GEMM), (32, 2048, 1024, 32, 4, nat.PATH_GEMV),
+    (36, 2048, 1024, 32, 4, nat.PATH_GEMM), (96, 2048, 1024, 128, 4, nat.PATH_GEMM),
+    (32, 512, 512, 32, 4, nat.PATH_GEMV), (112, 512, 512, 64, 4, nat.PATH_GEMV),
+    (33, 256, 128, 32, 4, nat.PATH_GEMV), (100, 256, 128, 128, 4, nat.PATH_GEMV),
+    # 8 pairs an expert, whatever the size
+    (64, 512, 512, 32, 4, nat.PATH_GEMM), (63, 512, 512, 32, 4, nat.PATH_GEMV),
+    (32, 256, 128, 16, 4, nat.PATH_GEMM), (31, 256, 128, 16, 4, nat.PATH_GEMV)])
+def test_layer_path_lines(n_tok, hidden, inter, n_exp, k, path):
+    """KLC_PATH_AUTO at the lines between the decode GEMVs and the grouped GEMM."""
+    assert nat.call("klc_moe_layer_path", n_tok, hidden, inter, n_exp, k, nat.PATH_AUTO, None) == path
+
+
 def test_attention_workspace_never_shrinks_with_the_count():
     """A workspace made for a ring's capacity serves every shorter span, across the lines between
     the kernels' block sizes (256, 8,192 and 65,536 keys)."""
