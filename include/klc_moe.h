@@ -453,7 +453,9 @@ int klc_attn_decode(const void* q, const void* k_cache, const void* v_cache, con
  * (pinned host memory, or NULL): 9 words the device writes while the step
  * runs: float32 norms |q|, |k| before RoPE, |q|, |k| after it, |q after - q|,
  * |k after - k|, int32 counts of non-finite q and k values after it, then
- * `tag` (not 0; the caller clears that word first).  Biases and sinks may be
+ * the low 32 bits of `tag` (not 0; the caller clears that word first; the
+ * record's memory must outlive the step's work on the stream, also when the
+ * call fails).  Biases and sinks may be
  * NULL.  hidden_size and n_heads * head_dim multiples of 8, at most 4096;
  * hidden, weights, caches and workspace 16-byte aligned; other limits as
  * klc_attn_decode's. */

@@ -899,7 +899,7 @@ extern "C" int klc_attn_step(const klc_attn_step_args* args, void* stream) {
               (long long)a.workspace_bytes, (long long)need);
   StepRecord rec{};
   if (a.host_record != nullptr) {
-    KLC_REQUIRE(a.tag != 0, KLC_ERR_ARGUMENT, "klc_attn_step: tag 0 (the caller clears the tag word to 0)");
+    KLC_REQUIRE((uint32_t)a.tag != 0, KLC_ERR_ARGUMENT, "klc_attn_step: tag 0 (the caller clears the tag word to 0)");
     hipPointerAttribute_t attr;
     const hipError_t e = hipPointerGetAttributes(&attr, a.host_record);
     KLC_REQUIRE(e == hipSuccess && attr.devicePointer != nullptr, KLC_ERR_ARGUMENT,

@@ -210,22 +210,28 @@ class DeviceKVCache:
 
 
 class _HostRecord:
-    """klc_attn_step's record in pinned host memory: 6 norms, 2 counts, tag."""
+    """klc_attn_step's record in pinned host memory: 6 norms, 2 counts, and the call's tag, another one
+    for every call on the record."""
 
     def __init__(self) -> None:
         self._held = torch.zeros(16, dtype=torch.int32, pin_memory=True)
         self.words = self._held.numpy()
         self.floats = self.words.view(np.float32)
         self.ptr = self._held.data_ptr()
+        self.tag = 0
 
     def __reduce__(self):
         return _HostRecord, ()  # a copy is a record of its own, with its own memory
 
+    def next_tag(self) -> int:
+        self.tag = self.tag % 0x7FFFFFFF + 1
+        return self.tag
+
     def wait(self, dev: torch.device, limit_s: float) -> None:
         """Spins until the device has written the tag; past ``limit_s`` it synchronises the current
         stream instead, which raises if the device failed."""
-        words, spins, deadline = self.words, 0, None
-        while words[8] != 1:
+        words, tag, spins, deadline = self.words, self.tag, 0, None
+        while words[8] != tag:
             spins += 1
             if spins & 1023 == 0:
                 now = time.perf_counter()
@@ -233,11 +239,20 @@ class _HostRecord:
                     deadline = now + limit_s
                 elif now > deadline:
                     torch.cuda.current_stream(dev).synchronize()
-                    if words[8] != 1:
+                    if words[8] != tag:
                         raise RuntimeError("the attention step finished without its host record")
                     return
 
+    def settle(self, dev: torch.device) -> None:
+        """After a call that did not end in :meth:`wait`: the current stream may still hold the write to
+        this record, so its memory stays referenced until the stream is done (for good if that cannot be
+        waited for)."""
+        _UNSETTLED.append(self)
+        torch.cuda.current_stream(dev).synchronize()
+        _UNSETTLED.remove(self)
 
+
+_UNSETTLED: list[_HostRecord] = []
 _TENSORS = (torch.Tensor, torch.nn.Parameter)
 
 
@@ -352,16 +367,20 @@ class StreamedAttention:
             record = _HostRecord()
         words = record.words
         words[8] = 0
-        rc = _native.load().klc_attn_step(
-            _STEP.pack(hidden_ptr, ptr[0], ptr[4], ptr[1], ptr[5], ptr[2], ptr[6], ptr[3], ptr[7],
-                       ptr[8] if len(ptr) == 9 else 0, inv_freq.data_ptr(), keys.data_ptr(), values.data_ptr(),
-                       workspace.data_ptr(), out.data_ptr(), record.ptr, size, o_size, nh, nkv, d, ring["cap"], slot,
-                       (total - count) % ring["cap"], count, kv_cache.kv_code, need, 1, float(position), scaling),
-            torch._C._cuda_getCurrentRawStream(index))
-        if rc < 0:
-            raise _native.KlcError("klc_attn_step", int(rc), _native.last_error())
-        ring["total"] = total
-        record.wait(dev, self._RECORD_WAIT_S)
+        args = _STEP.pack(hidden_ptr, ptr[0], ptr[4], ptr[1], ptr[5], ptr[2], ptr[6], ptr[3], ptr[7],
+                          ptr[8] if len(ptr) == 9 else 0, inv_freq.data_ptr(), keys.data_ptr(), values.data_ptr(),
+                          workspace.data_ptr(), out.data_ptr(), record.ptr, size, o_size, nh, nkv, d, ring["cap"],
+                          slot, (total - count) % ring["cap"], count, kv_cache.kv_code, need, record.next_tag(),
+                          float(position), scaling)
+        try:
+            rc = _native.load().klc_attn_step(args, torch._C._cuda_getCurrentRawStream(index))
+            if rc < 0:
+                raise _native.KlcError("klc_attn_step", int(rc), _native.last_error())
+            ring["total"] = total
+            record.wait(dev, self._RECORD_WAIT_S)
+        except BaseException:  # Ctrl-C during the wait too
+            record.settle(dev)
+            raise
         norms = record.floats[:6].tolist()
         diagnostics = {
             "rope_position": int(position),

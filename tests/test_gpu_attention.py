@@ -18,7 +18,7 @@ import numpy as np
 import pytest
 import torch
 
-from klcquant_amd import _native
+from klcquant_amd import _native, attention
 from klcquant_amd.attention import AttentionConfig, DeviceKVCache, StreamedAttention, rope_cos_sin
 from oracle import attention as oat
 from oracle.numerics import bf16_to_f32, f32_to_bf16
@@ -338,6 +338,37 @@ def test_attention_step_and_general_path_agree(gpu):
             assert diags[0][name] == diags[1][name] or np.isclose(diags[0][name], diags[1][name], rtol=1e-4, equal_nan=True)
         if poison:
             assert diags[0]["q_post_rope_nonfinite_count"] > 0
+
+
+def test_attention_step_interrupted_wait_keeps_the_record(gpu, monkeypatch):
+    """An exception in the wait leaves only after the stream is done with the record (whose memory could
+    otherwise be another tensor's by then), and the next step, with a tag of its own, reads its own values."""
+    nh, nkv, d, h = 64, 8, 64, 2880
+    g = torch.Generator(device=gpu).manual_seed(9)
+    pre = "model.layers.0.self_attn"
+    t = step_tensors(gpu, g, nh, nkv, d, h, h, pre)
+    attn, cache = StreamedAttention(AttentionConfig(**CFG)), DeviceKVCache(gpu, capacity=8)
+    x = torch.randn(h, generator=g, device=gpu).to(torch.bfloat16)
+    busy = torch.randn(4096, 4096, generator=g, device=gpu)
+    seen = []
+
+    def interrupted(record, dev, limit_s):
+        seen.append((record, int(record.words[8])))
+        raise KeyboardInterrupt
+
+    with monkeypatch.context() as m:
+        m.setattr(attention._HostRecord, "wait", interrupted)
+        for _ in range(40):
+            busy = busy @ busy * 1e-4  # a queue ahead of the step
+        with pytest.raises(KeyboardInterrupt):
+            attn.forward(0, x, t, 0, cache)
+    (record, before), = seen
+    assert before == 0 and record.words[8] == record.tag == 1 and attention._UNSETTLED == []
+    attn._records.append(record)
+    _, diag = attn.forward(0, 2 * x, t, 1, cache)
+    assert record.words[8] == record.tag == 2
+    q = torch.nn.functional.linear(2 * x, t[f"{pre}.q_proj.weight"], t[f"{pre}.q_proj.bias"])
+    assert np.isclose(diag["q_pre_rope_norm"], q.float().norm().item(), rtol=1e-3)
 
 
 def test_attention_rejects_bad_shapes(gpu):
