@@ -473,6 +473,9 @@ typedef struct klc_attn_step_args {
 } klc_attn_step_args;
 int64_t klc_attn_step_workspace_bytes(int64_t n_heads, int64_t n_kv, int64_t head_dim, int64_t count);
 int klc_attn_step(const klc_attn_step_args* args, void* stream);
+/* Waits on the host, reading the record's tag word, until it is `tag` (1) or
+ * limit_us microseconds have passed (0). */
+int klc_attn_step_wait(const void* host_record, int64_t tag, int64_t limit_us);
 
 /* ---- Synthetic inputs -------------------------------------------------------
  * Counter-based SplitMix64 stream, identical to klcquant_amd/synth.py:

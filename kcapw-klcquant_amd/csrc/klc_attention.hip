@@ -28,6 +28,8 @@
 // query head (38 us -> 20).
 #include <math.h>
 
+#include <chrono>
+
 #include "klc_common.h"
 
 namespace klc {
@@ -932,4 +934,17 @@ extern "C" int klc_attn_step(const klc_attn_step_args* args, void* stream) {
                                    launch_out<5>, launch_out<6>, launch_out<7>, launch_out<8>};
   return kOut[(nh * d / 8 + kWave - 1) / kWave - 1](in(a.o_weight), in(a.o_bias), ctx, static_cast<uint16_t*>(a.out),
                                                     (int)a.out_size, (int)(nh * d), st);
+}
+
+extern "C" int klc_attn_step_wait(const void* host_record, int64_t tag, int64_t limit_us) {
+  KLC_REQUIRE(host_record != nullptr && (uint32_t)tag != 0, KLC_ERR_ARGUMENT, "klc_attn_step_wait: no record or tag 0");
+  const uint32_t* word = static_cast<const uint32_t*>(host_record) + 8;
+  const auto begin = std::chrono::steady_clock::now();
+  for (;;) {
+    for (int i = 0; i < 256; ++i) {
+      if (__atomic_load_n(word, __ATOMIC_ACQUIRE) == (uint32_t)tag) return 1;
+      __builtin_ia32_pause();
+    }
+    if (std::chrono::steady_clock::now() - begin > std::chrono::microseconds(limit_us)) return 0;
+  }
 }

@@ -88,6 +88,7 @@ SIGNATURES: dict[str, tuple] = {
     "klc_attn_decode": (_I32, [_P, _P, _P, _P, _I64, _I64, _I64, _I64, _I64, _I64, _I32, _P, _I64, _P, _P]),
     "klc_attn_step_workspace_bytes": (_I64, [_I64, _I64, _I64, _I64]),
     "klc_attn_step": (_I32, [ctypes.c_char_p, _P]),
+    "klc_attn_step_wait": (_I32, [_P, _I64, _I64]),
     "klc_synth_fill": (_I32, [_P, _I64, _U64, _I32, _I32, _I32, _P]),
 }
 

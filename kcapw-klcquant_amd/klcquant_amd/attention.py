@@ -213,6 +213,8 @@ class _HostRecord:
     """klc_attn_step's record in pinned host memory: 6 norms, 2 counts, and the call's tag, another one
     for every call on the record."""
 
+    _SLICE_US = 20_000  # of one wait in the library
+
     def __init__(self) -> None:
         self._held = torch.zeros(16, dtype=torch.int32, pin_memory=True)
         self.words = self._held.numpy()
@@ -228,20 +230,19 @@ class _HostRecord:
         return self.tag
 
     def wait(self, dev: torch.device, limit_s: float) -> None:
-        """Spins until the device has written the tag; past ``limit_s`` it synchronises the current
-        stream instead, which raises if the device failed."""
-        words, tag, spins, deadline = self.words, self.tag, 0, None
-        while words[8] != tag:
-            spins += 1
-            if spins & 1023 == 0:
-                now = time.perf_counter()
-                if deadline is None:
-                    deadline = now + limit_s
-                elif now > deadline:
-                    torch.cuda.current_stream(dev).synchronize()
-                    if words[8] != tag:
-                        raise RuntimeError("the attention step finished without its host record")
-                    return
+        """Waits until the device has written the tag, in the library (the interpreter lock is free
+        meanwhile) and in slices, so that signals are handled; past ``limit_s`` it synchronises the
+        current stream instead, which raises if the device failed."""
+        arrived = _native.load().klc_attn_step_wait
+        if arrived(self.ptr, self.tag, self._SLICE_US) == 1:
+            return
+        deadline = time.perf_counter() + limit_s
+        while arrived(self.ptr, self.tag, self._SLICE_US) != 1:
+            if time.perf_counter() > deadline:
+                torch.cuda.current_stream(dev).synchronize()
+                if self.words[8] != self.tag:
+                    raise RuntimeError("the attention step finished without its host record")
+                return
 
     def settle(self, dev: torch.device) -> None:
         """After a call that did not end in :meth:`wait`: the current stream may still hold the write to

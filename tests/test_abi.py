@@ -5,8 +5,11 @@ from __future__ import annotations
 
 import ctypes
 import re
+import sys
+import threading
 from pathlib import Path
 
+import numpy as np
 import pytest
 
 from klcquant_amd import _native as nat
@@ -114,6 +117,33 @@ def test_route_entry_argument_errors():
 def test_layer_path_lines(n_tok, hidden, inter, n_exp, k, path):
     """KLC_PATH_AUTO at the lines between the decode GEMVs and the grouped GEMM."""
     assert nat.call("klc_moe_layer_path", n_tok, hidden, inter, n_exp, k, nat.PATH_AUTO, None) == path
+
+
+def test_attention_step_wait_leaves_the_interpreter_to_other_threads():
+    """The wait for a step's record ends by what another Python thread does, with thread switches of the
+    interpreter put off past the wait's limit; without the tag it ends at the limit."""
+    record = np.zeros(16, dtype=np.int32)
+    nat.load()
+    started = threading.Event()
+
+    def writer():
+        started.wait()
+        record[8] = 7
+
+    thread = threading.Thread(target=writer)
+    interval = sys.getswitchinterval()
+    thread.start()
+    try:
+        sys.setswitchinterval(60.0)
+        started.set()
+        assert nat.call("klc_attn_step_wait", record.ctypes.data, 7, 20_000_000) == 1
+    finally:
+        sys.setswitchinterval(interval)
+        thread.join()
+    assert nat.call("klc_attn_step_wait", record.ctypes.data, 8, 1000) == 0
+    for args in ((None, 7, 0), (record.ctypes.data, 0, 0), (record.ctypes.data, 1 << 32, 0)):
+        with pytest.raises(nat.KlcError):
+            nat.call("klc_attn_step_wait", *args)
 
 
 def test_attention_workspace_never_shrinks_with_the_count():

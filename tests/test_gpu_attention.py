@@ -371,6 +371,23 @@ def test_attention_step_interrupted_wait_keeps_the_record(gpu, monkeypatch):
     assert np.isclose(diag["q_pre_rope_norm"], q.float().norm().item(), rtol=1e-3)
 
 
+def test_attention_step_wait_past_its_limit(gpu, monkeypatch):
+    """Behind a queue longer than the wait's limit the step synchronises its stream: the same results."""
+    nh, nkv, d, h = 8, 2, 64, 256
+    g = torch.Generator(device=gpu).manual_seed(10)
+    t = step_tensors(gpu, g, nh, nkv, d, h, h, "model.layers.0.self_attn")
+    cfg = AttentionConfig(hidden_size=h, num_heads=nh, num_kv_heads=nkv, head_dim=d)
+    x = torch.randn(h, generator=g, device=gpu).to(torch.bfloat16)
+    want = StreamedAttention(cfg).forward(0, x, t, 5, DeviceKVCache(gpu, capacity=8))
+    busy = torch.randn(4096, 4096, generator=g, device=gpu)
+    monkeypatch.setattr(StreamedAttention, "_RECORD_WAIT_S", 0.0)
+    monkeypatch.setattr(attention._HostRecord, "_SLICE_US", 1)
+    for _ in range(40):
+        busy = busy @ busy * 1e-4
+    out, diag = StreamedAttention(cfg).forward(0, x, t, 5, DeviceKVCache(gpu, capacity=8))
+    assert torch.equal(out, want[0]) and diag == want[1]
+
+
 def test_attention_rejects_bad_shapes(gpu):
     x = torch.zeros(4096, dtype=torch.bfloat16, device=gpu)
     ws = torch.zeros(1 << 16, dtype=torch.uint8, device=gpu)
