@@ -13,8 +13,9 @@ StreamedAttention) and kv_cache_manager.py (KVCacheManager's methods, here
   epilogue, scores / softmax with sinks / value sum over the window, the
   output projection; the diagnostics come back through a pinned host record
   that the device writes while the step runs.  What that call does not take
-  (autograd, autocast, tensor subclasses, other layouts) runs as torch's
-  ``F.linear`` with klc_rope_append and klc_attn_decode between.
+  (autograd, autocast, tensor subclasses, other layouts, caches that choose
+  their own spans) runs as torch's ``F.linear`` with klc_rope_append and
+  klc_attn_decode between.
 """
 
 from __future__ import annotations
@@ -313,7 +314,7 @@ class StreamedAttention:
         size = hidden.shape[-1] if hidden.dim() else 0
         q, kv = nh * d, nkv * d
         if (type(hidden) is not torch.Tensor or hidden.dtype is not torch.bfloat16 or dev.type != "cuda"
-                or not isinstance(kv_cache, DeviceKVCache)
+                or not isinstance(kv_cache, DeviceKVCache) or type(kv_cache)._span is not DeviceKVCache._span
                 or size == 0 or size % 8 or size > 4096 or hidden.numel() != size or not hidden.is_contiguous()
                 or d % 8 or d > 128 or q > 4096 or nh % nkv or nh // nkv > 16 or _intercepted()):
             return None

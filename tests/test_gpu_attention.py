@@ -388,6 +388,25 @@ def test_attention_step_wait_past_its_limit(gpu, monkeypatch):
     assert torch.equal(out, want[0]) and diag == want[1]
 
 
+def test_attention_step_keeps_a_caches_own_span(gpu):
+    """A cache class that chooses the keys itself (here the last two) is asked for them."""
+    class LastTwo(DeviceKVCache):
+        @staticmethod
+        def _span(r, window):
+            return DeviceKVCache._span(r, min(window or 2, 2))
+
+    nh, nkv, d, h = 8, 2, 64, 256
+    g = torch.Generator(device=gpu).manual_seed(11)
+    t = step_tensors(gpu, g, nh, nkv, d, h, h, "model.layers.0.self_attn")
+    attn = StreamedAttention(AttentionConfig(hidden_size=h, num_heads=nh, num_kv_heads=nkv, head_dim=d))
+    xs = torch.randn(6, h, generator=g, device=gpu).to(torch.bfloat16)
+    own, windowed = LastTwo(gpu, capacity=16), DeviceKVCache(gpu, capacity=16)
+    for pos in range(6):
+        got, _ = attn.forward(0, xs[pos], t, pos, own)
+        want, _ = attn.forward(0, xs[pos], t, pos, windowed, sliding_window=2)
+        assert torch.allclose(got.float(), want.float(), rtol=2e-2, atol=1e-2)
+
+
 def test_attention_rejects_bad_shapes(gpu):
     x = torch.zeros(4096, dtype=torch.bfloat16, device=gpu)
     ws = torch.zeros(1 << 16, dtype=torch.uint8, device=gpu)
