@@ -714,7 +714,8 @@ AttnPlan attn_plan(int64_t count) {
   // 64 keys a score workgroup keep the chip busy on shorter contexts; larger
   // blocks leave fewer statistics for every value workgroup to read.  Core at
   // 12,000 keys with 64 / 128 / 256: 25.8 / 24.2 / 26.4 us, 16,384 30.6 /
-  // 27.6 / 27.5, 32,768 48.6 / 42.7 / 42.9.
+  // 27.6 / 27.5, 32,768 48.6 / 42.7 / 42.9, 65,537 109 / 85.1 / 76.8, 131,072
+  // 248 / 179 / 143, 262,144 719 / 480 / 350.
   a.score_keys = count <= 8192 ? 64 : count <= 65536 ? 128 : 256;
   a.nblk = (count + a.score_keys - 1) / a.score_keys;
   a.split_keys = count <= 8192 ? 128 : kPvKeys;  // 16,384 keys in splits of 128: 31.3 us against 27.6

@@ -13,6 +13,7 @@ from __future__ import annotations
 
 import copy
 import ctypes
+import threading
 
 import numpy as np
 import pytest
@@ -230,6 +231,14 @@ def test_split_decode_matches_oracle(gpu, nh, nkv, d, count, kv):
     assert np.all(np.abs(got - ref) <= context_tolerance(ref, kv)), np.abs(got - ref).max()
 
 
+@pytest.mark.parametrize("nh,nkv,d,count,kv", [
+    (8, 1, 64, 65537, "fp16"), (2, 1, 128, 66001, "bf16"), (16, 1, 128, 65800, "fp16"), (3, 1, 64, 131073, "bf16"),
+    (8, 1, 64, 65536, "fp16")])
+def test_long_split_decode_matches_oracle(gpu, nh, nkv, d, count, kv):
+    """Score blocks of 256 keys (past 65,536 keys), more of them than a value workgroup holds statistics of."""
+    test_split_decode_matches_oracle(gpu, nh, nkv, d, count, kv)
+
+
 def test_split_decode_infinite_scores(gpu):
     """A score block that is -inf throughout weighs nothing; a NaN key makes its KV head's queries NaN."""
     nh, nkv, d, count = 16, 2, 64, 600
@@ -405,6 +414,131 @@ def test_attention_step_keeps_a_caches_own_span(gpu):
         got, _ = attn.forward(0, xs[pos], t, pos, own)
         want, _ = attn.forward(0, xs[pos], t, pos, windowed, sliding_window=2)
         assert torch.allclose(got.float(), want.float(), rtol=2e-2, atol=1e-2)
+
+
+def small_step(gpu, seed, capacity=8, kv="fp16"):
+    """A small layer: (attention, hidden, tensors, a fresh cache)."""
+    nh, nkv, d, h = 8, 2, 64, 256
+    g = torch.Generator(device=gpu).manual_seed(seed)
+    t = step_tensors(gpu, g, nh, nkv, d, h, h, "model.layers.0.self_attn")
+    attn = StreamedAttention(AttentionConfig(hidden_size=h, num_heads=nh, num_kv_heads=nkv, head_dim=d))
+    return attn, torch.randn(h, generator=g, device=gpu).to(torch.bfloat16), t, DeviceKVCache(gpu, capacity=capacity,
+                                                                                            precision=kv)
+
+
+def test_attention_step_leaves_watched_calls_to_torch(gpu):
+    """Under anything that watches or replaces torch calls the one-call step declines, touching neither the
+    cache nor the stream (a capture holds nothing of it)."""
+    from torch.autograd import forward_ad
+    from torch.overrides import TorchFunctionMode
+    from torch.utils._python_dispatch import TorchDispatchMode
+
+    class Functions(TorchFunctionMode):
+        def __torch_function__(self, func, types, args=(), kwargs=None):
+            return func(*args, **(kwargs or {}))
+
+    class Dispatch(TorchDispatchMode):
+        def __torch_dispatch__(self, func, types, args=(), kwargs=None):
+            return func(*args, **(kwargs or {}))
+
+    attn, x, t, cache = small_step(gpu, 12)
+    declined = []
+
+    def step(y=None):
+        declined.append(attn._step(0, x, t, 0, cache, None) is None)
+        return None if y is None else y + 1
+
+    with torch.autocast("cuda", dtype=torch.bfloat16):
+        step()
+    with Functions():
+        step()
+    with Dispatch():
+        step()
+    with forward_ad.dual_level():
+        step()
+    torch.func.vmap(step)(torch.zeros(2, device=gpu))
+    torch.jit.trace(step, (torch.zeros(2, device=gpu),), check_trace=False)
+    y = torch.zeros(4, device=gpu)
+    graph = torch.cuda.CUDAGraph()
+    with torch.cuda.graph(graph):
+        z = step(y)
+    for n in range(3):
+        y.fill_(n)
+        graph.replay()
+        torch.cuda.synchronize()
+        assert z.tolist() == [n + 1.0] * 4
+    assert len(declined) >= 7 and all(declined) and not cache.layers
+    assert attn._step(0, x, t, 0, cache, None) is not None
+
+
+def test_attention_step_leaves_other_tensors_to_torch(gpu):
+    """Weights and inputs that the one call does not take as they lie give the general path's results:
+    the same values in another layout, type or class."""
+    class Sub(torch.Tensor):
+        pass
+
+    pre = "model.layers.0.self_attn"
+    attn, x, t, cache = small_step(gpu, 13)
+    want, _ = attn.forward(0, x, t, 7, cache)
+    strided = torch.empty(512, device=gpu, dtype=torch.bfloat16)[::2]
+    strided.copy_(x)
+    shifted_x = torch.empty(257, device=gpu, dtype=torch.bfloat16)[1:]
+    shifted_x.copy_(x)
+    q = t[f"{pre}.q_proj.weight"]
+    shifted = torch.empty(q.numel() + 1, device=gpu, dtype=torch.bfloat16)[1:].view(q.shape)
+    shifted.copy_(q)
+    for hidden, change in (
+            (strided, {}), (shifted_x, {}), (x.as_subclass(Sub), {}),
+            (x, {"q_proj.weight": shifted}), (x, {"q_proj.weight": q.t().contiguous().t()}),
+            (x, {"k_proj.weight": t[f"{pre}.k_proj.weight"].as_subclass(Sub)}),
+            (x, {"sinks": t[f"{pre}.sinks"].float()}),
+            (x, {"o_proj.weight": torch.nn.Parameter(t[f"{pre}.o_proj.weight"])})):
+        tensors = t | {f"{pre}.{n}": v for n, v in change.items()}
+        assert attn._step(0, hidden, tensors, 7, DeviceKVCache(gpu, capacity=8), None) is None, change.keys()
+        out, _ = attn.forward(0, hidden, tensors, 7, DeviceKVCache(gpu, capacity=8))
+        assert torch.allclose(out.float().detach(), want.float(), rtol=2e-2, atol=1e-2)
+    with torch.no_grad():  # nothing for autograd to see
+        p = t | {n: torch.nn.Parameter(v) for n, v in t.items()}
+        assert torch.equal(attn._step(0, x, p, 7, DeviceKVCache(gpu, capacity=8), None)[0], want)
+    # biases and sinks are read two bytes at a time, so they may lie anywhere; no bias tensor: the general path
+    def odd(v):
+        w = torch.empty(v.numel() + 1, device=gpu, dtype=torch.bfloat16)[1:]
+        w.copy_(v)
+        return w
+
+    moved = {n: odd(v) if v.dim() == 1 else v for n, v in t.items()}
+    assert torch.equal(attn._step(0, x, moved, 7, DeviceKVCache(gpu, capacity=8), None)[0], want)
+    out, _ = attn.forward(0, x, t | {f"{pre}.q_proj.bias": None}, 7, DeviceKVCache(gpu, capacity=8))
+    zero = torch.zeros_like(t[f"{pre}.q_proj.bias"])
+    ref, _ = attn.forward(0, x, t | {f"{pre}.q_proj.bias": zero}, 7, DeviceKVCache(gpu, capacity=8))
+    assert torch.allclose(out.float(), ref.float(), rtol=2e-2, atol=1e-2)
+
+
+def test_attention_step_on_streams_and_threads(gpu):
+    """Two threads with a stream and a cache each, on one StreamedAttention, give a single thread's bits."""
+    attn, _, t, _ = small_step(gpu, 14)
+    g = torch.Generator(device=gpu).manual_seed(15)
+    xs = torch.randn(2, 300, 256, generator=g, device=gpu).to(torch.bfloat16)
+    torch.cuda.synchronize()
+
+    def run(i, results):
+        with torch.cuda.stream(torch.cuda.Stream(gpu)):
+            cache = DeviceKVCache(gpu, capacity=512)
+            results[i] = [attn.forward(0, xs[i, pos], t, pos, cache) for pos in range(300)]
+            torch.cuda.current_stream(gpu).synchronize()
+
+    alone, together = {}, {}
+    for i in range(2):
+        run(i, alone)
+    threads = [threading.Thread(target=run, args=(i, together)) for i in range(2)]
+    for th in threads:
+        th.start()
+    for th in threads:
+        th.join()
+    for i in range(2):
+        for (a, da), (b, db) in zip(alone[i], together[i]):
+            assert torch.equal(a, b) and da == db
+    assert len(attn._records) <= 16
 
 
 def test_attention_rejects_bad_shapes(gpu):
