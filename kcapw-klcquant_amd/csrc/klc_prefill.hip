@@ -1,10 +1,10 @@
 // Prefill path: expert-grouped GEMM on MFMA (gfx950).
 //
-// For batches that give experts many tokens, each expert's weights are read
-// once per 64-token unit and multiplied into all of the unit's tokens:
-// a workgroup owns one GEMM unit (up to 64 tokens of one expert, from the
-// dispatch) and 256 output rows (4 waves, each one 64-row packed tile, i.e.
-// 4 row blocks of 16).  Per 128-deep k step every wave decodes its A chunks
+// For batches that give experts several tokens, each expert's weights are
+// read once per unit and multiplied into all of the unit's tokens: a workgroup
+// owns one GEMM unit (up to 64 tokens of one expert, from the dispatch; at
+// small mean loads up to 16 or 32, found from the expert offsets) and 256
+// output rows (4 waves, each one 64-row packed tile, i.e. 4 row blocks of 16).  Per 128-deep k step every wave decodes its A chunks
 // (MXFP4 -> bfloat16 with v_cvt_scalef32_pk_bf16_fp4, exact) and multiplies
 // them with v_mfma_f32_16x16x32_bf16 into each 16-token column block of B.
 //
@@ -229,8 +229,8 @@ __device__ __forceinline__ void moe_gemm_body(
   // In the narrow kernels an expert of one unit streams its weights past the
   // caches (B = 64 layer 302 -> 265 us, 300 tokens 352 -> 329, of 128
   // experts), while the units of a larger one find each other's lines there.
-  // The 64-token kernel gains nothing at its loads (777 tokens of 32 experts
-  // 288 -> 295 us, 2000 of 128 716 -> 728 with the second copy of its loops).
+  // The 64-token kernel loses at its loads (777 tokens of 32 experts 288 ->
+  // 295 us, 2000 of 128 716 -> 728 with the second copy of its loops).
   const bool only_unit = ne <= kTok;
   const int ncb = (nt + 15) >> 4;
   const int tid = threadIdx.x;
@@ -616,15 +616,23 @@ __device__ __forceinline__ void moe_gemm_body(
 #ifndef KLC_GEMM_WAVES_PER_EU
 #define KLC_GEMM_WAVES_PER_EU 2
 #endif
-// Waves per SIMD: two for the 64-token kernels (their accumulators fill the
-// registers), more for the narrow ones.
-template <int kCb>
+// Waves per SIMD to compile for, one from each workgroup of a CU: two for the
+// 64-token kernels (their accumulators fill the registers), as many as the LDS
+// holds workgroups for the narrow ones, which take 109 to 124 VGPRs, so that
+// their registers never hold fewer.
+template <bool kDown, int kPl, int kCb>
 __host__ __device__ constexpr int gemm_waves_per_eu() {
-  return kCb == 1 ? 4 : kCb == 2 ? 3 : KLC_GEMM_WAVES_PER_EU;
+  return kCb == kGemmCb ? KLC_GEMM_WAVES_PER_EU : 160 * 1024 / gemm_lds_bytes<kDown, kPl, kCb>();
 }
+static_assert(gemm_waves_per_eu<false, 1, 1>() == 4 && gemm_waves_per_eu<true, 1, 1>() == 4 &&
+                  gemm_waves_per_eu<true, 2, 1>() == 3,
+              "16-token units: gate_up and down; down with two planes");
+static_assert(gemm_waves_per_eu<false, 1, 2>() == 3 && gemm_waves_per_eu<true, 1, 2>() == 4 &&
+                  gemm_waves_per_eu<true, 2, 2>() == 2,
+              "32-token units");
 // The kernels: planes below 2 GiB (every layer call) and past it.
 template <bool kDown, int kPl, int kCb, bool kWide>
-__global__ __launch_bounds__(kGemmThreads) __attribute__((amdgpu_waves_per_eu(gemm_waves_per_eu<kCb>()))) void moe_gemm_kernel(
+__global__ __launch_bounds__(kGemmThreads) __attribute__((amdgpu_waves_per_eu(gemm_waves_per_eu<kDown, kPl, kCb>()))) void moe_gemm_kernel(
     const uint8_t* const* __restrict__ wptr, const uint16_t* __restrict__ bias, const uint16_t* __restrict__ act,
     int64_t act_plane, float* __restrict__ out, uint16_t* __restrict__ out_split, int64_t out_plane,
     float* __restrict__ out_raw, const int32_t* __restrict__ offsets, const int32_t* __restrict__ pairs,
@@ -636,13 +644,20 @@ __global__ __launch_bounds__(kGemmThreads) __attribute__((amdgpu_waves_per_eu(ge
 
 // Tokens per unit (in 16-token column blocks) by the call's mean pairs per
 // expert.  Below ~22 pairs an expert's weights are read for few tokens and the
-// layer is a weight stream: 16- and 32-token units leave registers and LDS for
-// 4 and 3 waves per SIMD instead of 2.  Layer times of 128 experts, float32
-// (16 / 32 / 64 tokens per unit): 100 tokens (3.1 pairs) 292 / 299 / 315 us,
-// 200 (6.3) 322 / 321 / 340, 300 (9.4) 345 / 330 / 355, 450 (14) 398 / 354 /
-// 386, 700 (22) 501 / 426 / 435, 1000 (31) 620 / 500 / 478; 32 experts, 200
-// tokens (25) 174 / 151 / 150.  Skewed loads split their hot experts over
-// more units: 300 tokens at Zipf 1.1 372 / 372 / 403.
+// layer is a weight stream: smaller units put more and smaller workgroups on a
+// CU (3 or 4, but 2 of the 32-token down with two planes) and let it stream
+// the weights.  The two gains are measured apart, 128 experts, 300 tokens
+// (9.4 pairs), float32, weights cached / streamed: 64-token units 367 / 357 us,
+// 32-token 352 / 329, 16-token 371 / 345; 100 tokens (3.1) 341 / 314, 327 /
+// 296, 328 / 291.  Layer times of 128 experts, float32 (16 / 32 / 64 tokens
+// per unit, the narrow ones streaming): 100 tokens 291 / 296 / 341 us, 200
+// (6.3 pairs) 324 / 318 / 361, 300 345 / 329 / 368, 450 (14) 398 / 355 / 386,
+// 700 (22) 500 / 424 / 435, 1000 (31) 620 / 500 / 478; 32 experts, 200 tokens
+// (25) 174 / 151 / 150.  The lines hold with skew, in bfloat16 and for smaller
+// layers: 300 tokens at Zipf 1.1 in bfloat16 358 / 344 / 377, 730 (22.8) 495 /
+// 420 / 435; 32 experts of 2048 x 1024, 180 tokens (22.5) 73.1 / 64.1 / 69.9,
+// at Zipf 1.1 72.5 / 68.4 / 82.4; 128 of 1536 x 2496, 730 tokens 268 / 218 /
+// 237.
 int gemm_column_blocks(int64_t n_pairs, int64_t n_exp, bool wide) {
   if (wide) return kGemmCb;
   if (n_pairs <= 5 * n_exp) return 1;
