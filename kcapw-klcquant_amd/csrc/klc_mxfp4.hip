@@ -5,14 +5,16 @@
 // output row is one input column of the checkpoint, so workgroups write runs
 // of every output row they touch, of a length that follows the call's size,
 // and there are enough of them for the chip however few matrices it has.
-// Measured (buffer sets in turn, nothing left in the caches) against one
-// workgroup per 64 output columns and all groups (and 768 columns x 4 groups
-// for bfloat16 of 64-row multiples): 1 x 5760 x 90 groups to float16 25.4 ->
-// 10.1 us, 16 x 2880 x 90 74 -> 63, 57 x 4160 x 24 86 -> 83, 100 x 2880 x 90
-// to float32 1,412 -> 716 (5.2 TB/s, a copy's rate), 32 x 2881 x 90 to
-// bfloat16 468 -> 176 (odd rows: one unaligned 16-byte store instead of eight
-// 2-byte ones), one packed 5760 x 90 26.4 -> 9.3, 128 x 2880 x 90 to bfloat16
-// 508 -> 471 (5.7 TB/s); packed, 57 x 4160 x 20 70 -> 72.  Values come from
+// Measured (new inputs and outputs every call) against one workgroup per 64
+// output columns and all groups (and 768 columns x 4 groups for bfloat16 of
+// 64-row multiples): 1 x 5760 x 90 groups to float16 25.4 -> 10.1 us, 16 x
+// 2880 x 90 74 -> 64, 24 x 2880 x 90 116 -> 90, 57 x 4160 x 20 71.4 -> 73.1
+// (58.3 -> 58.4 with a reused output), 57 x 4160 x 24 86.3 -> 86.1, 128 x 2880
+// x 90 535 -> 458 (5.9 TB/s), to bfloat16 508 -> 458; 100 x 2880 x 90 to
+// float32 1,400 -> 712 (5.3 TB/s, a copy's rate), 32 x 2881 x 90 to bfloat16
+// 468 -> 176 (odd rows: one unaligned 16-byte store instead of eight 2-byte
+// ones); packed, 1 x 5760 x 90 26.4 -> 9.3, 57 x 4160 x 20 70 -> 73.  Values
+// come from
 // gfx950's scaled E2M1 conversions (v_cvt_scalef32_pk_{bf16,f16,f32}_fp4),
 // exact for every scale byte below 255; the MX NaN scale 255 takes an integer
 // path (mxfp4_f32_bits) that reproduces the reference's +-inf / NaN.
@@ -413,26 +415,35 @@ int launch_dequant_shape(const uint8_t* blocks, const uint8_t* scales, uint8_t* 
   return check_launch("dequant_kernel");
 }
 
-// The workgroup shape, columns x groups (measured on four or more buffer
-// sets in turn, so nothing is left in the caches).  16-bit outputs of aligned
-// rows: 64 x 16 reads whole 256-byte pieces of each row and gives a small
-// call its workgroups; past that its 128-byte output runs cost more than they
-// save, and 256 x 4 (512-byte runs) is the one shape that lost nowhere, 128 x
-// 8 coming between.  64 x 16 / 256 x 4, us: 3 x 2880 x 90 groups (63 MB)
-// 12.7 / 16.0, 6 x 2880 x 90 (126 MB) 26.1 / 27.2, 8 x 2880 x 90 (168 MB) 33.6
-// / 33.5, 10 x 3840 x 56 (174 MB) 35.1 / 32.8, 20 x 3840 x 56 68.3 / 62.1, 57
-// x 4160 x 24 89.8 / 83.5, 38 x 3840 x 56 129.8 / 116.7, 128 x 2880 x 90 531
-// / 470.  float32 (its runs are twice as long): 384 x 4.  Odd row lengths
-// want long runs, since each run's ends share lines with its neighbours':
-// 1024 x 4 once that gives 2048 workgroups (93 x 3709 x 65 474 with 384 x 4,
-// 444), but not where its columns stand empty (1000 x 101 x 30 78 with 384 x
-// 4, 86; 500 x 201 x 33 to float32 106, 93; 200,000 x 1 x 1 332, 953).
+// The workgroup shape, columns x groups.  What decides is how much of a call's
+// input and output the 256 MB memory-side cache holds from call to call, so
+// each figure is given for new inputs and a reused output (as an allocator
+// gives it) / for new inputs and outputs, us.  16-bit outputs of aligned rows:
+// 64 x 16 up to 400 MB (whole 256-byte pieces of each row), 128 x 8 on 512
+// threads up to 1 GB, then 128 x 4.
+//   matrices x rows x groups   64 x 16        128 x 8        128 x 4
+//     8 x 2880 x 90 (168 MB)   29.1 / 33.4    29.7 / 32.6    31.6 / 33.0
+//    57 x 4160 x 17 (327 MB)   51.1 / 62.3    55.3 / 56.7    60.7 / 60.8
+//   100 x 2048 x 26 (431 MB)   71.7 / 81.5    71.0 / 75.1    75.9 / 75.2
+//    24 x 2880 x 90 (504 MB)   92.6 / 97.5    86.5 / 90.1    88.9 / 89.9
+//    38 x 3840 x 56 (662 MB)    130 / 128      126 / 124      123 / 122
+//    48 x 2880 x 90 (1.0 GB)    198 / 194      177 / 177      174 / 176
+//    64 x 2880 x 90 (1.3 GB)    265 / 264      237 / 238      230 / 235
+//   128 x 2880 x 90 (2.7 GB)    531 / 529      482 / 481      455 / 455
+// 256 x 4 is never more than 8 % from the best with new outputs, but 20 % at
+// 57 x 4160 x 17 with a reused one (61.2).  float32 (its runs are twice as
+// long): 384 x 4.  Odd row lengths want long runs, since each run's ends share
+// lines with its neighbours': 1024 x 4 once that gives 1200 workgroups (384 x
+// 4 / 1024 x 4: 93 x 3709 x 65 474 / 444, 48 x 1601 x 83 147 / 136, 25 x 2278
+// x 67, 1,275 workgroups, 85.5 / 81.9; 28 x 3627 x 19 to float32, 560, alike),
+// but not where its columns stand empty (1000 x 101 x 30 78 / 86; 500 x 201 x
+// 33 to float32 106 / 93; 200,000 x 1 x 1 332 / 953).
 template <int kDtype, bool kPacked>
 int launch_dequant_as(const uint8_t* blocks, const uint8_t* scales, uint8_t* out, int64_t n_mat, int64_t rows,
                       int64_t groups, int64_t packed_stride, hipStream_t stream) {
   if constexpr (!kPacked) {  // packed matrices have whole 64-row tiles
     if (rows % (kDtype == KLC_DTYPE_F32 ? 4 : 8) != 0) {
-      if (rows >= 192 && n_mat * ((groups + 3) / 4) * ((rows + 1023) / 1024) >= 2048)
+      if (rows >= 192 && n_mat * ((groups + 3) / 4) * ((rows + 1023) / 1024) >= 1200)
         return launch_dequant_shape<kDtype, false, false, 512, 1024, 4>(blocks, scales, out, n_mat, rows, groups, 0,
                                                                         stream);
       return launch_dequant_shape<kDtype, false, false, 256, 384, 4>(blocks, scales, out, n_mat, rows, groups, 0,
@@ -444,8 +455,11 @@ int launch_dequant_as(const uint8_t* blocks, const uint8_t* scales, uint8_t* out
                                                                     packed_stride, stream);
   } else {
     const int64_t bytes = n_mat * rows * groups * (17 + 64);
-    if (bytes >= (int64_t)160 << 20)
-      return launch_dequant_shape<kDtype, kPacked, true, 256, 256, 4>(blocks, scales, out, n_mat, rows, groups,
+    if (bytes >= (int64_t)1 << 30)
+      return launch_dequant_shape<kDtype, kPacked, true, 256, 128, 4>(blocks, scales, out, n_mat, rows, groups,
+                                                                      packed_stride, stream);
+    if (bytes >= (int64_t)400 << 20)
+      return launch_dequant_shape<kDtype, kPacked, true, 512, 128, 8>(blocks, scales, out, n_mat, rows, groups,
                                                                       packed_stride, stream);
     return launch_dequant_shape<kDtype, kPacked, true, 256, 64, 16>(blocks, scales, out, n_mat, rows, groups,
                                                                     packed_stride, stream);

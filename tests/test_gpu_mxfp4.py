@@ -74,8 +74,8 @@ def test_dequant_seeded_matches_oracle(gpu, n_mat, out_dim, groups):
                                                    (1, 136, 90), (3, 200, 33), (17, 2880, 9)])
 def test_dequant_shapes_match_oracle(gpu, n_mat, out_dim, groups, dtype, kind):
     """The workgroup shapes of aligned rows (64 x 16, float32 384 x 4) and odd ones (384 x 4, and 1024 x 4
-    from 192 rows where that gives 2048 workgroups: the 1029-row call) over partial parts and column
-    blocks, every scale byte: bit-exact.  (256 x 4 starts at 160 MB of input and output.)"""
+    from 192 rows where that gives 1200 workgroups: the 1029-row call) over partial parts and column
+    blocks, every scale byte: bit-exact.  (Larger shapes start at 400 MB of input and output.)"""
     blocks, scales = synth.mxfp4_expert_tensors(out_dim, groups, n_mat, out_dim, groups * 32, 0, 255)
     got = ops.mxfp4_dequant(torch.from_numpy(blocks).to(gpu), torch.from_numpy(scales).to(gpu), dtype)
     g = bf16_bits(got) if kind == "bf16" else got.cpu().numpy()
@@ -121,15 +121,17 @@ def test_dequant_large_call_equals_its_halves(gpu):
         torch.cuda.empty_cache()
 
 
-@pytest.mark.parametrize("n_mat,rows,groups", [(20, 2888, 90), (8, 5120, 61), (40, 1984, 28), (300, 392, 21)])
+@pytest.mark.parametrize("n_mat,rows,groups", [(20, 2888, 90), (29, 5120, 61), (96, 1984, 28), (640, 392, 21),
+                                                 (53, 2888, 90), (45, 5120, 61), (1700, 392, 21)])
 @pytest.mark.parametrize("dtype", [torch.bfloat16, torch.float16])
 def test_dequant_large_call_equals_single_matrices(gpu, n_mat, rows, groups, dtype):
-    """Calls past 160 MB of input and output take the 256 x 4 shape (here over partial column blocks and
-    parts), a matrix alone the 64 x 16 one: the same bits, checkpoint and packed layout, every scale byte."""
+    """Calls past 400 MB of input and output take the 128 x 8 shape and past 1 GB the 128 x 4 one (here over
+    partial column blocks and parts), a matrix alone the 64 x 16 one: the same bits, checkpoint and packed
+    layout, every scale byte."""
     g = torch.Generator(device=gpu).manual_seed(rows)
     blocks = torch.randint(0, 256, (n_mat, rows, groups, 16), dtype=torch.uint8, device=gpu, generator=g)
     scales = torch.randint(0, 256, (n_mat, rows, groups), dtype=torch.uint8, device=gpu, generator=g)
-    assert blocks.numel() // 16 * 81 >= 160 << 20
+    assert blocks.numel() // 16 * 81 >= 400 << 20
     big = ops.mxfp4_dequant(blocks, scales, dtype).view(torch.int16)
     for i in range(0, n_mat, max(1, n_mat // 20)):
         assert torch.equal(big[i], ops.mxfp4_dequant(blocks[i], scales[i], dtype).view(torch.int16))
