@@ -927,7 +927,8 @@ int run_moe_layer(const void* x, const void* router_w, const void* router_b, con
   if (!gemm && (rc = check_gemv_grid(n_tokens * k, n_experts))) return rc;
   if (gemm) {
     // in bfloat16 precision down's GEMM reads the hi plane alone: the zero lo plane is not written
-    // (47 MB at 2048 tokens: layer 640 -> 634 us; 2911 tokens, top-2, 2048 x 2048: 302 -> 296)
+    // (300 tokens 324 -> 320 us, 2911 of 32 experts, top-2, 2048 x 2048 238 -> 236; at 2048 tokens, 47 MB
+    // less, no difference past the runs' own: 652, 648 and 642, 652)
     const bool lo_plane = precision != KLC_PRECISION_BF16;
     if ((rc = launch_gemm_gate_up(w_gate_up, gate_up_bias, x, n_tokens, k, n_experts, offsets, sorted, units, hidden,
                                   inter, swiglu_limit, precision, lo_plane, gated, gated_raw, st)))

@@ -11,13 +11,13 @@
 // 2880 x 90 74 -> 64, 24 x 2880 x 90 116 -> 90, 57 x 4160 x 20 71.4 -> 73.1
 // (58.3 -> 58.4 with a reused output), 57 x 4160 x 24 86.3 -> 86.1, 128 x 2880
 // x 90 535 -> 458 (5.9 TB/s), to bfloat16 508 -> 458; 100 x 2880 x 90 to
-// float32 1,400 -> 712 (5.3 TB/s, a copy's rate), 32 x 2881 x 90 to bfloat16
+// float32 1,412 -> 716 (5.2 TB/s, a copy's rate), 32 x 2881 x 90 to bfloat16
 // 468 -> 176 (odd rows: one unaligned 16-byte store instead of eight 2-byte
 // ones); packed, 1 x 5760 x 90 26.4 -> 9.3, 57 x 4160 x 20 70 -> 73.  Values
-// come from
-// gfx950's scaled E2M1 conversions (v_cvt_scalef32_pk_{bf16,f16,f32}_fp4),
-// exact for every scale byte below 255; the MX NaN scale 255 takes an integer
-// path (mxfp4_f32_bits) that reproduces the reference's +-inf / NaN.
+// come from gfx950's scaled E2M1 conversions
+// (v_cvt_scalef32_pk_{bf16,f16,f32}_fp4), exact for every scale byte below
+// 255; the MX NaN scale 255 takes an integer path (mxfp4_f32_bits) that
+// reproduces the reference's +-inf / NaN.
 #include <algorithm>
 #include <type_traits>
 

@@ -103,7 +103,7 @@ def test_dequant_many_small_matrices_match_oracle(gpu, n_mat, out_dim, groups, d
 
 
 def test_dequant_large_call_equals_its_halves(gpu):
-    """160 x 2888 x 90 groups to bfloat16 (3.4 GB) takes the large-call shape, 2 matrices the small
+    """160 x 2888 x 90 groups to bfloat16 (3.4 GB) takes the largest calls' shape, 2 matrices the small
     one: the same bits, checkpoint and (2,880 rows) packed layout."""
     g = torch.Generator(device=gpu).manual_seed(9)
     for rows in (2888, 2880):

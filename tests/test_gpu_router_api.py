@@ -292,7 +292,7 @@ def test_locality_sticky_bonus_changes_selection(gpu, setup):
 
 
 def test_route_batch_gemm_streaming_matches_resident(gpu, setup, tmp_path):
-    """40 tokens at E = 16 take the grouped GEMM (n_tokens * k >= 8 * n_experts) in both stores: the resident
+    """40 tokens at E = 16 take the grouped GEMM (10 pairs an expert) in both stores: the resident
     store's one-call path (klc_moe_route) and the streaming store's separate kernels give the same bits,
     the same routing and the same expert_logs."""
     host, dev_w = setup
